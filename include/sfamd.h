@@ -310,6 +310,12 @@ int sfamd_prog_forward(const sfamd_prog_t* prog, int begin, int end,
                        const void* table, const void* in, void* out,
                        void* const* saved, void* ws, void* stream);
 
+/* The whole program without checkpoints, from `in` to `out`: the result of
+ * sfamd_prog_forward over all steps up to rounding (its fused stages may take
+ * more gates, since no adjoint runs over them). */
+int sfamd_prog_run(const sfamd_prog_t* prog, const void* table, const void* in,
+                   void* out, void* ws, void* stream);
+
 /* Adjoint sweep over steps [begin, end) in reverse.  saved[i - begin] holds
  * the input state of step i; g_out is the cotangent of the state after step
  * end-1 (PyTorch convention dL/dRe + i dL/dIm); g_in receives the cotangent

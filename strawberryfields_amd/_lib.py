@@ -118,6 +118,7 @@ SIGNATURES = {
     "sfamd_prog_destroy": (_I, [_P]),
     "sfamd_prog_build_table": (_I, [_P, _P, _P, _P]),
     "sfamd_prog_forward": (_I, [_P, _I, _I, _P, _P, _P, ctypes.POINTER(_P), _P, _P]),
+    "sfamd_prog_run": (_I, [_P, _P, _P, _P, _P, _P]),
     "sfamd_prog_adjoint": (
         _I,
         [_P, _I, _I, _P, ctypes.POINTER(_P), _P, _P, _P, _P, _P, _P],

@@ -1,5 +1,5 @@
-// Fused pure-state gate stages: descriptors shared by the planner
-// (program.hip) and the kernels (fused.hip).
+// Fused pure-state gate stages of two modes: descriptors shared by the planner
+// (program.hip) and the kernels (fused.hip).  Larger stages: mstage.h.
 #pragma once
 
 #include "common.h"
@@ -7,7 +7,6 @@
 namespace sfamd {
 
 constexpr int kStageMaxGates = 40;   // gates per stage (kernel-argument space)
-constexpr int kStageMaxTile = 4096;  // amplitudes per LDS tile (D^K)
 constexpr int kStageMaxD = 20;       // cutoffs with compiled stage kernels: 2..20
 constexpr int kStageMaxModes = 24;   // modes outside the tile
 // dynamic LDS a stage may use: gfx950 has 160 KB of LDS per compute unit

@@ -6,8 +6,7 @@
 namespace sfamd {
 
 bool stage_supported(int D, int K) {
-  if (D < 2 || D > kStageMaxD || K < 2 || K > 4) return false;
-  return ipow(D, K) <= kStageMaxTile;
+  return D >= 2 && D <= kStageMaxD && K == 2;
 }
 
 int64_t stage_gate_elems(int kind, int D, bool derivs) {

@@ -23,6 +23,7 @@
 // are the exact derivatives of the truncated matrices.
 #include "common.h"
 #include "fused.h"
+#include "mstage.h"
 
 namespace {
 
@@ -571,6 +572,42 @@ __device__ void write_stage_image(int kind, int D, const cpx<T>* __restrict__ en
   for (int64_t l = threadIdx.x; l < cnt; l += blockDim.x) dst[l] = entry[l];
 }
 
+// A gate's matrix-core images (mstage.h), one after the other: G, then (parts
+// = 3) G^H and dG/dp0^H.  Operator p (one for a single-mode gate; for a
+// beamsplitter the gate on the modular anti-diagonal {(k, (p - k) mod D)},
+// blockdiag(B_p, B_(p+D))), entry (mb, t) of half-lane h: row rp = h % 8 of
+// column group h / 8, i.e. output amplitude (rp / 2) P + 2 mb + rp % 2 and input
+// amplitude (h / 8) P + t; zero outside the operator.
+template <typename T>
+__device__ void write_matrix_images(int kind, int D, const cpx<T>* __restrict__ entry, cpx<T>* __restrict__ dst,
+                                    int parts) {
+  const bool two = kind == SFAMD_OP_BEAMSPLITTER;
+  const int P = sfamd::mst_p(D), NE = P * sfamd::mst_mb(D), n = (two ? D : 1) * NE;
+  const int64_t deriv = two ? bs_nb(D) : (int64_t)D * D;
+  const unsigned MN = ((1u << 20) + NE - 1) / NE, MP = ((1u << 20) + P - 1) / P;  // exact below 2^10
+  const int h = threadIdx.x & 31;
+  for (int x = threadIdx.x >> 5; x < parts * n; x += blockDim.x >> 5) {
+    const int which = x >= 2 * n ? 2 : x >= n ? 1 : 0, y = x - which * n;
+    const int p = (int)((unsigned)y * MN >> 20), i = y - p * NE;
+    const int mb = (int)((unsigned)i * MP >> 20), t = i - mb * P, tr = 2 * mb + (h & 1);
+    const int row = ((h & 7) >> 1) * P + tr, col = (h >> 3) * P + t;
+    cpx<T> v = mk<T>(0, 0);
+    if (tr < P && row < D && col < D) {
+      const int a = which ? col : row, b = which ? row : col;  // entry (a, b) of G or dG
+      const cpx<T>* m = entry + (which == 2 ? deriv : 0);
+      if (!two) {
+        v = m[a * D + b];
+      } else if ((a <= p) == (b <= p)) {
+        const int s = a <= p ? p : p + D;
+        const int lo = bs_lo(s, D), c = bs_hi(s, D) - lo + 1;
+        v = m[bs_block_off(s, D) + (a - lo) * c + (b - lo)];
+      }
+      if (which) v = cconj(v);
+    }
+    dst[x * 32 + h] = v;
+  }
+}
+
 template <typename T>
 __global__ void __launch_bounds__(256) k_build(sfamd::BuildBatch b, int D, const double* params, cpx<T>* table) {
   // one LDS buffer serves every builder: passive-gate blocks, D/S columns, or
@@ -586,10 +623,11 @@ __global__ void __launch_bounds__(256) k_build(sfamd::BuildBatch b, int D, const
     p1 = params[2 * pidx + 1];
   }
   cpx<T>* out = table + d.off;
-  switch (d.kind) {
+  const int kind = d.kind & 255;
+  switch (kind) {
     case SFAMD_OP_ROTATION:
     case SFAMD_OP_KERR:
-      build_diag<T>(d.kind, p0, D, out);
+      build_diag<T>(kind, p0, D, out);
       break;
     case SFAMD_OP_DISPLACEMENT:
       build_disp<T>(p0, p1, D, out, reinterpret_cast<cd(*)[2][SFAMD_MAX_CUTOFF]>(&sm_col[0][0][0]));
@@ -618,12 +656,15 @@ __global__ void __launch_bounds__(256) k_build(sfamd::BuildBatch b, int D, const
     default:
       break;
   }
-  if (d.img_fwd >= 0 || d.img_adj >= 0) {
-    // the entry was written by this workgroup: the barrier orders those
-    // stores before the reads below (same compute unit)
-    __syncthreads();
-    if (d.img_fwd >= 0) write_stage_image<T>(d.kind, D, out, table + d.img_fwd, false);
-    if (d.img_adj >= 0) write_stage_image<T>(d.kind, D, out, table + d.img_adj, true);
+  const bool diag = kind == SFAMD_OP_ROTATION || kind == SFAMD_OP_KERR;
+  // the entry was written by this workgroup: the barrier orders those
+  // stores before the reads below (same compute unit)
+  if (d.img0 >= 0 || d.img1 >= 0 || d.kind > 255) __syncthreads();
+  if (d.img0 >= 0) write_stage_image<T>(kind, D, out, table + d.img0, false);
+  if (d.img1 >= 0) write_stage_image<T>(kind, D, out, table + d.img1, true);
+  if (!diag && (d.kind & sfamd::kBuildMatrixFwd)) {
+    const int64_t size = kind == SFAMD_OP_BEAMSPLITTER ? 2 * bs_nb(D) : 3 * (int64_t)D * D;
+    write_matrix_images<T>(kind, D, out, out + size, d.kind & sfamd::kBuildMatrixAdj ? 3 : 1);
   }
 }
 

@@ -8,6 +8,7 @@
 // captured into a HIP graph by the caller (sfamd_graph_*).
 #include <algorithm>
 #include <cstring>
+#include <functional>
 #include <new>
 #include <vector>
 
@@ -15,6 +16,7 @@
 #include "fiber.h"
 #include "fused.h"
 #include "mfma.h"
+#include "mstage.h"
 #include "slab.h"
 
 using namespace sfamd;
@@ -295,23 +297,29 @@ int adjoint_op(const OpPlan& op, int n, int D, const void* table, const void* ps
 
 }  // namespace
 
-// One step of execution: a single operation (element-wise kernels) or a
-// fused stage of gates on K local modes of a pure state (fused.hip).
+// One step of execution: a single operation (or a run of diagonal gates), or a
+// fused stage of gates on K local modes of a pure state: on the vector ALUs
+// (K = 2, fused.hip) or on the matrix cores (K >= 3, mstage.hip).
+enum StepKind { kStepSingle = 0, kStepDiagRun, kStepStage, kStepMatrixStage };
 struct Step {
-  int fused;
-  int op;  // single operation index (fused == 0)
+  int kind;
+  int op;  // single operation index (kStepSingle)
   int K;
-  int diag;  // a run of rotation / Kerr gates in one pass (fused == 0)
   std::vector<int> ops;  // operation indices in execution order
   StageArgs args;
+  MArgs margs;
   DiagRun run;
 };
 
 struct sfamd_prog {
   int n, D, dtype, mixed_in, nops, nwg, fuse_K;
   std::vector<OpPlan> ops;
-  std::vector<int32_t> img_fwd, img_adj;  // per op: its stage-image regions, or -1
+  std::vector<int32_t> img0, img1;          // per op: its vector-ALU stage images, or copies of its phases; -1: none
+  std::vector<int32_t> mimg_fwd, mimg_adj;  // per op: its matrix-core images, or -1
   std::vector<Step> steps;
+  // the whole program without checkpoints or adjoint (sfamd_prog_run): matrix-core
+  // stages hold one tile in LDS, so they take more gates; empty: the same as steps
+  std::vector<Step> fsteps;
   std::vector<int64_t> state_elems;  // elements at the input of step i (i = nsteps: output)
   int64_t table_elems, max_state;
   int final_mixed;
@@ -327,49 +335,338 @@ bool fusable(const OpPlan& op) {
 
 int op_nmodes(const OpPlan& op) { return two_mode_kind(op.kind) ? 2 : 1; }
 
-bool op_in(const OpPlan& op, unsigned mask) {
-  if (!(mask >> op.m0 & 1u)) return false;
-  return !two_mode_kind(op.kind) || (mask >> op.m1 & 1u);
-}
-
 unsigned op_mask(const OpPlan& op) {
   unsigned m = 1u << op.m0;
   if (two_mode_kind(op.kind)) m |= 1u << op.m1;
   return m;
 }
 
+// LDS a stage needs, by the kernels that run it: fixed bytes and bytes per gate
+struct StageCost {
+  int64_t base, budget, budget_full;
+  int max_gates;
+  std::function<int64_t(const OpPlan&)> gate;
+};
+
+// An operation as the stage search sees it.
+struct StageOp {
+  unsigned modes;
+  int64_t cost;
+};
+
 // ops of `rem` (program order) absorbable into a stage on `mask`: an op joins
 // if its modes lie in the mask, no earlier op left outside the stage touches
-// one of them (gates on disjoint modes commute) and the adjoint kernel's LDS
-// (one tile per gate plus two, and every gate's matrix + derivatives) fits
-void absorb(const std::vector<OpPlan>& ops, const std::vector<int>& rem, unsigned mask, int D, int Kc,
-            int64_t tile_bytes, int64_t esz, int64_t budget, std::vector<int>* got) {
-  got->clear();
+// one of them (gates on disjoint modes commute) and the stage's LDS fits.
+// Returns their number; `skip` marks operations that an earlier stage takes,
+// `got` receives the indices.
+int absorb(const std::vector<StageOp>& ops, const std::vector<int>& rem, unsigned mask, const StageCost& sc,
+           int64_t budget, const char* skip, std::vector<int>* got) {
+  if (got) got->clear();
   unsigned blocked = 0;
-  int64_t used = 3 * tile_bytes;  // the stage input and two cotangent tiles
+  int64_t used = sc.base;
+  int count = 0;
   for (int i : rem) {
-    const OpPlan& op = ops[i];
-    const unsigned om = op_mask(op);
-    const int64_t cost = tile_bytes + (((stage_gate_elems(op.kind, D, true) + 1) & ~(int64_t)1) * esz) +
-                         2 * (stage_threads(D, Kc) / 64) * 8;
-    if ((int)got->size() < kStageMaxGates && op_in(op, mask) && !(om & blocked) && used + cost <= budget) {
-      got->push_back(i);
-      used += cost;
+    const StageOp& op = ops[i];
+    if (!(op.modes & mask) || (skip && skip[i])) continue;
+    if (count < sc.max_gates && !(op.modes & ~mask) && !(op.modes & blocked) && used + op.cost <= budget) {
+      if (got) got->push_back(i);
+      ++count;
+      used += op.cost;
     } else {
-      blocked |= om;
+      blocked |= op.modes;
+      if ((blocked & mask) == mask) break;  // nothing further can join
     }
+  }
+  return count;
+}
+
+bool is_diag_kind(int kind) { return kind == SFAMD_OP_ROTATION || kind == SFAMD_OP_KERR; }
+
+Step new_step(int kind, int op) {
+  Step st;
+  st.kind = kind;
+  st.op = op;
+  st.K = 0;
+  memset(&st.args, 0, sizeof(st.args));
+  memset(&st.margs, 0, sizeof(st.margs));
+  memset(&st.run, 0, sizeof(st.run));
+  return st;
+}
+
+constexpr int kMstGatesForTwo = 4;            // gates each of two workgroups per CU must still hold
+
+// log2 of the tiles a workgroup of a matrix-core stage holds: as many as fill
+// the 16 columns of a beamsplitter's matrix-core operand, if every CU still
+// has a group
+int group_log2(const sfamd_prog* p, int Kc) {
+  const int D = p->D;
+  const int64_t ntiles = ipow(D, p->n - Kc);
+  int l = 0;
+  while (mst_group_ok(D, Kc, l + 1) && (mst_tile(D, Kc) / (D * D) << l) <= 8 && (ntiles >> (l + 1)) >= kComputeUnits)
+    ++l;
+  return l;
+}
+
+// What a stage of Kc local modes may hold.  kStepStage: one tile per gate plus
+// three and every gate's matrices (the adjoint kernel's LDS).
+// kStepMatrixStage: the adjoint keeps one tile per gate with operators plus two,
+// the forward-only plan one tile group.
+StageCost stage_cost(const sfamd_prog* p, int kind, int Kc, bool forward_only) {
+  const int D = p->D;
+  const int64_t esz = elem_size(p->dtype);
+  // a launch has one workgroup per tile (up to the grid cap): when that is
+  // more than one per compute unit, two should fit in a CU's LDS at once
+  const bool many = ipow(D, p->n - Kc) > kComputeUnits;
+  StageCost sc;
+  sc.budget_full = kStageLdsBudget;
+  sc.budget = many ? kStageLdsPerCu / 2 - 512 : kStageLdsBudget;
+  if (kind == kStepStage) {
+    const int64_t tile = stage_tile(D, Kc) * esz, slots = 2 * (stage_threads(D, Kc) / 64) * 8;
+    sc.max_gates = kStageMaxGates;
+    sc.base = 3 * tile;  // the stage input and two cotangent tiles
+    sc.gate = [=](const OpPlan& op) {
+      return tile + (((stage_gate_elems(op.kind, D, true) + 1) & ~(int64_t)1) * esz) + slots;
+    };
+    return sc;
+  }
+  const int lgt = group_log2(p, Kc);
+  const int64_t tile = ((int64_t)mst_tile_lds(D, Kc) << lgt) * esz, phases = (int64_t)(D + 1) * esz;
+  sc.max_gates = kMstMaxGates;
+  sc.budget_full = kMstLdsMax;
+  if ((ipow(D, p->n - Kc) >> lgt) <= kComputeUnits) sc.budget = sc.budget_full;
+  if (forward_only) {
+    sc.base = tile;
+    sc.budget = sc.budget_full;
+    sc.gate = [=](const OpPlan& op) { return is_diag_kind(op.kind) ? phases : 0; };
+    return sc;
+  }
+  const int64_t slots = 2 * mst_waves(D, Kc, lgt) * 8;
+  // two workgroups per CU only if each still holds kMstGatesForTwo gates
+  if (sc.budget < 2 * tile + kMstGatesForTwo * (tile + slots)) sc.budget = sc.budget_full;
+  sc.base = 2 * tile;
+  sc.gate = [=](const OpPlan& op) { return (is_diag_kind(op.kind) ? phases : tile) + slots; };
+  return sc;
+}
+
+// Can a stage of this kind hold one gate of any kind?
+bool stage_fits(const sfamd_prog* p, int kind, int Kc, bool forward_only) {
+  if (Kc < 2 || Kc > p->n) return false;
+  if (kind == kStepStage ? (p->n > kStageMaxModes || !stage_supported(p->D, Kc))
+                         : (p->n > kMstMaxModes || !mst_supported(p->D, Kc)))
+    return false;
+  if (ipow(p->D, p->n - Kc) >= ((int64_t)1 << 31)) return false;
+  const StageCost sc = stage_cost(p, kind, Kc, forward_only);
+  OpPlan bs{SFAMD_OP_BEAMSPLITTER, 0, 1, 0, 0, 0};
+  return sc.base + sc.gate(bs) <= sc.budget_full;
+}
+
+void fill_stage(const sfamd_prog* p, Step& st, unsigned mask) {
+  const int n = p->n, D = p->D, Kc = st.K;
+  StageArgs& a = st.args;
+  a.ngates = (int)st.ops.size();
+  int lmodes[4], nl = 0, nlc = 0;
+  for (int md = 0; md < n; ++md) {
+    if (mask >> md & 1u)
+      lmodes[nl++] = md;
+    else
+      a.nl_stride[nlc++] = ipow(D, n - 1 - md);
+  }
+  a.nnl = nlc;
+  a.ntiles = (int32_t)ipow(D, nlc);
+  for (int t = 0; t < Kc; ++t) a.loc_stride[t] = ipow(D, n - 1 - lmodes[t]);
+  int64_t mf = 0, ma = 0;
+  for (int gi = 0; gi < a.ngates; ++gi) {
+    const OpPlan& op = p->ops[st.ops[gi]];
+    StageGate& g = a.g[gi];
+    g.kind = (int8_t)op.kind;
+    g.a0 = g.a1 = 0;
+    for (int t = 0; t < Kc; ++t) {
+      if (lmodes[t] == op.m0) g.a0 = (int8_t)t;
+      if (op.kind == SFAMD_OP_BEAMSPLITTER && lmodes[t] == op.m1) g.a1 = (int8_t)t;
+    }
+    g.op = st.ops[gi];
+    g.s0 = (int32_t)ipow(D, Kc - 1 - g.a0);
+    g.s1 = (int32_t)ipow(D, Kc - 1 - g.a1);
+    // one region per gate, 16-byte aligned in LDS: the matrix in the
+    // forward kernel, matrix + derivative in the adjoint
+    g.moff = (int32_t)mf;
+    g.amoff = (int32_t)ma;
+    mf += (stage_gate_elems(op.kind, D, false) + 1) & ~(int64_t)1;
+    ma += (stage_gate_elems(op.kind, D, true) + 1) & ~(int64_t)1;
+  }
+  a.mat_fwd = (int32_t)mf;
+  a.mat_adj = (int32_t)ma;
+}
+
+// order of the modes in a state, slowest first, and their strides
+struct ModeOrder {
+  int n = 0, at[32];
+  int64_t stride[32];  // by mode
+  void set_strides(int D) {
+    int64_t s = 1;
+    for (int i = n - 1; i >= 0; --i) {
+      stride[at[i]] = s;
+      s *= D;
+    }
+  }
+};
+
+ModeOrder canonical_order(int n, int D) {
+  ModeOrder o;
+  o.n = n;
+  for (int m = 0; m < n; ++m) o.at[m] = m;
+  o.set_strides(D);
+  return o;
+}
+
+// a matrix-core stage on the modes of `mask`, from states in mode order `in` to
+// states in mode order `out`
+void fill_matrix_stage(const sfamd_prog* p, Step& st, unsigned mask, bool forward_only, const ModeOrder& in,
+                       const ModeOrder& out) {
+  const int n = p->n, D = p->D, Kc = st.K;
+  MArgs& a = st.margs;
+  memset(&a, 0, sizeof(a));
+  a.ngates = (int)st.ops.size();
+  int lmodes[kMstMaxK], nl = 0;
+  for (int i = n - 1; i >= 0; --i)  // fastest first
+    if (!(mask >> in.at[i] & 1u)) {
+      a.nl_stride[a.nnl] = in.stride[in.at[i]];
+      a.out_nl_stride[a.nnl++] = out.stride[in.at[i]];
+    }
+  for (int i = 0; i < n; ++i)  // slowest first
+    if (mask >> in.at[i] & 1u) lmodes[nl++] = in.at[i];
+  a.ntiles = (int32_t)ipow(D, a.nnl);
+  a.lgt = group_log2(p, Kc);
+  for (int t = 0; t < Kc; ++t) a.loc_stride[t] = in.stride[lmodes[t]];
+  int u = 0;
+  for (int i = 0; i < n; ++i)
+    for (int t = 0; t < Kc; ++t)
+      if (lmodes[t] == out.at[i]) {
+        a.out_stride[u] = out.stride[out.at[i]];
+        a.out_lds[u++] = mst_stride(D, Kc, t);
+      }
+  for (int gi = 0; gi < a.ngates; ++gi) {
+    const OpPlan& op = p->ops[st.ops[gi]];
+    MGate& g = a.g[gi];
+    const bool two = op.kind == SFAMD_OP_BEAMSPLITTER;
+    int ax0 = 0, ax1 = -1;
+    for (int t = 0; t < Kc; ++t) {
+      if (lmodes[t] == op.m0) ax0 = t;
+      if (two && lmodes[t] == op.m1) ax1 = t;
+    }
+    int u = 0;
+    for (int t = 0; t < Kc; ++t)
+      if (t != ax0 && t != ax1) g.cs[u++] = mst_stride(D, Kc, t);
+    g.kind = op.kind;
+    g.a0 = ax0;
+    g.l1 = two ? mst_stride(D, Kc, ax1) : 0;
+    g.ds = mst_stride(D, Kc, ax0) - g.l1;
+    g.wrap = D * g.l1;
+    g.op = st.ops[gi];
+    g.two = two;
+    if (is_diag_kind(op.kind))
+      ++a.ndiag;
+    else
+      ++a.nheavy;
+  }
+}
+
+// table offsets of a matrix-core stage's images, once they are placed; every
+// gate, also a rotation or Kerr gate, names the forward image of the next gate
+// with operators and the adjoint image of the previous one (at the ends, and in
+// a stage without such gates, an image that is loaded and not used)
+void link_matrix_stage(const sfamd_prog* p, MArgs& a, int spare) {
+  int nd = 0;
+  a.h0_fwd = a.hl_adj = spare;
+  int off = spare, two = 0;
+  for (int gi = 0; gi < a.ngates; ++gi) {
+    MGate& g = a.g[gi];
+    g.padj = off;
+    g.two |= two << 2;
+    if (is_diag_kind(g.kind)) {
+      g.fwd = nd++ * p->D;
+      continue;
+    }
+    g.fwd = p->mimg_fwd[g.op];
+    g.adj = p->mimg_adj[g.op] < 0 ? spare : p->mimg_adj[g.op];
+    off = a.hl_adj = g.adj;
+    two = a.hl_two = g.two & 1;
+  }
+  off = spare;
+  two = 0;
+  for (int gi = a.ngates - 1; gi >= 0; --gi) {
+    MGate& g = a.g[gi];
+    g.nfwd = off;
+    g.two |= two << 1;
+    if (is_diag_kind(g.kind)) continue;
+    off = a.h0_fwd = g.fwd;
+    two = a.h0_two = g.two & 1;
+  }
+}
+
+// Mode orders between the stages of a forward-only run (masks: their local
+// modes, first: the first of them).  A stage whose local modes are not the
+// fastest ones reads and writes single amplitudes, one cache line each (6
+// modes, cutoff 16, complex64, 134 MB: two beamsplitters on modes 0 to 2 292 us,
+// one on the last modes 58 us, a device copy 38 us).  The states between the
+// stages are the library's own, so each stage writes its output with the next stage's local modes
+// fastest: reads are whole tiles, and writes are runs of the mode that the two
+// stages share, placed fastest of all.  Unused local modes are chosen to share
+// one with the stage before.
+void order_stages(const sfamd_prog* p, std::vector<Step>* steps, size_t first, std::vector<unsigned> masks) {
+  const int n = p->n, D = p->D;
+  const size_t count = masks.size();
+  if (n <= (*steps)[first].K) return;
+  for (size_t i = 0; i < count; ++i) {
+    unsigned used = 0;
+    for (int op : (*steps)[first + i].ops) used |= op_mask(p->ops[op]);
+    const unsigned before = i ? masks[i - 1] : 1u << (n - 1);
+    const unsigned after = i + 1 < count ? masks[i + 1] : 1u << (n - 1);
+    unsigned m = used;
+    auto fill = [&](unsigned from) {
+      for (int md = n - 1; md >= 0; --md)
+        if (__builtin_popcount(m) < (*steps)[first + i].K && (from >> md & 1u)) m |= 1u << md;
+    };
+    if (!(used & before)) fill(before & ~(before - 1u));  // one mode of the stage before
+    if (!(used & after)) fill(after & ~(after - 1u));
+    fill(before);
+    fill(~0u >> (32 - n));
+    masks[i] = m;
+  }
+  ModeOrder in = canonical_order(n, D);
+  for (size_t i = 0; i < count; ++i) {
+    ModeOrder out = canonical_order(n, D);
+    if (i + 1 < count) {
+      int k = 0;
+      const unsigned next = masks[i + 1], mine = masks[i];
+      for (int pass = 0; pass < 3; ++pass)  // others, the next stage's own, the shared ones (fastest)
+        for (int j = 0; j < n; ++j) {
+          const unsigned b = 1u << in.at[j];
+          const int cls = !(next & b) ? 0 : !(mine & b) ? 1 : 2;
+          if (cls == pass) out.at[k++] = in.at[j];
+        }
+      out.set_strides(D);
+    }
+    MArgs& a = (*steps)[first + i].margs;
+    fill_matrix_stage(p, (*steps)[first + i], masks[i], true, in, out);
+    a.permuted = 1;
+    // no shared mode: the workgroup takes neighbouring tiles, for runs of that many amplitudes
+    if (a.out_stride[(*steps)[first + i].K - 1] != 1)
+      while (mst_group_ok(D, (*steps)[first + i].K, a.lgt + 1) && (a.ntiles >> (a.lgt + 1)) >= 4 * kComputeUnits &&
+             mst_lds_fwd(D, (*steps)[first + i].K, a.lgt + 1, a.ndiag, p->dtype) <= kMstLds / 2)
+        ++a.lgt;
+    in = out;
   }
 }
 
 // greedy partition of a run of fusable ops into stages of Kc local modes
-void plan_run(sfamd_prog* p, const std::vector<int>& run, int Kc) {
-  const int n = p->n, D = p->D;
-  const int64_t esz = elem_size(p->dtype);
-  const int64_t tile_bytes = stage_tile(D, Kc) * esz;
-  // a launch has one workgroup per tile (up to the grid cap): when that is
-  // more than one per compute unit, two must fit in a CU's LDS at once
-  const int64_t ntiles = ipow(D, n - Kc);
-  const int64_t budget = ntiles > kComputeUnits ? kStageLdsPerCu / 2 - 512 : kStageLdsBudget;
+void plan_run(const sfamd_prog* p, const std::vector<int>& run, int kind, int Kc, bool forward_only,
+              std::vector<Step>* steps) {
+  const int n = p->n;
+  const StageCost sc = stage_cost(p, kind, Kc, forward_only);
+  const ModeOrder order = canonical_order(n, p->D);
+  std::vector<unsigned> masks;   // of this run's steps
+  std::vector<size_t> stages;    // its matrix-core stages
   std::vector<int> rem = run;
   std::vector<unsigned> cands;
   // all Kc-subsets when few, else subsets grown from the next ops
@@ -389,7 +686,10 @@ void plan_run(sfamd_prog* p, const std::vector<int>& run, int Kc) {
       for (int u = t + 1; u < Kc; ++u) idx[u] = idx[u - 1] + 1;
     }
   }
-  std::vector<int> got, best, rem2, got2;
+  std::vector<int> got, best;
+  std::vector<StageOp> sops(p->nops);
+  for (int i : run) sops[i] = StageOp{op_mask(p->ops[i]), sc.gate(p->ops[i])};
+  std::vector<char> taken(p->nops, 0);
   while (!rem.empty()) {
     std::vector<unsigned> local = cands;
     if (local.empty()) {
@@ -406,28 +706,22 @@ void plan_run(sfamd_prog* p, const std::vector<int>& run, int Kc) {
     best.clear();
     // the occupancy budget is a preference: a gate too large for it (compact
     // beamsplitter tables at high cutoff) gets a stage of the full budget
-    for (int64_t bud : {budget, kStageLdsBudget}) {
+    for (int64_t bud : {sc.budget, sc.budget_full}) {
       long bkey = -1;
       for (unsigned m : local) {
-        absorb(p->ops, rem, m, D, Kc, tile_bytes, esz, bud, &got);
+        absorb(sops, rem, m, sc, bud, nullptr, &got);
         // one step of lookahead: the gates this stage takes plus the most the
         // next stage could take after it (on c3: 49 stages instead of 52);
         // ties go to more gates now, then to tiles that include the last
         // modes (contiguous runs)
         long nxt = 0;
         if (!got.empty() && local.size() > 1 && got.size() < rem.size()) {
-          rem2.clear();
-          size_t gi = 0;
-          for (int i : rem) {
-            if (gi < got.size() && got[gi] == i)
-              ++gi;
-            else
-              rem2.push_back(i);
-          }
+          for (int i : got) taken[i] = 1;
           for (unsigned m2 : local) {
-            absorb(p->ops, rem2, m2, D, Kc, tile_bytes, esz, bud, &got2);
-            if ((long)got2.size() > nxt) nxt = (long)got2.size();
+            const long k = absorb(sops, rem, m2, sc, bud, taken.data(), nullptr);
+            if (k > nxt) nxt = k;
           }
+          for (int i : got) taken[i] = 0;
         }
         const long key = (((long)got.size() + nxt) << 40) + ((long)got.size() << 26) + (long)m;
         if (key > bkey) {
@@ -440,62 +734,23 @@ void plan_run(sfamd_prog* p, const std::vector<int>& run, int Kc) {
     }
     if (best.empty()) {
       // no stage holds the next operation: it runs on its own, unfused
-      Step one;
-      one.fused = 0;
-      one.op = rem.front();
-      one.K = 0;
-      one.diag = 0;
+      Step one = new_step(kStepSingle, rem.front());
       one.ops.push_back(rem.front());
-      memset(&one.args, 0, sizeof(one.args));
-      memset(&one.run, 0, sizeof(one.run));
-      p->steps.push_back(one);
+      steps->push_back(one);
+      masks.push_back(0);
       rem.erase(rem.begin());
       continue;
     }
-    Step st;
-    st.fused = 1;
-    st.op = best.front();
+    Step st = new_step(kind, best.front());
     st.K = Kc;
-    st.diag = 0;
     st.ops = best;
-    memset(&st.run, 0, sizeof(st.run));
-    StageArgs& a = st.args;
-    memset(&a, 0, sizeof(a));
-    a.ngates = (int)best.size();
-    int lmodes[4], nl = 0, nlc = 0;
-    for (int md = 0; md < n; ++md) {
-      if (bm >> md & 1u)
-        lmodes[nl++] = md;
-      else
-        a.nl_stride[nlc++] = ipow(D, n - 1 - md);
-    }
-    a.nnl = nlc;
-    a.ntiles = (int32_t)ipow(D, nlc);
-    a.grid = 0;
-    for (int t = 0; t < Kc; ++t) a.loc_stride[t] = ipow(D, n - 1 - lmodes[t]);
-    int64_t mf = 0, ma = 0;
-    for (int gi = 0; gi < a.ngates; ++gi) {
-      const OpPlan& op = p->ops[best[gi]];
-      StageGate& g = a.g[gi];
-      g.kind = (int8_t)op.kind;
-      g.a0 = g.a1 = 0;
-      for (int t = 0; t < Kc; ++t) {
-        if (lmodes[t] == op.m0) g.a0 = (int8_t)t;
-        if (op.kind == SFAMD_OP_BEAMSPLITTER && lmodes[t] == op.m1) g.a1 = (int8_t)t;
-      }
-      g.op = best[gi];
-      g.s0 = (int32_t)ipow(D, Kc - 1 - g.a0);
-      g.s1 = (int32_t)ipow(D, Kc - 1 - g.a1);
-      // one region per gate, 16-byte aligned in LDS: the matrix in the
-      // forward kernel, matrix + derivative in the adjoint
-      g.moff = (int32_t)mf;
-      g.amoff = (int32_t)ma;
-      mf += (stage_gate_elems(op.kind, D, false) + 1) & ~(int64_t)1;
-      ma += (stage_gate_elems(op.kind, D, true) + 1) & ~(int64_t)1;
-    }
-    a.mat_fwd = (int32_t)mf;
-    a.mat_adj = (int32_t)ma;
-    p->steps.push_back(st);
+    if (kind == kStepStage)
+      fill_stage(p, st, bm);
+    else
+      fill_matrix_stage(p, st, bm, forward_only, order, order);
+    steps->push_back(st);
+    masks.push_back(bm);
+    if (kind == kStepMatrixStage) stages.push_back(steps->size() - 1);
     std::vector<int> nrem;
     size_t bi = 0;
     for (int i : rem) {
@@ -506,56 +761,42 @@ void plan_run(sfamd_prog* p, const std::vector<int>& run, int Kc) {
     }
     rem.swap(nrem);
   }
+  if (forward_only && kind == kStepMatrixStage && stages.size() == masks.size())
+    order_stages(p, steps, steps->size() - masks.size(), masks);
 }
 
-void plan_steps(sfamd_prog* p) {
+// `kind`, Kc: the stages of the plan (Kc = 0: none)
+void plan_steps(const sfamd_prog* p, int kind, int Kc, bool forward_only, std::vector<Step>* steps) {
   const int n = p->n, D = p->D;
-  const int Kc = p->fuse_K < n ? p->fuse_K : n;
-  const int64_t esz = elem_size(p->dtype);
-  // fusion needs compiled stage kernels and room for at least one gate of any kind
-  int gmax = 0;
-  if (Kc >= 2 && n <= kStageMaxModes && stage_supported(D, Kc)) {
-    const int64_t one = 4 * stage_tile(D, Kc) * esz + stage_gate_elems(SFAMD_OP_BEAMSPLITTER, D, true) * esz + 256;
-    gmax = one <= kStageLdsBudget ? 1 : 0;
-  }
   std::vector<int> run;
   auto flush = [&]() {
-    if (!run.empty()) plan_run(p, run, Kc);
+    if (!run.empty()) plan_run(p, run, kind, Kc, forward_only, steps);
     run.clear();
   };
-  auto is_diag = [&](int i) {
-    const int k = p->ops[i].kind;
-    return k == SFAMD_OP_ROTATION || k == SFAMD_OP_KERR;
-  };
+  auto is_diag = [&](int i) { return is_diag_kind(p->ops[i].kind); };
   for (int i = 0; i < p->nops; ++i) {
-    if (gmax >= 1 && fusable(p->ops[i])) {
+    if (Kc >= 2 && fusable(p->ops[i])) {
       run.push_back(i);
       continue;
     }
     flush();
     // consecutive rotation / Kerr gates on the same representation share one pass
-    if (is_diag(i) && !p->steps.empty()) {
-      Step& last = p->steps.back();
-      if (!last.fused && is_diag(last.ops.back()) && p->ops[last.ops.back()].mixed_in == p->ops[i].mixed_in &&
-          (int)last.ops.size() < kDiagRunMax) {
+    if (is_diag(i) && !steps->empty()) {
+      Step& last = steps->back();
+      if (last.kind <= kStepDiagRun && is_diag(last.ops.back()) &&
+          p->ops[last.ops.back()].mixed_in == p->ops[i].mixed_in && (int)last.ops.size() < kDiagRunMax) {
         last.ops.push_back(i);
-        last.diag = 1;
+        last.kind = kStepDiagRun;
         continue;
       }
     }
-    Step st;
-    st.fused = 0;
-    st.op = i;
-    st.K = 0;
-    st.diag = 0;
+    Step st = new_step(kStepSingle, i);
     st.ops.push_back(i);
-    memset(&st.args, 0, sizeof(st.args));
-    memset(&st.run, 0, sizeof(st.run));
-    p->steps.push_back(st);
+    steps->push_back(st);
   }
   flush();
-  for (Step& st : p->steps) {
-    if (!st.diag) continue;
+  for (Step& st : *steps) {
+    if (st.kind != kStepDiagRun) continue;
     DiagRun& r = st.run;
     const OpPlan& first = p->ops[st.ops.front()];
     r.n = n;
@@ -569,18 +810,169 @@ void plan_steps(sfamd_prog* p) {
       r.mode[g] = op.m0;
       r.kind[g] = op.kind;
       r.op[g] = st.ops[g];
-      r.toff[g] = op.off;
       int64_t dv = 1;
       for (int t = 0; t < n - 2 - op.m0; ++t) dv *= R;
       r.rowdiv[g] = dv;
     }
   }
+}
+
+// Do stages of K local modes pay on this state?  Past the caches a stage whose
+// local modes are not the last ones moves single amplitudes (the forward-only
+// plan orders the modes of its intermediate states against that), so kernels
+// with one pass per gate catch up.  One layer of the layered circuit, forward
+// and adjoint, unfused / fused, us (complex64: 6 modes cutoff 12, 24 MB: 2670 /
+// 2420; 6 modes 14, 60 MB: 4570 / 6200; 7 modes 10, 80 MB: 8060 / 11100; 8 modes 8,
+// 134 MB: 13950 / 10250; 9 modes 5, 16 MB: 4760 / 4280; complex128: 9 modes 5,
+// 31 MB: 4310 / 6670; 6 modes 12, 48 MB: 5750 / 3630; 6 modes 14, 120 MB: 14150 /
+// 13500); forward only (complex64: 6 modes 16, 134 MB: 2750 / 1930; 8 modes 8:
+// 4640 / 2410; complex128: 6 modes 14: 3930 / 2390; 7 modes 10, 160 MB: 4850 / 5460).
+bool stages_pay(const sfamd_prog* p, int kind, bool forward_only) {
+  const int D = p->D;
+  const int64_t mb = ipow(D, p->n) * elem_size(p->dtype) / 1000000, wide = p->dtype == SFAMD_C64 ? 1 : 2;
+  // vector-ALU stages: 5 modes cutoff 13 (3 MB) 1154 / 728, cutoff 16 (8 MB) 1402 / 1813; complex128 cutoff 13
+  // (6 MB) 1848 / 1337, cutoff 16 (17 MB) 3770 / 4640
+  if (kind == kStepStage) return mb < (wide == 1 ? 6 : 10);
+  if (forward_only) return !(D == 9 || D == 10) || mb < 64;
+  if (D <= 5) return mb < 20;
+  return D <= 8 || mb < 32 * wide;
+}
+
+// The stages of a plan for a requested number of local modes: matrix-core
+// stages for three and more, vector-ALU stages for two (a beamsplitter on two
+// local modes has one column, so a matrix-core operand would be 15/16 empty) and
+// where the matrix-core adjoint's tiles exceed the LDS.
+void pick_stages(const sfamd_prog* p, bool forward_only, int* kind, int* Kc) {
+  const int K = p->fuse_K < p->n ? p->fuse_K : p->n;
+  *kind = kStepMatrixStage;
+  *Kc = K;
+  if (K >= 3 && stage_fits(p, kStepMatrixStage, K, forward_only)) {
+    if (!stages_pay(p, kStepMatrixStage, forward_only)) *Kc = 0;
+    return;
+  }
+  *kind = kStepStage;
+  *Kc = K >= 2 && stage_fits(p, kStepStage, 2, false) && (p->fuse_K == 2 || stages_pay(p, kStepStage, false)) ? 2 : 0;
+}
+
+void plan_program(sfamd_prog* p) {
+  int kind, Kc, fkind, fKc;
+  pick_stages(p, false, &kind, &Kc);
+  plan_steps(p, kind, Kc, false, &p->steps);
+  pick_stages(p, true, &fkind, &fKc);
+  if (fKc >= 3 && fkind == kStepMatrixStage) plan_steps(p, fkind, fKc, true, &p->fsteps);
   // state sizes at step inputs
   p->state_elems.clear();
   for (const Step& st : p->steps) {
     const OpPlan& op = p->ops[st.ops.front()];
-    p->state_elems.push_back(ipow(D, op.mixed_in ? 2 * n : n));
+    p->state_elems.push_back(ipow(p->D, op.mixed_in ? 2 * p->n : p->n));
   }
+}
+
+// Lay the gate table out: every operation's entry, followed by its matrix-core
+// operator images (G; for a gate in a step with an adjoint G^H and dG/dp0^H
+// too), then each matrix-core stage's phases as one region (the entries
+// themselves in the forward-only plan, copies in the other) and the vector-ALU
+// stages' images, one region per kernel.
+void place_table(sfamd_prog* p) {
+  p->img0.assign(p->nops, -1);
+  p->img1.assign(p->nops, -1);
+  p->mimg_fwd.assign(p->nops, -1);
+  p->mimg_adj.assign(p->nops, -1);
+  std::vector<char> in_phases(p->nops, 0);
+  bool matrix = false;
+  for (const std::vector<Step>* steps : {&p->steps, &p->fsteps})
+    for (const Step& st : *steps) {
+      if (st.kind != kStepMatrixStage) continue;
+      matrix = true;
+      for (int op : st.ops) {
+        if (is_diag_kind(p->ops[op].kind)) {
+          if (steps == &p->fsteps) in_phases[op] = 1;
+          continue;
+        }
+        p->mimg_fwd[op] = 0;
+        if (steps == &p->steps) p->mimg_adj[op] = 0;
+      }
+    }
+  int64_t off = 0;
+  for (int i = 0; i < p->nops; ++i) {
+    OpPlan& op = p->ops[i];
+    if (in_phases[i]) continue;
+    op.off = off;
+    off += table_size(op.kind, p->D);
+    if (p->mimg_fwd[i] >= 0) {
+      p->mimg_fwd[i] = (int32_t)off;
+      off += mst_img_elems(op.kind, p->D, false);
+    }
+    if (p->mimg_adj[i] >= 0) {
+      p->mimg_adj[i] = (int32_t)off;
+      off += mst_img_elems(op.kind, p->D, true);
+    }
+  }
+  const int32_t spare = (int32_t)off;  // readable where a kernel loads an operator that it does not use
+  if (matrix) off += 2 * mst_img(p->D);
+  for (Step& st : p->fsteps) {
+    if (st.kind != kStepMatrixStage) continue;
+    st.margs.phases = (int32_t)off;
+    for (int op : st.ops)
+      if (in_phases[op]) {
+        p->ops[op].off = off;
+        off += p->D;
+      }
+  }
+  for (Step& st : p->steps) {
+    if (st.kind == kStepStage) {
+      StageArgs& a = st.args;
+      a.img_fwd = off;
+      off += a.mat_fwd;
+      a.img_adj = off;
+      off += a.mat_adj;
+      for (int gi = 0; gi < a.ngates; ++gi) {
+        p->img0[a.g[gi].op] = (int32_t)(a.img_fwd + a.g[gi].moff);
+        p->img1[a.g[gi].op] = (int32_t)(a.img_adj + a.g[gi].amoff);
+      }
+    } else if (st.kind == kStepMatrixStage) {
+      st.margs.phases = (int32_t)off;
+      for (int op : st.ops)
+        if (is_diag_kind(p->ops[op].kind)) {
+          p->img0[op] = (int32_t)off;
+          off += p->D;
+        }
+    }
+  }
+  p->table_elems = off;
+  for (std::vector<Step>* steps : {&p->steps, &p->fsteps})
+    for (Step& st : *steps) {
+      if (st.kind == kStepMatrixStage) link_matrix_stage(p, st.margs, spare);
+      if (st.kind == kStepDiagRun)
+        for (int g = 0; g < st.run.ngates; ++g) st.run.toff[g] = p->ops[st.run.op[g]].off;
+    }
+}
+
+// one step forward, in -> dst (tmp: scratch state)
+int step_forward(const sfamd_prog* p, const Step& st, const void* table, const void* in, void* dst, void* tmp,
+                 hipStream_t s) {
+  switch (st.kind) {
+    case kStepStage: {
+      const int grid = (int)(st.args.ntiles < p->nwg ? st.args.ntiles : p->nwg);
+      return stage_fwd(p->D, st.K, in, dst, table, st.args, grid, p->dtype, s);
+    }
+    case kStepMatrixStage: {
+      const int groups = (st.margs.ntiles + (1 << st.margs.lgt) - 1) >> st.margs.lgt;
+      return mst_fwd(p->D, st.K, in, dst, table, st.margs, groups < kMaxGrid ? groups : kMaxGrid, p->dtype, s);
+    }
+    case kStepDiagRun:
+      return diag_run_fwd(in, dst, table, st.run, p->dtype, s);
+    default:
+      return apply_op(p->ops[st.op], p->n, p->D, table, in, dst, tmp, p->dtype, s);
+  }
+}
+
+// partial columns that a step's adjoint writes: stages one per workgroup
+int step_columns(const sfamd_prog* p, const Step& st, bool* one_pass) {
+  *one_pass = st.kind == kStepStage || st.kind == kStepMatrixStage;
+  const int nt = st.kind == kStepStage ? st.args.ntiles
+                                       : (st.margs.ntiles + (1 << st.margs.lgt) - 1) >> st.margs.lgt;
+  return *one_pass && nt < p->nwg ? nt : p->nwg;
 }
 
 }  // namespace
@@ -627,7 +1019,7 @@ extern "C" int sfamd_build_gate(int kind, double p0, double p1, int D, int dtype
   b.p1 = p1;
   b.d[0].kind = kind;
   b.d[0].off = 0;
-  b.d[0].img_fwd = b.d[0].img_adj = -1;
+  b.d[0].img0 = b.d[0].img1 = -1;
   return launch_build(b, 1, D, nullptr, out, dtype, (hipStream_t)stream);
 }
 
@@ -710,21 +1102,20 @@ extern "C" int sfamd_prog_create(const sfamd_op_t* ops, int nops, int n, int D, 
   p->nops = nops;
   p->fuse_K = fuse_K;
   int mixed = p->mixed_in;
-  int64_t off = 0, max_state = ipow(D, mixed ? 2 * n : n);
+  int64_t max_state = ipow(D, mixed ? 2 * n : n);
   for (int i = 0; i < nops; ++i) {
     const int st = validate_op(ops[i].kind, ops[i].mode0, ops[i].mode1, n, D);
     if (st != 0) {
       delete p;
       return st;
     }
-    OpPlan op{ops[i].kind, ops[i].mode0, ops[i].mode1, mixed, 0, off};
+    OpPlan op{ops[i].kind, ops[i].mode0, ops[i].mode1, mixed, 0, 0};
     if (op.kind == SFAMD_OP_MIX && mixed) {
       delete p;
       return SFAMD_E_STATE;
     }
     if (op.kind == SFAMD_OP_LOSS && !mixed) op.mix_first = 1;
     if (op.kind == SFAMD_OP_LOSS || op.kind == SFAMD_OP_MIX) mixed = 1;
-    off += table_size(op.kind, D);
     p->ops.push_back(op);
     const int64_t se = ipow(D, mixed ? 2 * n : n);
     if (se > max_state) max_state = se;
@@ -733,23 +1124,8 @@ extern "C" int sfamd_prog_create(const sfamd_op_t* ops, int nops, int n, int D, 
   }
   p->max_state = max_state;
   p->final_mixed = mixed;
-  plan_steps(p);
-  // the fused stages' matrix images follow the operations' entries
-  p->img_fwd.assign(nops, -1);
-  p->img_adj.assign(nops, -1);
-  for (Step& st : p->steps) {
-    if (!st.fused) continue;
-    StageArgs& a = st.args;
-    a.img_fwd = off;
-    off += a.mat_fwd;
-    a.img_adj = off;
-    off += a.mat_adj;
-    for (int gi = 0; gi < a.ngates; ++gi) {
-      p->img_fwd[a.g[gi].op] = (int32_t)(a.img_fwd + a.g[gi].moff);
-      p->img_adj[a.g[gi].op] = (int32_t)(a.img_adj + a.g[gi].amoff);
-    }
-  }
-  p->table_elems = off;
+  plan_program(p);
+  place_table(p);
   p->state_elems.push_back(ipow(D, mixed ? 2 * n : n));
   int64_t nwg = (max_state + kBlock - 1) / kBlock;
   if (nwg > 4096) nwg = 4096;
@@ -797,10 +1173,12 @@ extern "C" int sfamd_prog_build_table(const sfamd_prog_t* p, const double* param
     const int cnt = p->nops - first < kMaxBuildPerLaunch ? p->nops - first : kMaxBuildPerLaunch;
     b.first = first;
     for (int i = 0; i < cnt; ++i) {
-      b.d[i].kind = p->ops[first + i].kind;  // MIX entries build nothing
+      const int op = first + i;
+      b.d[i].kind = p->ops[op].kind |  // MIX entries build nothing
+                    (p->mimg_fwd[op] >= 0 ? kBuildMatrixFwd : 0) | (p->mimg_adj[op] >= 0 ? kBuildMatrixAdj : 0);
       b.d[i].off = (int32_t)p->ops[first + i].off;
-      b.d[i].img_fwd = p->img_fwd[first + i];
-      b.d[i].img_adj = p->img_adj[first + i];
+      b.d[i].img0 = p->img0[op];
+      b.d[i].img1 = p->img1[op];
     }
     RET_IF(launch_build(b, cnt, p->D, params, table, p->dtype, (hipStream_t)stream));
   }
@@ -833,15 +1211,25 @@ extern "C" int sfamd_prog_forward(const sfamd_prog_t* p, int begin, int end, con
     else
       dst = (cur == A) ? B : A;
     if (dst == cur) return SFAMD_E_ARG;
-    const Step& st = p->steps[i];
-    if (st.fused) {
-      int grid = (int)(st.args.ntiles < p->nwg ? st.args.ntiles : p->nwg);
-      RET_IF(stage_fwd(p->D, st.K, cur, dst, table, st.args, grid, p->dtype, s));
-    } else if (st.diag) {
-      RET_IF(diag_run_fwd(cur, dst, table, st.run, p->dtype, s));
-    } else {
-      RET_IF(apply_op(p->ops[st.op], p->n, p->D, table, cur, dst, Ct, p->dtype, s));
-    }
+    RET_IF(step_forward(p, p->steps[i], table, cur, dst, Ct, s));
+    cur = dst;
+  }
+  return 0;
+}
+
+extern "C" int sfamd_prog_run(const sfamd_prog_t* p, const void* table, const void* in, void* out, void* ws,
+                              void* stream) {
+  CHECK_ARG(p);
+  if (p->fsteps.empty())
+    return sfamd_prog_forward(p, 0, (int)p->steps.size(), table, in, out, nullptr, ws, stream);
+  CHECK_ARG(in && out && in != out && ws);
+  char* A = (char*)ws;
+  char* B = A + p->max_state * elem_size(p->dtype);
+  char* Ct = B + p->max_state * elem_size(p->dtype);
+  const void* cur = in;
+  for (size_t i = 0; i < p->fsteps.size(); ++i) {
+    void* dst = i + 1 == p->fsteps.size() ? out : (cur == A ? (void*)B : (void*)A);
+    RET_IF(step_forward(p, p->fsteps[i], table, cur, dst, Ct, (hipStream_t)stream));
     cur = dst;
   }
   return 0;
@@ -867,11 +1255,13 @@ extern "C" int sfamd_prog_adjoint(const sfamd_prog_t* p, int begin, int end, con
     if (!saved[i - begin]) return SFAMD_E_ARG;
     void* dst = (i == begin) ? g_in : ((lam == LA) ? LB : LA);
     const Step& st = p->steps[i];
-    if (st.fused) {
-      // one workgroup per tile at most, one partial column per workgroup
-      const int grid = (int)(st.args.ntiles < nwg ? st.args.ntiles : nwg);
-      RET_IF(stage_adj(p->D, st.K, saved[i - begin], lam, dst, table, st.args, grid, partial, nwg, p->dtype, s));
-    } else if (st.diag) {
+    bool one_pass;
+    const int ncol = step_columns(p, st, &one_pass);
+    if (st.kind == kStepStage) {
+      RET_IF(stage_adj(p->D, st.K, saved[i - begin], lam, dst, table, st.args, ncol, partial, nwg, p->dtype, s));
+    } else if (st.kind == kStepMatrixStage) {
+      RET_IF(mst_adj(p->D, st.K, saved[i - begin], lam, dst, table, st.margs, ncol, partial, nwg, p->dtype, s));
+    } else if (st.kind == kStepDiagRun) {
       RET_IF(diag_run_adj(saved[i - begin], lam, dst, table, st.run, partial, nwg, p->dtype, s));
     } else {
       RET_IF(adjoint_op(p->ops[st.op], p->n, p->D, table, saved[i - begin], lam, dst, T1, T2,
@@ -884,9 +1274,10 @@ extern "C" int sfamd_prog_adjoint(const sfamd_prog_t* p, int begin, int end, con
   ol.n = 0;
   for (int i = begin; i < end; ++i) {
     const Step& st = p->steps[i];
-    const int ncol = st.fused ? (int)(st.args.ntiles < nwg ? st.args.ntiles : nwg) : nwg;
+    bool one_pass;
+    const int ncol = step_columns(p, st, &one_pass);
     for (int op : st.ops) {
-      ol.cols[ol.n] = (uint16_t)(st.fused ? ((unsigned)ncol | kOpColsOnePass) : (unsigned)ncol);
+      ol.cols[ol.n] = (uint16_t)(one_pass ? ((unsigned)ncol | kOpColsOnePass) : (unsigned)ncol);
       ol.ops[ol.n++] = op;
       if (ol.n == kOpListMax) {
         RET_IF(reduce_grads(partial, grads, ol, nwg, s));

@@ -35,14 +35,19 @@ def _elem_bytes(dtype):
 
 
 def default_fuse(n, D):
-    """Local modes per fused stage: the largest K in {3, 2} with a D^K tile of
-    at most 4096 amplitudes (stage kernels exist for cutoffs 2..20)."""
+    """Local modes per fused stage (stage kernels exist for cutoffs 2..20).
+
+    Three, and more at the lowest cutoffs, where a tile of three modes leaves
+    the matrix cores idle and a stage takes few gates: one layer of the layered
+    circuit, forward and adjoint, with 3 / 4 / 5 / 6 local modes took 814 / 787 /
+    487 / 398 us on 10 modes at cutoff 3, 284 / 216 / 253 us on 8 at cutoff 4, 400 /
+    270 / 554 us on 7 at cutoff 5 and 2041 / 1716 us on 8 at cutoff 6, but 133 / 216 us
+    on 5 modes at cutoff 7.  Cutoffs above 16 take two (three keep too few
+    gates' tiles in LDS for the adjoint)."""
     if n < 2 or D < 2 or D > 20:
         return 0
-    for K in (3, 2):
-        if K <= n and D**K <= 4096:
-            return K
-    return 0
+    want = 6 if D <= 3 else 4 if D <= 5 or (D == 6 and n >= 7) else 3 if D <= 16 else 2
+    return min(want, n)
 
 
 class CompiledCircuit:
@@ -155,6 +160,21 @@ class CompiledCircuit:
             _lib.ptr(state_in),
             _lib.ptr(out),
             sv,
+            _lib.ptr(self.ws),
+            self._stream(),
+        )
+        return out
+
+    def run(self, state_in, out=None):
+        """The whole program without checkpoints (nothing is differentiated)."""
+        if out is None:
+            out = self.new_state(self.nsteps)
+        _lib.call(
+            "sfamd_prog_run",
+            self.handle,
+            _lib.ptr(self.table),
+            _lib.ptr(state_in),
+            _lib.ptr(out),
             _lib.ptr(self.ws),
             self._stream(),
         )
@@ -275,7 +295,7 @@ def run_circuit(cc, params, state_in, segment=None):
     cc.build_table(params)
     if cc.nsteps == 0:
         return state_in.clone()
-    return cc.forward(0, cc.nsteps, state_in.detach().contiguous())
+    return cc.run(state_in.detach().contiguous())
 
 
 # --------------------------------------------------------------------- readout
@@ -699,7 +719,10 @@ class GradEvaluator:
     def _enqueue(self):
         cc = self.cc
         cc.build_table(self.params)
-        cc.forward(0, cc.nsteps, self.state_in, out=self.psi, saved=self.saved[: cc.nsteps])
+        if self.forward_only:
+            cc.run(self.state_in, out=self.psi)
+        else:
+            cc.forward(0, cc.nsteps, self.state_in, out=self.psi, saved=self.saved[: cc.nsteps])
         _lib.call(
             "sfamd_fidelity_loss",
             _lib.ptr(self.target),

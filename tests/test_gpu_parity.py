@@ -520,6 +520,44 @@ def test_fused_single_gate_adjoint_matches_unfused_at_large_cutoffs(D):
         assert dg < 1e-5, (op, res[0][2], res[3][2])
 
 
+@pytest.mark.parametrize("dtype", [C128, C64])
+@pytest.mark.parametrize(
+    "n,D,K",
+    # one and several tiles; 1, 2 and 3 blocks of 16 rows and a last lane group with 0..3 amplitudes missing;
+    # column counts below, at and above 16; tile groups (low cutoffs); threads without elements (D = 10, 11)
+    [(3, 2, 3), (7, 3, 6), (6, 4, 4), (5, 5, 4), (7, 5, 3), (5, 8, 3), (4, 9, 3), (4, 10, 3), (3, 11, 3), (4, 13, 3),
+     (4, 16, 3), (3, 17, 3), (3, 20, 3)],
+)
+def test_matrix_core_stages_match_unfused(dtype, n, D, K):
+    """Stages of K >= 3 local modes on random states: the forward sweep with
+    checkpoints, the forward-only program (whose intermediate states have other
+    mode orders), lam_in and the gradients against the unfused kernels on the
+    same gate tables.  A gate is a D-term contraction with unit roundoff u in
+    either path, so a circuit of m gates differs by at most about 8 D m u
+    relative to the largest amplitude or gradient (sums of up to D^n terms in
+    blocks, whose rounding averages out)."""
+    rng = np.random.default_rng(71 + D)
+    ops = [o[:2] for o in circuits.layered(n, 1, rng)]
+    ops += [("BS", (n - 1, 0)), ("K", (0,)), ("D", (n - 1,)), ("R", (n - 1,))]
+    g = torch.Generator().manual_seed(n * 100 + D)
+    st = torch.randn([D] * n, dtype=dtype, generator=g).to(DEV)
+    lam = torch.randn([D] * n, dtype=dtype, generator=g).to(DEV)
+    params = (torch.rand(len(ops), 2, dtype=torch.float64, generator=g) * 0.4).to(DEV)
+    res = []
+    for fuse in (0, K):
+        cc = runtime.CompiledCircuit(ops, n, D, False, dtype, DEV, fuse=fuse)
+        cc.build_table(params)
+        saved = [st] + [cc.new_state(i) for i in range(1, cc.nsteps)]
+        out = cc.forward(0, cc.nsteps, st, saved=saved)
+        gin = cc.new_state(0)
+        grads = torch.zeros(2 * len(ops), dtype=torch.float64, device=DEV)
+        cc.adjoint(0, cc.nsteps, saved, lam, gin, grads)
+        res.append((out, cc.run(st), gin, grads))
+    tol = 8 * D * len(ops) * (2.0**-24 if dtype == C64 else 2.0**-53)
+    for a, b in zip(*res):
+        assert float((a - b).abs().max()) <= tol * float(a.abs().max())
+
+
 def test_fused_gradient_vs_finite_differences_c128():
     n, D = 4, 5
     rng = np.random.default_rng(31)
