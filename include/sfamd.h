@@ -284,7 +284,9 @@ typedef struct {
  * state are grouped into steps that each apply many gates to LDS tiles of
  * fuse_K local modes (gates on disjoint modes commute, so a gate may move to
  * an earlier step when no earlier gate shares a mode); fuse_K = 0 gives one
- * step per operation.  Host memory only. */
+ * step per operation.  With fuse_K | SFAMD_FUSE_MIXED the unitary gates on a
+ * density matrix are grouped the same way.  Host memory only. */
+#define SFAMD_FUSE_MIXED 0x100
 int sfamd_prog_create(const sfamd_op_t* ops, int nops, int n, int D,
                       int mixed_in, int dtype, int fuse_K, sfamd_prog_t** out);
 int sfamd_prog_info(const sfamd_prog_t* prog, sfamd_prog_info_t* info);

@@ -25,6 +25,8 @@ C64, C128 = 0, 1
     OP_CROSS_KERR,
     OP_CUBIC_PHASE,
 ) = range(11)
+FUSE_MIXED = 0x100  # fuse_K flag of sfamd_prog_create: stages on density matrices too
+
 OP_KINDS = {
     "R": OP_ROTATION,
     "K": OP_KERR,

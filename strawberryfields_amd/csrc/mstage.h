@@ -95,7 +95,8 @@ struct MArgs {
   int32_t hl_adj, hl_two;  // the last one
   int32_t lgt;     // log2 of the tiles a workgroup holds at once
   int32_t phases;  // table offset of the rotation / Kerr phases, in gate order
-  int32_t permuted, pad;  // the output's mode order is not the input's
+  int32_t permuted;  // the output's mode order is not the input's
+  int32_t side;      // 1: conjugate gates (column axes of a density matrix), gradients to the second pass
   int64_t loc_stride[kMstMaxK];     // input strides of the local modes, in tile axis order (slowest first)
   int64_t nl_stride[kMstMaxModes];  // input strides of the other modes, fastest first (zeros past nnl)
   // The output's mode order may differ from the input's (forward-only plans):

@@ -1,4 +1,5 @@
-// Fused gate stages on a pure state (ket) with the gates on matrix cores.
+// Fused gate stages with the gates on matrix cores: many gates per pass over a
+// ket, or over a density matrix on one side.
 //
 // A stage is a set of K "local" modes and an ordered list of gates that act
 // only on those modes (R, K, D, S on one local mode; BS on two).  The ket is
@@ -37,6 +38,10 @@
 // sweep multiplies the state by the conjugate phases again.  Parameter sums are
 // reduced per wave by DPP lane moves and per workgroup in a fixed order
 // (deterministic), one partial per workgroup.
+//
+// A density matrix is a ket of 2 n axes: a launch on row axes applies the gates,
+// one on column axes (`side`) their conjugates, as G on the conjugated tile,
+// so both read the same operators.
 #pragma once
 
 #include "mstage.h"
@@ -115,9 +120,11 @@ struct Walk {
   bool mine;           // the thread has elements (the others read element 0 and store nothing)
   unsigned digits;     // inner digits, axis t at bit 5 t
   int64_t goff, base, s0;
+  T im;                // sign of the imaginary parts: conj(G) x = conj(G conj(x))
   bool valid;          // the group's tile exists and the thread has elements
 
-  __device__ __forceinline__ explicit Walk(const sfamd::MArgs& a) : base(0), s0(a.loc_stride[0]), valid(true) {
+  __device__ __forceinline__ explicit Walk(const sfamd::MArgs& a)
+      : base(0), s0(a.loc_stride[0]), im(a.side ? (T)-1 : (T)1), valid(true) {
     tt = (int)threadIdx.x & (Gm::TT - 1);
     const unsigned i = threadIdx.x >> Gm::LG;
     d0 = (int)(i / I);
@@ -180,11 +187,11 @@ struct Walk {
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
       const int d = d0 + j * W;
-      if ((j + 1) * W <= D || d < D) tile[lds + d * S0] = v[j];
+      if ((j + 1) * W <= D || d < D) tile[lds + d * S0] = mk<T>(v[j].re, im * v[j].im);
     }
   }
   __device__ __forceinline__ void store(const C<T>* tile, C<T>* __restrict__ dst) const {
-    if (valid) each([&](int d, int o) { dst[base + (int64_t)d * s0] = tile[o]; });
+    if (valid) each([&](int d, int o) { dst[base + (int64_t)d * s0] = mk<T>(tile[o].re, im * tile[o].im); });
   }
   // The group's tiles to a state whose mode order may differ: the same walk
   // over the tile axes in the output's order, so that neighbouring threads
@@ -628,13 +635,13 @@ k_mst_adj(const C<T>* __restrict__ psi_in, const C<T>* __restrict__ lam_out, C<T
   }
   __syncthreads();
   // one partial per workgroup and gate parameter, at
-  // partial[((op * 2 + 0) * 2 + slot) * nwg + blockIdx.x]; the gradient
-  // reduction reads the launch's gridDim.x columns of pass 0 only
+  // partial[((op * 2 + side) * 2 + slot) * nwg + blockIdx.x]; the gradient
+  // reduction reads the launch's gridDim.x columns
   for (int idx = threadIdx.x; idx < 2 * a.ngates; idx += NT) {
     const int gi = idx >> 1, slot = idx & 1;
     double s = 0.0;
     for (int w = 0; w < NW; ++w) s += gsl[idx * NW + w];
-    partial[((int64_t)a.g[gi].op * 4 + slot) * nwg + blockIdx.x] = s;
+    partial[((int64_t)a.g[gi].op * 4 + a.side * 2 + slot) * nwg + blockIdx.x] = s;
   }
 }
 

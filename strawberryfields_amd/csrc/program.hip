@@ -299,7 +299,9 @@ int adjoint_op(const OpPlan& op, int n, int D, const void* table, const void* ps
 
 // One step of execution: a single operation (or a run of diagonal gates), or a
 // fused stage of gates on K local modes of a pure state: on the vector ALUs
-// (K = 2, fused.hip) or on the matrix cores (K >= 3, mstage.hip).
+// (K = 2, fused.hip) or on the matrix cores (K >= 3, mstage.hip).  On a density
+// matrix a matrix-core stage is two launches: the gates on the row axes of its
+// modes, then their conjugates on the column axes.
 enum StepKind { kStepSingle = 0, kStepDiagRun, kStepStage, kStepMatrixStage };
 struct Step {
   int kind;
@@ -307,12 +309,13 @@ struct Step {
   int K;
   std::vector<int> ops;  // operation indices in execution order
   StageArgs args;
-  MArgs margs;
+  MArgs margs[2];  // [1]: the column axes of a density matrix
+  bool mixed;      // the stage acts on a density matrix
   DiagRun run;
 };
 
 struct sfamd_prog {
-  int n, D, dtype, mixed_in, nops, nwg, fuse_K;
+  int n, D, dtype, mixed_in, nops, nwg, fuse_K, fuse_mixed;
   std::vector<OpPlan> ops;
   std::vector<int32_t> img0, img1;          // per op: its vector-ALU stage images, or copies of its phases; -1: none
   std::vector<int32_t> mimg_fwd, mimg_adj;  // per op: its matrix-core images, or -1
@@ -328,10 +331,18 @@ struct sfamd_prog {
 namespace {
 
 bool fusable(const OpPlan& op) {
-  return !op.mixed_in && (op.kind == SFAMD_OP_ROTATION || op.kind == SFAMD_OP_KERR ||
-                          op.kind == SFAMD_OP_DISPLACEMENT || op.kind == SFAMD_OP_SQUEEZE ||
-                          op.kind == SFAMD_OP_BEAMSPLITTER);
+  return op.kind == SFAMD_OP_ROTATION || op.kind == SFAMD_OP_KERR || op.kind == SFAMD_OP_DISPLACEMENT ||
+         op.kind == SFAMD_OP_SQUEEZE || op.kind == SFAMD_OP_BEAMSPLITTER;
 }
+
+// The stages of one representation: its axes (n of a ket, 2 n of a density
+// matrix: row and column of each mode in turn, slowest first), the kind of its
+// stages and their local axes (0: no stages).
+struct Stages {
+  bool mixed;
+  int axes, kind, Kc;
+  int modes(int n) const { return Kc < n ? Kc : n; }  // that a stage takes gates of
+};
 
 int op_nmodes(const OpPlan& op) { return two_mode_kind(op.kind) ? 2 : 1; }
 
@@ -387,6 +398,7 @@ Step new_step(int kind, int op) {
   st.kind = kind;
   st.op = op;
   st.K = 0;
+  st.mixed = false;
   memset(&st.args, 0, sizeof(st.args));
   memset(&st.margs, 0, sizeof(st.margs));
   memset(&st.run, 0, sizeof(st.run));
@@ -398,9 +410,9 @@ constexpr int kMstGatesForTwo = 4;            // gates each of two workgroups pe
 // log2 of the tiles a workgroup of a matrix-core stage holds: as many as fill
 // the 16 columns of a beamsplitter's matrix-core operand, if every CU still
 // has a group
-int group_log2(const sfamd_prog* p, int Kc) {
+int group_log2(const sfamd_prog* p, int axes, int Kc) {
   const int D = p->D;
-  const int64_t ntiles = ipow(D, p->n - Kc);
+  const int64_t ntiles = ipow(D, axes - Kc);
   int l = 0;
   while (mst_group_ok(D, Kc, l + 1) && (mst_tile(D, Kc) / (D * D) << l) <= 8 && (ntiles >> (l + 1)) >= kComputeUnits)
     ++l;
@@ -411,12 +423,12 @@ int group_log2(const sfamd_prog* p, int Kc) {
 // three and every gate's matrices (the adjoint kernel's LDS).
 // kStepMatrixStage: the adjoint keeps one tile per gate with operators plus two,
 // the forward-only plan one tile group.
-StageCost stage_cost(const sfamd_prog* p, int kind, int Kc, bool forward_only) {
-  const int D = p->D;
+StageCost stage_cost(const sfamd_prog* p, const Stages& sg, bool forward_only) {
+  const int D = p->D, kind = sg.kind, Kc = sg.Kc;
   const int64_t esz = elem_size(p->dtype);
   // a launch has one workgroup per tile (up to the grid cap): when that is
   // more than one per compute unit, two should fit in a CU's LDS at once
-  const bool many = ipow(D, p->n - Kc) > kComputeUnits;
+  const bool many = ipow(D, sg.axes - Kc) > kComputeUnits;
   StageCost sc;
   sc.budget_full = kStageLdsBudget;
   sc.budget = many ? kStageLdsPerCu / 2 - 512 : kStageLdsBudget;
@@ -429,11 +441,11 @@ StageCost stage_cost(const sfamd_prog* p, int kind, int Kc, bool forward_only) {
     };
     return sc;
   }
-  const int lgt = group_log2(p, Kc);
+  const int lgt = group_log2(p, sg.axes, Kc);
   const int64_t tile = ((int64_t)mst_tile_lds(D, Kc) << lgt) * esz, phases = (int64_t)(D + 1) * esz;
   sc.max_gates = kMstMaxGates;
   sc.budget_full = kMstLdsMax;
-  if ((ipow(D, p->n - Kc) >> lgt) <= kComputeUnits) sc.budget = sc.budget_full;
+  if ((ipow(D, sg.axes - Kc) >> lgt) <= kComputeUnits) sc.budget = sc.budget_full;
   if (forward_only) {
     sc.base = tile;
     sc.budget = sc.budget_full;
@@ -449,13 +461,15 @@ StageCost stage_cost(const sfamd_prog* p, int kind, int Kc, bool forward_only) {
 }
 
 // Can a stage of this kind hold one gate of any kind?
-bool stage_fits(const sfamd_prog* p, int kind, int Kc, bool forward_only) {
-  if (Kc < 2 || Kc > p->n) return false;
-  if (kind == kStepStage ? (p->n > kStageMaxModes || !stage_supported(p->D, Kc))
-                         : (p->n > kMstMaxModes || !mst_supported(p->D, Kc)))
+bool stage_fits(const sfamd_prog* p, const Stages& sg, bool forward_only) {
+  if (sg.Kc < 2 || sg.Kc > sg.axes) return false;
+  if (sg.kind == kStepStage ? (sg.mixed || sg.axes > kStageMaxModes || !stage_supported(p->D, sg.Kc))
+                            : (sg.axes > kMstMaxModes || !mst_supported(p->D, sg.Kc)))
     return false;
-  if (ipow(p->D, p->n - Kc) >= ((int64_t)1 << 31)) return false;
-  const StageCost sc = stage_cost(p, kind, Kc, forward_only);
+  int64_t tiles = 1;
+  for (int i = sg.Kc; i < sg.axes; ++i)
+    if ((tiles *= p->D) >= ((int64_t)1 << 31)) return false;
+  const StageCost sc = stage_cost(p, sg, forward_only);
   OpPlan bs{SFAMD_OP_BEAMSPLITTER, 0, 1, 0, 0, 0};
   return sc.base + sc.gate(bs) <= sc.budget_full;
 }
@@ -519,13 +533,14 @@ ModeOrder canonical_order(int n, int D) {
   return o;
 }
 
-// a matrix-core stage on the modes of `mask`, from states in mode order `in` to
-// states in mode order `out`
-void fill_matrix_stage(const sfamd_prog* p, Step& st, unsigned mask, bool forward_only, const ModeOrder& in,
-                       const ModeOrder& out) {
-  const int n = p->n, D = p->D, Kc = st.K;
-  MArgs& a = st.margs;
+// a matrix-core stage on the axes of `mask`, from states in axis order `in` to
+// states in axis order `out`; side 1: on the column axes of a density matrix
+void fill_matrix_stage(const sfamd_prog* p, Step& st, unsigned mask, const ModeOrder& in, const ModeOrder& out,
+                       int side) {
+  const int n = in.n, D = p->D, Kc = st.K;
+  MArgs& a = st.margs[side];
   memset(&a, 0, sizeof(a));
+  a.side = side;
   a.ngates = (int)st.ops.size();
   int lmodes[kMstMaxK], nl = 0;
   for (int i = n - 1; i >= 0; --i)  // fastest first
@@ -536,7 +551,7 @@ void fill_matrix_stage(const sfamd_prog* p, Step& st, unsigned mask, bool forwar
   for (int i = 0; i < n; ++i)  // slowest first
     if (mask >> in.at[i] & 1u) lmodes[nl++] = in.at[i];
   a.ntiles = (int32_t)ipow(D, a.nnl);
-  a.lgt = group_log2(p, Kc);
+  a.lgt = group_log2(p, n, Kc);
   for (int t = 0; t < Kc; ++t) a.loc_stride[t] = in.stride[lmodes[t]];
   int u = 0;
   for (int i = 0; i < n; ++i)
@@ -550,9 +565,10 @@ void fill_matrix_stage(const sfamd_prog* p, Step& st, unsigned mask, bool forwar
     MGate& g = a.g[gi];
     const bool two = op.kind == SFAMD_OP_BEAMSPLITTER;
     int ax0 = 0, ax1 = -1;
+    const int m0 = st.mixed ? 2 * op.m0 + side : op.m0, m1 = st.mixed ? 2 * op.m1 + side : op.m1;
     for (int t = 0; t < Kc; ++t) {
-      if (lmodes[t] == op.m0) ax0 = t;
-      if (two && lmodes[t] == op.m1) ax1 = t;
+      if (lmodes[t] == m0) ax0 = t;
+      if (two && lmodes[t] == m1) ax1 = t;
     }
     int u = 0;
     for (int t = 0; t < Kc; ++t)
@@ -568,6 +584,24 @@ void fill_matrix_stage(const sfamd_prog* p, Step& st, unsigned mask, bool forwar
       ++a.ndiag;
     else
       ++a.nheavy;
+  }
+}
+
+// a matrix-core stage on the modes of `mask`, both states in the canonical axis
+// order: on a density matrix both its sides, the tile completed by the fastest
+// other axes where the modes are fewer than the local axes
+void fill_matrix_step(const sfamd_prog* p, Step& st, unsigned mask) {
+  const int axes = st.mixed ? 2 * p->n : p->n;
+  const ModeOrder order = canonical_order(axes, p->D);
+  for (int side = 0; side <= (st.mixed ? 1 : 0); ++side) {
+    unsigned m = mask;
+    if (st.mixed) {
+      m = 0;
+      for (int md = 0; md < p->n; ++md)
+        if (mask >> md & 1u) m |= 1u << (2 * md + side);
+      for (int a = axes - 1; __builtin_popcount(m) < st.K; --a) m |= 1u << a;
+    }
+    fill_matrix_stage(p, st, m, order, order, side);
   }
 }
 
@@ -647,8 +681,8 @@ void order_stages(const sfamd_prog* p, std::vector<Step>* steps, size_t first, s
         }
       out.set_strides(D);
     }
-    MArgs& a = (*steps)[first + i].margs;
-    fill_matrix_stage(p, (*steps)[first + i], masks[i], true, in, out);
+    MArgs& a = (*steps)[first + i].margs[0];
+    fill_matrix_stage(p, (*steps)[first + i], masks[i], in, out, 0);
     a.permuted = 1;
     // no shared mode: the workgroup takes neighbouring tiles, for runs of that many amplitudes
     if (a.out_stride[(*steps)[first + i].K - 1] != 1)
@@ -660,13 +694,12 @@ void order_stages(const sfamd_prog* p, std::vector<Step>* steps, size_t first, s
 }
 
 // greedy partition of a run of fusable ops into stages of Kc local modes
-void plan_run(const sfamd_prog* p, const std::vector<int>& run, int kind, int Kc, bool forward_only,
+void plan_run(const sfamd_prog* p, const std::vector<int>& run, const Stages& sg, bool forward_only,
               std::vector<Step>* steps) {
-  const int n = p->n;
-  const StageCost sc = stage_cost(p, kind, Kc, forward_only);
-  const ModeOrder order = canonical_order(n, p->D);
-  std::vector<unsigned> masks;   // of this run's steps
-  std::vector<size_t> stages;    // its matrix-core stages
+  const int n = p->n, kind = sg.kind, Kc = sg.modes(n);
+  const StageCost sc = stage_cost(p, sg, forward_only);
+  std::vector<unsigned> masks;  // of this run's steps
+  size_t nstages = 0;           // its matrix-core stages
   std::vector<int> rem = run;
   std::vector<unsigned> cands;
   // all Kc-subsets when few, else subsets grown from the next ops
@@ -742,15 +775,16 @@ void plan_run(const sfamd_prog* p, const std::vector<int>& run, int kind, int Kc
       continue;
     }
     Step st = new_step(kind, best.front());
-    st.K = Kc;
+    st.K = sg.Kc;
+    st.mixed = sg.mixed;
     st.ops = best;
     if (kind == kStepStage)
       fill_stage(p, st, bm);
     else
-      fill_matrix_stage(p, st, bm, forward_only, order, order);
+      fill_matrix_step(p, st, bm);
     steps->push_back(st);
     masks.push_back(bm);
-    if (kind == kStepMatrixStage) stages.push_back(steps->size() - 1);
+    nstages += kind == kStepMatrixStage;
     std::vector<int> nrem;
     size_t bi = 0;
     for (int i : rem) {
@@ -761,25 +795,16 @@ void plan_run(const sfamd_prog* p, const std::vector<int>& run, int kind, int Kc
     }
     rem.swap(nrem);
   }
-  if (forward_only && kind == kStepMatrixStage && stages.size() == masks.size())
+  if (forward_only && !sg.mixed && nstages == masks.size())
     order_stages(p, steps, steps->size() - masks.size(), masks);
 }
 
-// `kind`, Kc: the stages of the plan (Kc = 0: none)
-void plan_steps(const sfamd_prog* p, int kind, int Kc, bool forward_only, std::vector<Step>* steps) {
+// sg: the stages on kets and on density matrices
+void plan_steps(const sfamd_prog* p, const Stages (&sg)[2], bool forward_only, std::vector<Step>* steps) {
   const int n = p->n, D = p->D;
-  std::vector<int> run;
-  auto flush = [&]() {
-    if (!run.empty()) plan_run(p, run, kind, Kc, forward_only, steps);
-    run.clear();
-  };
   auto is_diag = [&](int i) { return is_diag_kind(p->ops[i].kind); };
-  for (int i = 0; i < p->nops; ++i) {
-    if (Kc >= 2 && fusable(p->ops[i])) {
-      run.push_back(i);
-      continue;
-    }
-    flush();
+  std::vector<int> run;
+  auto single = [&](int i) {
     // consecutive rotation / Kerr gates on the same representation share one pass
     if (is_diag(i) && !steps->empty()) {
       Step& last = steps->back();
@@ -787,12 +812,33 @@ void plan_steps(const sfamd_prog* p, int kind, int Kc, bool forward_only, std::v
           p->ops[last.ops.back()].mixed_in == p->ops[i].mixed_in && (int)last.ops.size() < kDiagRunMax) {
         last.ops.push_back(i);
         last.kind = kStepDiagRun;
-        continue;
+        return;
       }
     }
     Step st = new_step(kStepSingle, i);
     st.ops.push_back(i);
     steps->push_back(st);
+  };
+  auto flush = [&]() {
+    if (run.empty()) return;
+    const Stages& g = sg[p->ops[run.front()].mixed_in];
+    // on a density matrix rotation and Kerr gates alone take one pass, a stage two
+    bool heavy = !g.mixed;
+    for (int i : run) heavy = heavy || !is_diag(i);
+    if (heavy)
+      plan_run(p, run, g, forward_only, steps);
+    else
+      for (int i : run) single(i);
+    run.clear();
+  };
+  for (int i = 0; i < p->nops; ++i) {
+    if (sg[p->ops[i].mixed_in].Kc >= 2 && fusable(p->ops[i])) {
+      if (!run.empty() && p->ops[run.front()].mixed_in != p->ops[i].mixed_in) flush();
+      run.push_back(i);
+      continue;
+    }
+    flush();
+    single(i);
   }
   flush();
   for (Step& st : *steps) {
@@ -838,28 +884,52 @@ bool stages_pay(const sfamd_prog* p, int kind, bool forward_only) {
   return D <= 8 || mb < 32 * wide;
 }
 
+// Stages on a density matrix against one or two passes per gate.  The adjoint
+// of a stage is five launches (rows, then columns, forward again and backward)
+// and holds few gates where a tile of cutoff 13 and more fills the LDS; the
+// column of every mode strides over the rows of the others, so large states
+// lose.  One layer of the noisy layered circuit, forward and adjoint, unfused /
+// staged, us: complex64, 2 modes cutoff 8 177 / 91, 12 225 / 159, 16 313 / 259, 18
+// 421 / 676; 3 modes 6 475 / 190, 8 679 / 176, 10 1167 / 668, 12 1763 / 1560, 13 2593 /
+// 3319, 16 5886 / 10204; complex128, 2 modes 12 374 / 220; 3 modes 8 849 / 247, 12
+// 4109 / 2633, 13 6514 / 7735.  Forward only they always pay: 3 modes cutoff 16,
+// complex64 1780 / 1356, complex128 5537 / 2387; 2 modes 20 159 / 134 and 442 / 242.
+bool dm_stages_pay(const sfamd_prog* p, bool forward_only) {
+  if (forward_only || p->D <= 12) return true;
+  return p->D <= 16 && p->n == 2;
+}
+
 // The stages of a plan for a requested number of local modes: matrix-core
 // stages for three and more, vector-ALU stages for two (a beamsplitter on two
 // local modes has one column, so a matrix-core operand would be 15/16 empty) and
-// where the matrix-core adjoint's tiles exceed the LDS.
-void pick_stages(const sfamd_prog* p, bool forward_only, int* kind, int* Kc) {
+// where the matrix-core adjoint's tiles exceed the LDS.  On a density matrix a
+// stage of fewer modes has the other side's axes for columns.
+Stages pick_stages(const sfamd_prog* p, bool forward_only, bool mixed) {
   const int K = p->fuse_K < p->n ? p->fuse_K : p->n;
-  *kind = kStepMatrixStage;
-  *Kc = K;
-  if (K >= 3 && stage_fits(p, kStepMatrixStage, K, forward_only)) {
-    if (!stages_pay(p, kStepMatrixStage, forward_only)) *Kc = 0;
-    return;
+  Stages sg{mixed, mixed ? 2 * p->n : p->n, kStepMatrixStage, K};
+  if (mixed) {
+    sg.Kc = p->fuse_K < 3 ? 3 : p->fuse_K < sg.axes ? p->fuse_K : sg.axes;
+    if (!p->fuse_mixed || p->fuse_K < 2 || p->n < 2 || !stage_fits(p, sg, forward_only) || !dm_stages_pay(p, forward_only)) sg.Kc = 0;
+    return sg;
   }
-  *kind = kStepStage;
-  *Kc = K >= 2 && stage_fits(p, kStepStage, 2, false) && (p->fuse_K == 2 || stages_pay(p, kStepStage, false)) ? 2 : 0;
+  if (K >= 3 && stage_fits(p, sg, forward_only)) {
+    if (!stages_pay(p, kStepMatrixStage, forward_only)) sg.Kc = 0;
+    return sg;
+  }
+  sg.kind = kStepStage;
+  sg.Kc = 2;
+  if (K < 2 || !stage_fits(p, sg, false) || !(p->fuse_K == 2 || stages_pay(p, kStepStage, false))) sg.Kc = 0;
+  return sg;
 }
 
 void plan_program(sfamd_prog* p) {
-  int kind, Kc, fkind, fKc;
-  pick_stages(p, false, &kind, &Kc);
-  plan_steps(p, kind, Kc, false, &p->steps);
-  pick_stages(p, true, &fkind, &fKc);
-  if (fKc >= 3 && fkind == kStepMatrixStage) plan_steps(p, fkind, fKc, true, &p->fsteps);
+  const Stages both[2] = {pick_stages(p, false, false), pick_stages(p, false, true)};
+  plan_steps(p, both, false, &p->steps);
+  const Stages fwd[2] = {pick_stages(p, true, false), pick_stages(p, true, true)};
+  bool matrix = false;
+  for (const OpPlan& op : p->ops)
+    matrix = matrix || (fwd[op.mixed_in].Kc >= 3 && fwd[op.mixed_in].kind == kStepMatrixStage && fusable(op));
+  if (matrix) plan_steps(p, fwd, true, &p->fsteps);
   // state sizes at step inputs
   p->state_elems.clear();
   for (const Step& st : p->steps) {
@@ -912,7 +982,7 @@ void place_table(sfamd_prog* p) {
   if (matrix) off += 2 * mst_img(p->D);
   for (Step& st : p->fsteps) {
     if (st.kind != kStepMatrixStage) continue;
-    st.margs.phases = (int32_t)off;
+    st.margs[0].phases = st.margs[1].phases = (int32_t)off;
     for (int op : st.ops)
       if (in_phases[op]) {
         p->ops[op].off = off;
@@ -931,7 +1001,7 @@ void place_table(sfamd_prog* p) {
         p->img1[a.g[gi].op] = (int32_t)(a.img_adj + a.g[gi].amoff);
       }
     } else if (st.kind == kStepMatrixStage) {
-      st.margs.phases = (int32_t)off;
+      st.margs[0].phases = st.margs[1].phases = (int32_t)off;
       for (int op : st.ops)
         if (is_diag_kind(p->ops[op].kind)) {
           p->img0[op] = (int32_t)off;
@@ -940,9 +1010,14 @@ void place_table(sfamd_prog* p) {
     }
   }
   p->table_elems = off;
+  // vector-ALU stages are the same in both plans
+  for (Step& f : p->fsteps)
+    for (size_t i = 0; f.kind == kStepStage && i < p->steps.size(); ++i)
+      if (p->steps[i].kind == kStepStage && p->steps[i].op == f.op) f.args = p->steps[i].args;
   for (std::vector<Step>* steps : {&p->steps, &p->fsteps})
     for (Step& st : *steps) {
-      if (st.kind == kStepMatrixStage) link_matrix_stage(p, st.margs, spare);
+      if (st.kind == kStepMatrixStage)
+        for (int side = 0; side <= (st.mixed ? 1 : 0); ++side) link_matrix_stage(p, st.margs[side], spare);
       if (st.kind == kStepDiagRun)
         for (int g = 0; g < st.run.ngates; ++g) st.run.toff[g] = p->ops[st.run.op[g]].off;
     }
@@ -957,8 +1032,11 @@ int step_forward(const sfamd_prog* p, const Step& st, const void* table, const v
       return stage_fwd(p->D, st.K, in, dst, table, st.args, grid, p->dtype, s);
     }
     case kStepMatrixStage: {
-      const int groups = (st.margs.ntiles + (1 << st.margs.lgt) - 1) >> st.margs.lgt;
-      return mst_fwd(p->D, st.K, in, dst, table, st.margs, groups < kMaxGrid ? groups : kMaxGrid, p->dtype, s);
+      const MArgs& a = st.margs[0];
+      const int groups = (a.ntiles + (1 << a.lgt) - 1) >> a.lgt, grid = groups < kMaxGrid ? groups : kMaxGrid;
+      if (!st.mixed) return mst_fwd(p->D, st.K, in, dst, table, a, grid, p->dtype, s);
+      RET_IF(mst_fwd(p->D, st.K, in, tmp, table, a, grid, p->dtype, s));
+      return mst_fwd(p->D, st.K, tmp, dst, table, st.margs[1], grid, p->dtype, s);
     }
     case kStepDiagRun:
       return diag_run_fwd(in, dst, table, st.run, p->dtype, s);
@@ -967,12 +1045,14 @@ int step_forward(const sfamd_prog* p, const Step& st, const void* table, const v
   }
 }
 
-// partial columns that a step's adjoint writes: stages one per workgroup
+// partial columns that a step's adjoint writes, and whether only for one pass:
+// stages one per workgroup
 int step_columns(const sfamd_prog* p, const Step& st, bool* one_pass) {
-  *one_pass = st.kind == kStepStage || st.kind == kStepMatrixStage;
+  const bool stage = st.kind == kStepStage || st.kind == kStepMatrixStage;
+  *one_pass = stage && !st.mixed;
   const int nt = st.kind == kStepStage ? st.args.ntiles
-                                       : (st.margs.ntiles + (1 << st.margs.lgt) - 1) >> st.margs.lgt;
-  return *one_pass && nt < p->nwg ? nt : p->nwg;
+                                       : (st.margs[0].ntiles + (1 << st.margs[0].lgt) - 1) >> st.margs[0].lgt;
+  return stage && nt < p->nwg ? nt : p->nwg;
 }
 
 }  // namespace
@@ -1100,7 +1180,8 @@ extern "C" int sfamd_prog_create(const sfamd_op_t* ops, int nops, int n, int D, 
   p->dtype = dtype;
   p->mixed_in = mixed_in ? 1 : 0;
   p->nops = nops;
-  p->fuse_K = fuse_K;
+  p->fuse_K = fuse_K & ~SFAMD_FUSE_MIXED;
+  p->fuse_mixed = (fuse_K & SFAMD_FUSE_MIXED) != 0;
   int mixed = p->mixed_in;
   int64_t max_state = ipow(D, mixed ? 2 * n : n);
   for (int i = 0; i < nops; ++i) {
@@ -1260,7 +1341,13 @@ extern "C" int sfamd_prog_adjoint(const sfamd_prog_t* p, int begin, int end, con
     if (st.kind == kStepStage) {
       RET_IF(stage_adj(p->D, st.K, saved[i - begin], lam, dst, table, st.args, ncol, partial, nwg, p->dtype, s));
     } else if (st.kind == kStepMatrixStage) {
-      RET_IF(mst_adj(p->D, st.K, saved[i - begin], lam, dst, table, st.margs, ncol, partial, nwg, p->dtype, s));
+      const void *psi = saved[i - begin], *lo = lam;
+      if (st.mixed) {  // the rows again, the columns backward, the rows backward
+        RET_IF(mst_fwd(p->D, st.K, psi, T1, table, st.margs[0], ncol, p->dtype, s));
+        RET_IF(mst_adj(p->D, st.K, T1, lam, T2, table, st.margs[1], ncol, partial, nwg, p->dtype, s));
+        lo = T2;
+      }
+      RET_IF(mst_adj(p->D, st.K, psi, lo, dst, table, st.margs[0], ncol, partial, nwg, p->dtype, s));
     } else if (st.kind == kStepDiagRun) {
       RET_IF(diag_run_adj(saved[i - begin], lam, dst, table, st.run, partial, nwg, p->dtype, s));
     } else {

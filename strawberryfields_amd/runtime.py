@@ -54,7 +54,7 @@ class CompiledCircuit:
     """A planned circuit (structure only) bound to one device and dtype.
 
     The plan is a list of steps: fused stages (many gates on LDS tiles of
-    ``fuse`` local modes, pure states) or single operations.  Checkpoints and
+    ``fuse`` local modes) or single operations.  Checkpoints and
     segments are expressed in steps; gradients are indexed by operation.
     """
 
@@ -73,8 +73,9 @@ class CompiledCircuit:
             arr[i].pad = 0
         handle = ctypes.c_void_p()
         self.fuse = default_fuse(self.n, self.D) if fuse is None else int(fuse)
+        fuse_K = self.fuse | _lib.FUSE_MIXED if self.fuse >= 2 else self.fuse
         st = self.lib.sfamd_prog_create(
-            arr, len(self.ops), self.n, self.D, int(self.mixed_in), self.code, self.fuse, ctypes.byref(handle)
+            arr, len(self.ops), self.n, self.D, int(self.mixed_in), self.code, fuse_K, ctypes.byref(handle)
         )
         _lib.check(st, "sfamd_prog_create")
         self.handle = handle

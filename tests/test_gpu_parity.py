@@ -558,6 +558,44 @@ def test_matrix_core_stages_match_unfused(dtype, n, D, K):
         assert float((a - b).abs().max()) <= tol * float(a.abs().max())
 
 
+@pytest.mark.parametrize("dtype", [C128, C64])
+@pytest.mark.parametrize(
+    "n,D,K,mixed",
+    # fewer modes than local axes (the tile completed by the other side's axes), an adjoint plan of
+    # its own next to a longer forward-only one, a pure start with stages on both representations,
+    # cutoffs with and without a staged adjoint, low cutoffs with tile groups and wide tiles
+    [(2, 4, 2, True), (2, 7, 2, False), (2, 16, 2, True), (2, 20, 2, True), (3, 3, 3, True), (3, 4, 5, True),
+     (3, 6, 3, False), (3, 9, 3, True), (3, 13, 3, True), (4, 3, 4, False)],
+)
+def test_density_matrix_stages_match_unfused(dtype, n, D, K, mixed):
+    """Stages on the row and column axes of a density matrix on random states
+    (not Hermitian ones): forward with checkpoints, forward-only program, lam_in
+    and the gradients against the unfused kernels.  Every gate is two D-term
+    contractions in either path, so a circuit of m gates differs by at most
+    about 16 D m u relative to the largest entry (a loss is a sum of at most D
+    terms too)."""
+    rng = np.random.default_rng(81 + D)
+    ops = [o[:2] for o in circuits.layered(n, 1, rng, loss=True)]
+    ops += [("BS", (n - 1, 0)), ("K", (0,)), ("R", (1,)), ("LOSS", (1,)), ("D", (n - 1,)), ("S", (0,)), ("R", (n - 1,))]
+    g = torch.Generator().manual_seed(n * 100 + D)
+    st = torch.randn([D] * (2 * n if mixed else n), dtype=dtype, generator=g).to(DEV)
+    lam = torch.randn([D] * (2 * n), dtype=dtype, generator=g).to(DEV)
+    params = (torch.rand(len(ops), 2, dtype=torch.float64, generator=g) * 0.4).to(DEV)
+    res = []
+    for fuse in (0, K):
+        cc = runtime.CompiledCircuit(ops, n, D, mixed, dtype, DEV, fuse=fuse)
+        cc.build_table(params)
+        saved = [st] + [cc.new_state(i) for i in range(1, cc.nsteps)]
+        out = cc.forward(0, cc.nsteps, st, saved=saved)
+        gin = cc.new_state(0)
+        grads = torch.zeros(2 * len(ops), dtype=torch.float64, device=DEV)
+        cc.adjoint(0, cc.nsteps, saved, lam, gin, grads)
+        res.append((out, cc.run(st), gin, grads))
+    tol = 16 * D * len(ops) * (2.0**-24 if dtype == C64 else 2.0**-53)
+    for a, b in zip(*res):
+        assert float((a - b).abs().max()) <= tol * float(a.abs().max())
+
+
 def test_fused_gradient_vs_finite_differences_c128():
     n, D = 4, 5
     rng = np.random.default_rng(31)
