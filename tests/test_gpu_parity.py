@@ -596,6 +596,36 @@ def test_density_matrix_stages_match_unfused(dtype, n, D, K, mixed):
         assert float((a - b).abs().max()) <= tol * float(a.abs().max())
 
 
+@pytest.mark.parametrize("keep_always", [None, 0])
+@pytest.mark.parametrize("segment", [None, 1, 3])
+def test_kept_step_inputs_give_the_recomputed_gradients(segment, keep_always, monkeypatch):
+    """The step inputs that the forward keeps are those the backward would
+    recompute with the same kernels: gradients are bit-identical for every
+    segment length, below and above the size that is kept without a look at the
+    free memory, with none kept, and in a second backward of a retained graph."""
+    if keep_always is not None:
+        monkeypatch.setattr(runtime, "KEEP_ALWAYS", keep_always)
+    n, D = 4, 6
+    rng = np.random.default_rng(91)
+    ops = [o[:2] for o in circuits.layered(n, 2, rng)]
+    cc = runtime.CompiledCircuit(ops, n, D, False, C64, DEV, fuse=2)
+    vac = torch.zeros([D] * n, dtype=C64, device=DEV)
+    vac.view(-1)[0] = 1.0
+    p0 = torch.tensor(rng.uniform(0, 0.4, (len(ops), 2)), dtype=torch.float64, device=DEV)
+    res = []
+    for kept in (True, False):
+        if not kept:
+            monkeypatch.setattr(runtime.CompiledCircuit, "keeps_inputs", lambda self, b, e: False)
+        p = p0.clone().requires_grad_(True)
+        loss = runtime.run_circuit(cc, p, vac, segment)[..., 1].abs().square().sum()
+        for again in (True, False):
+            p.grad = None
+            loss.backward(retain_graph=again)
+            res.append(p.grad)
+    for g in res[1:]:
+        assert torch.equal(g, res[0])
+
+
 def test_fused_gradient_vs_finite_differences_c128():
     n, D = 4, 5
     rng = np.random.default_rng(31)
