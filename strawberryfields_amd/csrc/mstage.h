@@ -63,6 +63,14 @@ __host__ __device__ constexpr int mst_waves(int D, int K, int lgt) {
   while (64 * w < (mst_tile(D, K) / D << lgt) && w < 16) w *= 2;
   return w;
 }
+// Do the registers of the adjoint kernel let two workgroups share a compute
+// unit (8 waves each: 128 vector registers per lane)?  At cutoffs 9 to 12 in
+// complex64 the compiler is held to that (131 without: 6 modes, cutoff 9,
+// forward and adjoint 991 -> 842 us); complex128 needs 205 there, complex64 172
+// and more from cutoff 13 on.
+__host__ __device__ constexpr bool mst_two_groups(int D, int dtype) {
+  return D <= 8 || (D <= 12 && dtype == SFAMD_C64);
+}
 // kernels exist for groups of 2^lgt tiles up to 1024 inner elements
 __host__ __device__ constexpr bool mst_group_ok(int D, int K, int lgt) {
   return lgt <= kMstMaxLgt && (mst_tile(D, K) / D << lgt) <= 1024 && (lgt == 0 || mst_tile(D, K) << lgt <= 16384);

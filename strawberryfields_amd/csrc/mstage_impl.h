@@ -575,8 +575,15 @@ __device__ __forceinline__ void gate_adj(const Gate& g, int gi, const C<T>* __re
   __syncthreads();
 }
 
+// waves per SIMD that the adjoint kernel's registers must allow
 template <typename T, typename Gm>
-__global__ void __launch_bounds__(Gm::NT)
+constexpr int adj_waves() {
+  return (sfamd::mst_two_groups(Gm::D, sizeof(T) == 4 ? SFAMD_C64 : SFAMD_C128) && Gm::LG == 0 && Gm::NW == 8) ? 4
+                                                                                                    : (Gm::NW + 3) / 4;
+}
+
+template <typename T, typename Gm>
+__global__ void __launch_bounds__(Gm::NT, (adj_waves<T, Gm>()))
 k_mst_adj(const C<T>* __restrict__ psi_in, const C<T>* __restrict__ lam_out, C<T>* __restrict__ lam_in,
           const C<T>* __restrict__ table, sfamd::MArgs a, double* __restrict__ partial, int nwg) {
   constexpr int NW = Gm::NW, NT = Gm::NT;

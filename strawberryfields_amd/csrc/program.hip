@@ -453,8 +453,9 @@ StageCost stage_cost(const sfamd_prog* p, const Stages& sg, bool forward_only) {
     return sc;
   }
   const int64_t slots = 2 * mst_waves(D, Kc, lgt) * 8;
-  // two workgroups per CU only if each still holds kMstGatesForTwo gates
-  if (sc.budget < 2 * tile + kMstGatesForTwo * (tile + slots)) sc.budget = sc.budget_full;
+  // two workgroups per CU only if the kernel's registers allow it and each still holds kMstGatesForTwo gates
+  if (!mst_two_groups(D, p->dtype) || sc.budget < 2 * tile + kMstGatesForTwo * (tile + slots))
+    sc.budget = sc.budget_full;
   sc.base = 2 * tile;
   sc.gate = [=](const OpPlan& op) { return (is_diag_kind(op.kind) ? phases : tile) + slots; };
   return sc;
@@ -1209,6 +1210,14 @@ extern "C" int sfamd_prog_create(const sfamd_op_t* ops, int nops, int n, int D, 
   place_table(p);
   p->state_elems.push_back(ipow(D, mixed ? 2 * n : n));
   int64_t nwg = (max_state + kBlock - 1) / kBlock;
+  // and a workgroup for every tile of a stage (6 modes, cutoff 4, one stage of 8 gates: 256 amplitudes
+  // for each of 16 workgroups against one tile for each of 64, adjoint launch and reduction 38 -> 14 us)
+  for (const Step& st : p->steps) {
+    bool one_pass;
+    p->nwg = 4096;
+    const int64_t groups = st.kind == kStepStage || st.kind == kStepMatrixStage ? step_columns(p, st, &one_pass) : 0;
+    if (groups > nwg) nwg = groups;
+  }
   if (nwg > 4096) nwg = 4096;
   if (nwg < 1) nwg = 1;
   p->nwg = (int)nwg;

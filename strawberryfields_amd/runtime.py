@@ -41,14 +41,14 @@ def default_fuse(n, D):
 
     Three, and more at the lowest cutoffs, where a tile of three modes leaves
     the matrix cores idle and a stage takes few gates: one layer of the layered
-    circuit, forward and adjoint, with 3 / 4 / 5 / 6 local modes took 814 / 787 /
-    487 / 398 us on 10 modes at cutoff 3, 284 / 216 / 253 us on 8 at cutoff 4, 400 /
-    270 / 554 us on 7 at cutoff 5 and 2041 / 1716 us on 8 at cutoff 6, but 133 / 216 us
-    on 5 modes at cutoff 7.  Cutoffs above 16 take two (three keep too few
-    gates' tiles in LDS for the adjoint)."""
+    circuit, forward and adjoint, with 3 / 4 / 5 / 6 local modes took 541 / 414 /
+    339 / 407 us on 10 modes at cutoff 3, 300 / 221 / 255 us on 8 at cutoff 4, 1024 /
+    727 / 787 us on 8 at cutoff 5, 395 / 337 us on 7 and 2074 / 1730 us on 8 at cutoff
+    6, but 132 / 161 us on 5 modes at cutoff 6.  Cutoffs above 16 take two (three
+    keep too few gates' tiles in LDS for the adjoint)."""
     if n < 2 or D < 2 or D > 20:
         return 0
-    want = 6 if D <= 3 else 4 if D <= 5 or (D == 6 and n >= 7) else 3 if D <= 16 else 2
+    want = 5 if D <= 3 else 4 if D <= 5 or (D == 6 and n >= 7) else 3 if D <= 16 else 2
     return min(want, n)
 
 
