@@ -575,13 +575,14 @@ __device__ void write_stage_image(int kind, int D, const cpx<T>* __restrict__ en
 // A gate's matrix-core images (mstage.h), one after the other: G, then (parts
 // = 3) G^H and dG/dp0^H.  Operator p (one for a single-mode gate; for a
 // beamsplitter the gate on the modular anti-diagonal {(k, (p - k) mod D)},
-// blockdiag(B_p, B_(p+D))), entry (mb, t) of half-lane h: row rp = h % 8 of
+// blockdiag(B_p, B_(p+D)); for S2 on the diagonal {(k, (k + p) mod D)}, the
+// blocks of the differences -p and D - p), entry (mb, t) of half-lane h: row rp = h % 8 of
 // column group h / 8, i.e. output amplitude (rp / 2) P + 2 mb + rp % 2 and input
 // amplitude (h / 8) P + t; zero outside the operator.
 template <typename T>
 __device__ void write_matrix_images(int kind, int D, const cpx<T>* __restrict__ entry, cpx<T>* __restrict__ dst,
                                     int parts) {
-  const bool two = kind == SFAMD_OP_BEAMSPLITTER;
+  const bool two = sfamd::mst_two_mode(kind), diff = kind == SFAMD_OP_TWO_MODE_SQUEEZE;
   const int P = sfamd::mst_p(D), NE = P * sfamd::mst_mb(D), n = (two ? D : 1) * NE;
   const int64_t deriv = two ? bs_nb(D) : (int64_t)D * D;
   const unsigned MN = ((1u << 20) + NE - 1) / NE, MP = ((1u << 20) + P - 1) / P;  // exact below 2^10
@@ -597,8 +598,8 @@ __device__ void write_matrix_images(int kind, int D, const cpx<T>* __restrict__ 
       const cpx<T>* m = entry + (which == 2 ? deriv : 0);
       if (!two) {
         v = m[a * D + b];
-      } else if ((a <= p) == (b <= p)) {
-        const int s = a <= p ? p : p + D;
+      } else if (diff ? (a < D - p) == (b < D - p) : (a <= p) == (b <= p)) {
+        const int s = diff ? (a < D - p ? D - 1 - p : 2 * D - 1 - p) : a <= p ? p : p + D;
         const int lo = bs_lo(s, D), c = bs_hi(s, D) - lo + 1;
         v = m[bs_block_off(s, D) + (a - lo) * c + (b - lo)];
       }
@@ -663,7 +664,7 @@ __global__ void __launch_bounds__(256) k_build(sfamd::BuildBatch b, int D, const
   if (d.img0 >= 0) write_stage_image<T>(kind, D, out, table + d.img0, false);
   if (d.img1 >= 0) write_stage_image<T>(kind, D, out, table + d.img1, true);
   if (!diag && (d.kind & sfamd::kBuildMatrixFwd)) {
-    const int64_t size = kind == SFAMD_OP_BEAMSPLITTER ? 2 * bs_nb(D) : 3 * (int64_t)D * D;
+    const int64_t size = sfamd::mst_two_mode(kind) ? 2 * bs_nb(D) : 3 * (int64_t)D * D;
     write_matrix_images<T>(kind, D, out, out + size, d.kind & sfamd::kBuildMatrixAdj ? 3 : 1);
   }
 }

@@ -38,9 +38,25 @@ __host__ __device__ constexpr int mst_tile(int D, int K) {
 __host__ __device__ constexpr int mst_p(int D) { return (D + 3) / 4; }
 __host__ __device__ constexpr int mst_mb(int D) { return (mst_p(D) + 1) / 2; }
 __host__ __device__ constexpr int mst_img(int D) { return mst_p(D) * mst_mb(D) * 32; }
+// two-mode gates of a stage: the photon-number sum or (S2) difference is conserved
+__host__ __device__ constexpr bool mst_two_mode(int kind) {
+  return kind == SFAMD_OP_BEAMSPLITTER || kind == SFAMD_OP_MZGATE || kind == SFAMD_OP_CROSS_KERR ||
+         kind == SFAMD_OP_TWO_MODE_SQUEEZE;
+}
 // operators of a gate: one for a single-mode gate, one per modular
-// anti-diagonal of the two modes for a beamsplitter
-__host__ __device__ constexpr int mst_nop(int kind, int D) { return kind == SFAMD_OP_BEAMSPLITTER ? D : 1; }
+// anti-diagonal (S2: diagonal) of the two modes for a two-mode gate
+__host__ __device__ constexpr int mst_nop(int kind, int D) { return mst_two_mode(kind) ? D : 1; }
+// Derivative by the second parameter (the first of a gate with one is read as
+// zero weights): dG/dp1 = (i / 2) (wa n + wb N) G with the first mode's digit n
+// before and N after the gate; both weights in bits 4 to 9 of MGate::two.
+constexpr int mst_weights(int kind) {
+  const int wa = kind == SFAMD_OP_BEAMSPLITTER || kind == SFAMD_OP_MZGATE ? 2
+                 : kind == SFAMD_OP_DISPLACEMENT || kind == SFAMD_OP_TWO_MODE_SQUEEZE ? -2
+                 : kind == SFAMD_OP_SQUEEZE ? -1
+                                            : 0;
+  const int wb = kind == SFAMD_OP_MZGATE ? 0 : -wa;
+  return (wa + 2) << 4 | (wb + 2) << 7;
+}
 // image entries of a gate: forward (G) and adjoint (G^H, then dG/dp0^H); rotation and Kerr gates use their
 // table entry
 __host__ __device__ constexpr int64_t mst_img_elems(int kind, int D, bool adj) {
@@ -81,14 +97,15 @@ __host__ __device__ constexpr bool mst_group_ok(int D, int K, int lgt) {
 // scalar loads drop the two low bits of their base.
 struct MGate {
   int32_t kind;
-  int32_t a0;         // local axis of the first mode (0 = slowest)
-  int32_t ds, wrap;   // LDS step from amplitude k to k + 1, and what is added where a beamsplitter's second digit wraps
+  int32_t a0;         // rotation / Kerr: local axis of the mode (0 = slowest); two modes: -1 if their photon-number
+                      // difference is conserved, 0 if the sum is
+  int32_t ds, wrap;   // LDS step from amplitude k to k + 1, and what is added where the second digit wraps
   int32_t l1;         // LDS stride of the second axis (0: one mode)
   int32_t cs[kMstMaxK - 1];  // LDS strides of the other local axes, slowest first
   int32_t op;         // program operation index (gradient slot)
   int32_t fwd, adj;   // table offsets of the images (rotation / Kerr: fwd = index of its phases in LDS)
   int32_t nfwd, padj; // the next gate's forward and the previous gate's adjoint image (gates with operators)
-  int32_t two;        // bit 0: this gate is a beamsplitter, bit 1: the next one, bit 2: the previous one
+  int32_t two;        // bit 0: this gate has two modes, bit 1: the next one, bit 2: the previous one; and mst_weights
 };
 
 // The fields every workgroup reads first come first.
@@ -99,7 +116,7 @@ struct MArgs {
   int32_t ntiles;  // D^nnl
   int32_t grid;    // workgroups of the launch (set by the launcher)
   int32_t nnl;     // modes outside the tile
-  int32_t h0_fwd, h0_two;  // the first gate with operators: its image, whether it is a beamsplitter
+  int32_t h0_fwd, h0_two;  // the first gate with operators: its image, whether it has two modes
   int32_t hl_adj, hl_two;  // the last one
   int32_t lgt;     // log2 of the tiles a workgroup holds at once
   int32_t phases;  // table offset of the rotation / Kerr phases, in gate order

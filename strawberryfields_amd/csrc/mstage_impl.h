@@ -2,7 +2,7 @@
 // ket, or over a density matrix on one side.
 //
 // A stage is a set of K "local" modes and an ordered list of gates that act
-// only on those modes (R, K, D, S on one local mode; BS on two).  The ket is
+// only on those modes (R, K, D, S, V on one local mode; BS, MZ, S2, CK on two).  The ket is
 // cut into tiles of the D^K amplitudes of the local modes for one assignment
 // of the other modes' digits.  A workgroup loads a tile into LDS, applies every
 // gate of the stage there and writes the tile back, so a stage costs one read
@@ -18,8 +18,10 @@
 // dense gate is one operator on the D^(K-1) fibers of its axis; a beamsplitter
 // is D operators, one per modular anti-diagonal {(k, (p - k) mod D)} of its
 // two axes (the photon-number blocks s = p and s = p + D side by side), on the
-// D^(K-2) positions of the other local axes.  A fiber belongs to one wave, so
-// gates work in place with one barrier per gate.
+// D^(K-2) positions of the other local axes; S2 has the diagonals
+// {(k, (k + p) mod D)} instead, with its difference blocks -p and D - p.  MZ and CK
+// are applied like beamsplitters.  A fiber belongs to one wave, so gates work in
+// place with one barrier per gate.
 //
 // The operators are not staged in LDS: the table build writes them in lane
 // order (complex entries, each shared by the two lanes holding its real and
@@ -31,9 +33,9 @@
 // cotangent tile, recomputes the stage forward keeping the input tile of every
 // gate with operators, and runs the gates backward: lam_in = G^H lam_out,
 // mu = dG/dp0^H lam_out, g0 = Re conj(mu) psi_in, and the phase parameter from
-// dG/dphi = i f (out - in) G (D: f = 1 on the mode's digit, S: f = 1/2;
-// BS: f = -1 on the first mode's digit):
-//   g1 = f sum_k k [Im conj(lam_in[k]) psi_in[k] - Im conj(lam_out[k]) psi_out[k]].
+// dG/dp1 = i (wa n + wb N) G with the (first) mode's digit n before and N after
+// the gate (D: -1, 1; S: -1/2, 1/2; BS: 1, -1; MZ: 1, 0; S2: -1, 1):
+//   g1 = -sum_k k [wa Im conj(lam_in[k]) psi_in[k] + wb Im conj(lam_out[k]) psi_out[k]].
 // Rotation and Kerr gates multiply in place and take no tile: the backward
 // sweep multiplies the state by the conjugate phases again.  Parameter sums are
 // reduced per wave by DPP lane moves and per workgroup in a fixed order
@@ -282,14 +284,15 @@ __device__ __forceinline__ void warm_gates(const sfamd::MArgs& a) {
 
 // The lane's place in item `item` (block * operators + operator) of a gate:
 // the LDS offset of its column's amplitude k = grp P + q is lo + q ds, plus
-// `wrap` where the second digit (p - k) mod D of a beamsplitter wraps around.
+// `wrap` where the second digit, (p - k) mod D or for S2 (k + p) mod D, wraps
+// around.
 // Slots past amplitude D - 1 (in the last lane groups) read amplitude D - 1 and
 // count as zero.  Everything but the gate's strides is the same for all gates,
 // so the compiler computes it once per kernel.
 template <typename Gm, bool TWO>
 struct Place {
   static constexpr int D = Gm::D, P = Gm::P;
-  int base, lo, ds, wrap, p;
+  int base, lo, ds, wrap, p, last;  // last: amplitude from whose successor on the second digit wraps
   bool valid;
   __device__ __forceinline__ Place(int item, const Gate& g) {
     const int lane = threadIdx.x & 63;
@@ -301,6 +304,7 @@ struct Place {
     if (!valid) f = NC - 1;
     ds = g.ds;
     wrap = g.wrap;
+    last = TWO ? (p ^ g.a0) + (g.a0 & D) : 0;  // p, or D - 1 - p where the difference is conserved
     base = p * g.l1;
 #pragma unroll
     for (int u = NCX - 1; u >= 0; --u) {
@@ -314,9 +318,9 @@ struct Place {
   __device__ __forceinline__ int grp() const { return (threadIdx.x & 63) >> 4; }
   __device__ __forceinline__ bool has(int q) const { return 3 * P + q < D || grp() * P + q < D; }
   __device__ __forceinline__ int at(int q) const {
-    if (3 * P + q < D) return lo + q * ds + (TWO && grp() * P + q > p ? wrap : 0);
+    if (3 * P + q < D) return lo + q * ds + (TWO && grp() * P + q > last ? wrap : 0);
     const int k = grp() * P + q < D ? grp() * P + q : D - 1;
-    return base + k * ds + (TWO && k > p ? wrap : 0);
+    return base + k * ds + (TWO && k > last ? wrap : 0);
   }
 };
 
@@ -477,7 +481,7 @@ __device__ __forceinline__ void heavy_adj(const Gate& g, const C<T>* __restrict_
   const int wave = wave_index();
   const C<T>* himg = table + g.adj;
   const C<T>* dimg = himg + (TWO ? Gm::D : 1) * Gm::IMG;
-  const T f = TWO ? (T)-1 : (g.kind == SFAMD_OP_SQUEEZE ? (T)0.5 : (T)1);
+  const T wi = (T)0.5 * (T)(2 - ((g.two >> 4) & 7)), wo = (T)0.5 * (T)(2 - ((g.two >> 7) & 7));
 #pragma unroll
   for (int j = 0; j < J; ++j) {
     const int item = wave + j * Gm::NW;
@@ -504,18 +508,19 @@ __device__ __forceinline__ void heavy_adj(const Gate& g, const C<T>* __restrict_
         else
           apply_image<T, Gm>(op.d, l, mu);
       }
-      T s1 = (T)0, s0 = (T)0;
+      T si = (T)0, so = (T)0, s0 = (T)0;
 #pragma unroll
       for (int q = 0; q < Gm::P; ++q) {
         // (amplitudes past D - 1 are zero in acc, x, l and po)
-        const T t = im_conj_mul(acc_amp<T>(acc, q), x[q]) - im_conj_mul(l[q], po[q]);
-        s1 += (T)(pl.grp() * Gm::P + q) * t;
+        const T k = (T)(pl.grp() * Gm::P + q);
+        si += k * im_conj_mul(acc_amp<T>(acc, q), x[q]);
+        so += k * im_conj_mul(l[q], po[q]);
         s0 += re_conj_mul(acc_amp<T>(mu, q), x[q]);
       }
       write_fiber<T, Gm, TWO>(lam, pl, acc);
       if (pl.valid) {
         g0 += s0;
-        g1 += f * s1;
+        g1 += wi * si + wo * so;
       }
     }
   }

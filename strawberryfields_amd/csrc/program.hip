@@ -330,11 +330,6 @@ struct sfamd_prog {
 
 namespace {
 
-bool fusable(const OpPlan& op) {
-  return op.kind == SFAMD_OP_ROTATION || op.kind == SFAMD_OP_KERR || op.kind == SFAMD_OP_DISPLACEMENT ||
-         op.kind == SFAMD_OP_SQUEEZE || op.kind == SFAMD_OP_BEAMSPLITTER;
-}
-
 // The stages of one representation: its axes (n of a ket, 2 n of a density
 // matrix: row and column of each mode in turn, slowest first), the kind of its
 // stages and their local axes (0: no stages).
@@ -343,6 +338,14 @@ struct Stages {
   int axes, kind, Kc;
   int modes(int n) const { return Kc < n ? Kc : n; }  // that a stage takes gates of
 };
+
+// the vector-ALU stages hold the gates of the layered circuit, the matrix-core stages every unitary gate
+bool fusable(const OpPlan& op, const Stages& sg) {
+  return op.kind == SFAMD_OP_ROTATION || op.kind == SFAMD_OP_KERR || op.kind == SFAMD_OP_DISPLACEMENT ||
+         op.kind == SFAMD_OP_SQUEEZE || op.kind == SFAMD_OP_BEAMSPLITTER ||
+         (sg.kind == kStepMatrixStage && (mst_two_mode(op.kind) || op.kind == SFAMD_OP_CUBIC_PHASE));
+}
+
 
 int op_nmodes(const OpPlan& op) { return two_mode_kind(op.kind) ? 2 : 1; }
 
@@ -564,7 +567,7 @@ void fill_matrix_stage(const sfamd_prog* p, Step& st, unsigned mask, const ModeO
   for (int gi = 0; gi < a.ngates; ++gi) {
     const OpPlan& op = p->ops[st.ops[gi]];
     MGate& g = a.g[gi];
-    const bool two = op.kind == SFAMD_OP_BEAMSPLITTER;
+    const bool two = mst_two_mode(op.kind), diff = op.kind == SFAMD_OP_TWO_MODE_SQUEEZE;
     int ax0 = 0, ax1 = -1;
     const int m0 = st.mixed ? 2 * op.m0 + side : op.m0, m1 = st.mixed ? 2 * op.m1 + side : op.m1;
     for (int t = 0; t < Kc; ++t) {
@@ -575,12 +578,12 @@ void fill_matrix_stage(const sfamd_prog* p, Step& st, unsigned mask, const ModeO
     for (int t = 0; t < Kc; ++t)
       if (t != ax0 && t != ax1) g.cs[u++] = mst_stride(D, Kc, t);
     g.kind = op.kind;
-    g.a0 = ax0;
+    g.a0 = !two ? ax0 : diff ? -1 : 0;
     g.l1 = two ? mst_stride(D, Kc, ax1) : 0;
-    g.ds = mst_stride(D, Kc, ax0) - g.l1;
-    g.wrap = D * g.l1;
+    g.ds = mst_stride(D, Kc, ax0) + (diff ? g.l1 : -g.l1);
+    g.wrap = (diff ? -D : D) * g.l1;
     g.op = st.ops[gi];
-    g.two = two;
+    g.two = (two ? 1 : 0) | mst_weights(op.kind);
     if (is_diag_kind(op.kind))
       ++a.ndiag;
     else
@@ -833,7 +836,8 @@ void plan_steps(const sfamd_prog* p, const Stages (&sg)[2], bool forward_only, s
     run.clear();
   };
   for (int i = 0; i < p->nops; ++i) {
-    if (sg[p->ops[i].mixed_in].Kc >= 2 && fusable(p->ops[i])) {
+    const Stages& g = sg[p->ops[i].mixed_in];
+    if (g.Kc >= 2 && fusable(p->ops[i], g)) {
       if (!run.empty() && p->ops[run.front()].mixed_in != p->ops[i].mixed_in) flush();
       run.push_back(i);
       continue;
@@ -929,7 +933,8 @@ void plan_program(sfamd_prog* p) {
   const Stages fwd[2] = {pick_stages(p, true, false), pick_stages(p, true, true)};
   bool matrix = false;
   for (const OpPlan& op : p->ops)
-    matrix = matrix || (fwd[op.mixed_in].Kc >= 3 && fwd[op.mixed_in].kind == kStepMatrixStage && fusable(op));
+    matrix = matrix || (fwd[op.mixed_in].Kc >= 3 && fwd[op.mixed_in].kind == kStepMatrixStage &&
+                        fusable(op, fwd[op.mixed_in]));
   if (matrix) plan_steps(p, fwd, true, &p->fsteps);
   // state sizes at step inputs
   p->state_elems.clear();

@@ -596,6 +596,41 @@ def test_density_matrix_stages_match_unfused(dtype, n, D, K, mixed):
         assert float((a - b).abs().max()) <= tol * float(a.abs().max())
 
 
+@pytest.mark.parametrize("dtype", [C128, C64])
+@pytest.mark.parametrize("n,D,K,mixed", [(3, 2, 3, False), (6, 4, 4, False), (3, 7, 3, False), (4, 8, 3, False),
+                                         (4, 9, 3, False), (3, 16, 3, False), (3, 20, 3, False), (2, 6, 2, True),
+                                         (3, 5, 3, True)])
+def test_matrix_core_stages_of_every_unitary_gate(dtype, n, D, K, mixed):
+    """S2 (difference blocks), MZ, CK and V next to the other gates in matrix-core
+    stages against the unfused kernels, both mode orders of every two-mode gate;
+    kets and density matrices.  Bound as for the stages of the layered circuit:
+    8 D m u (16 on a density matrix, where every gate acts twice) of the largest
+    entry for m gates of D-term contractions."""
+    ops = [("S2", (0, 1)), ("R", (0,)), ("MZ", (1, 0)), ("V", (0,)), ("CK", (n - 1, 0)), ("BS", (0, n - 1)), ("D", (1,)),
+           ("S2", (n - 1, 0)), ("K", (1,)), ("V", (n - 1,)), ("MZ", (0, n - 1)), ("CK", (0, 1)), ("S", (0,)), ("S2", (1, 0))]
+    g = torch.Generator().manual_seed(n * 100 + D)
+    shape = [D] * (2 * n if mixed else n)
+    st = torch.randn(shape, dtype=dtype, generator=g).to(DEV)
+    lam = torch.randn(shape, dtype=dtype, generator=g).to(DEV)
+    params = (torch.rand(len(ops), 2, dtype=torch.float64, generator=g) * 0.4).to(DEV)
+    for i, op in enumerate(ops):
+        if op[0] == "V":
+            params[i, 0] *= 0.05
+    res = []
+    for fuse in (0, K):
+        cc = runtime.CompiledCircuit(ops, n, D, mixed, dtype, DEV, fuse=fuse)
+        cc.build_table(params)
+        saved = [st] + [cc.new_state(i) for i in range(1, cc.nsteps)]
+        out = cc.forward(0, cc.nsteps, st, saved=saved)
+        gin = cc.new_state(0)
+        grads = torch.zeros(2 * len(ops), dtype=torch.float64, device=DEV)
+        cc.adjoint(0, cc.nsteps, saved, lam, gin, grads)
+        res.append((out, cc.run(st), gin, grads))
+    tol = (16 if mixed else 8) * D * len(ops) * (2.0**-24 if dtype == C64 else 2.0**-53)
+    for a, b in zip(*res):
+        assert float((a - b).abs().max()) <= tol * float(a.abs().max())
+
+
 @pytest.mark.parametrize("keep_always", [None, 0])
 @pytest.mark.parametrize("segment", [None, 1, 3])
 def test_kept_step_inputs_give_the_recomputed_gradients(segment, keep_always, monkeypatch):
