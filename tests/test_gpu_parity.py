@@ -631,6 +631,31 @@ def test_matrix_core_stages_of_every_unitary_gate(dtype, n, D, K, mixed):
         assert float((a - b).abs().max()) <= tol * float(a.abs().max())
 
 
+@pytest.mark.parametrize("dtype", [C128, C64])
+@pytest.mark.parametrize(
+    "n,D,modes",
+    # outputs fewer than a tile's 16 rows, exactly 16, between one and two tiles, tiles of 32 with a ragged edge
+    # and off the diagonal; traced ranges of one position, below, at and above the staged 32 and 64, and chunked;
+    # kept modes first, last (the other way of staging) and mixed
+    [(2, 3, [0]), (2, 3, [1]), (3, 4, [0, 2]), (5, 4, [1]), (2, 20, [1]), (3, 16, [0]), (4, 6, [0, 1]), (4, 6, [2, 3]),
+     (4, 7, [1, 3]), (6, 5, [0, 3, 4]), (5, 8, [0, 1]), (5, 8, [3, 4]), (2, 64, [0]), (2, 5, [0, 1]), (6, 8, [5])],
+)
+def test_reduced_dm_of_a_ket_vs_matrix_product(dtype, n, D, modes):
+    """M M^H with M the kept x traced matrix of a random ket, against the same
+    product in complex128 on the CPU.  Both sum NR products in 64 bits (rounding
+    at most 2 NR u of the largest entry, a diagonal one), then round once to the
+    state's precision."""
+    g = torch.Generator().manual_seed(D * 10 + n)
+    psi = torch.randn([D] * n, dtype=dtype, generator=g)
+    rest = [m for m in range(n) if m not in modes]
+    k = len(modes)
+    M = psi.to(C128).permute(modes + rest).reshape(D**k, -1)
+    ref = (M @ M.conj().T).reshape([D] * (2 * k)).permute([a for i in range(k) for a in (i, k + i)])
+    got = runtime.reduced_dm(psi.to(DEV), n, D, False, modes).cpu()
+    tol = 2 * M.shape[1] * 2.0**-53 + (2.0**-23 if dtype == C64 else 0.0)
+    assert float((got.to(C128) - ref).abs().max()) <= tol * float(ref.abs().max())
+
+
 @pytest.mark.parametrize("keep_always", [None, 0])
 @pytest.mark.parametrize("segment", [None, 1, 3])
 def test_kept_step_inputs_give_the_recomputed_gradients(segment, keep_always, monkeypatch):
