@@ -286,8 +286,10 @@ __device__ __forceinline__ void warm_gates(const sfamd::MArgs& a) {
 // the LDS offset of its column's amplitude k = grp P + q is lo + q ds, plus
 // `wrap` where the second digit, (p - k) mod D or for S2 (k + p) mod D, wraps
 // around.
-// Slots past amplitude D - 1 (in the last lane groups) read amplitude D - 1 and
-// count as zero.  Everything but the gate's strides is the same for all gates,
+// Slots past amplitude D - 1 (in the last lane groups) read amplitude D - 1,
+// which the operators' zero columns and a zero weight in the parameter sums
+// leave out (zeros selected after each read cost 2 vector instructions per
+// amplitude: 3 modes, cutoff 9, density matrix, complex128 1797 -> 1759 us).  Everything but the gate's strides is the same for all gates,
 // so the compiler computes it once per kernel.
 template <typename Gm, bool TWO>
 struct Place {
@@ -327,10 +329,7 @@ struct Place {
 template <typename T, typename Gm, bool TWO>
 __device__ __forceinline__ void read_fiber(const C<T>* tile, const Place<Gm, TWO>& pl, C<T> (&x)[Gm::P]) {
 #pragma unroll
-  for (int q = 0; q < Gm::P; ++q) {
-    const C<T> v = tile[pl.at(q)];
-    x[q] = pl.has(q) ? v : mk<T>(0, 0);
-  }
+  for (int q = 0; q < Gm::P; ++q) x[q] = tile[pl.at(q)];
 }
 
 template <typename T, typename Gm, bool TWO>
@@ -470,12 +469,12 @@ struct AdjOp {
   }
 };
 
-// One gate with operators backward: lam in place; xt = its input tile, pt = its
-// output tile; `op` holds the wave's first operators.  `between` runs while the LDS reads are
-// in flight.
+// One gate with operators backward: lam in place; xt = its input tile, followed
+// by its output tile; `op` holds the wave's first operators.  `between` runs
+// while the LDS reads are in flight.
 template <typename T, typename Gm, bool TWO, typename F>
 __device__ __forceinline__ void heavy_adj(const Gate& g, const C<T>* __restrict__ table, const C<T>* xt,
-                                          const C<T>* pt, C<T>* lam, const AdjOp<T, Gm>& op, T& g0, T& g1, F between) {
+                                          C<T>* lam, const AdjOp<T, Gm>& op, T& g0, T& g1, F between) {
   constexpr int N = Gm::items(TWO), J = Gm::per_wave(TWO);
   constexpr bool kReload = TWO && J > 1 && Gm::NW % Gm::D != 0;
   const int wave = wave_index();
@@ -494,7 +493,7 @@ __device__ __forceinline__ void heavy_adj(const Gate& g, const C<T>* __restrict_
       typename Mx<T>::acc4 acc[Gm::MB], mu[Gm::MB];
       read_fiber<T, Gm, TWO>(lam, pl, l);
       read_fiber<T, Gm, TWO>(xt, pl, x);
-      read_fiber<T, Gm, TWO>(pt, pl, po);
+      read_fiber<T, Gm, TWO>(xt + Gm::GS, pl, po);
       if (j == 0) between();
       if (kReload && j > 0) {
         C<T> other[Gm::NE];
@@ -511,8 +510,8 @@ __device__ __forceinline__ void heavy_adj(const Gate& g, const C<T>* __restrict_
       T si = (T)0, so = (T)0, s0 = (T)0;
 #pragma unroll
       for (int q = 0; q < Gm::P; ++q) {
-        // (amplitudes past D - 1 are zero in acc, x, l and po)
-        const T k = (T)(pl.grp() * Gm::P + q);
+        // (slots past D - 1: acc and mu are zero, l and po are not)
+        const T k = pl.has(q) ? (T)(pl.grp() * Gm::P + q) : (T)0;
         si += k * im_conj_mul(acc_amp<T>(acc, q), x[q]);
         so += k * im_conj_mul(l[q], po[q]);
         s0 += re_conj_mul(acc_amp<T>(mu, q), x[q]);
@@ -569,9 +568,9 @@ __device__ __forceinline__ void gate_adj(const Gate& g, int gi, const C<T>* __re
     auto flush = [&]() { sum.template flush<Gm>(gsl, first); };
     if (wave_index() >= N) flush();
     if (two)
-      heavy_adj<T, Gm, true>(g, table, at - Gm::GS, at, lam, op, g0, g1, flush);
+      heavy_adj<T, Gm, true>(g, table, at - Gm::GS, lam, op, g0, g1, flush);
     else
-      heavy_adj<T, Gm, false>(g, table, at - Gm::GS, at, lam, op, g0, g1, flush);
+      heavy_adj<T, Gm, false>(g, table, at - Gm::GS, lam, op, g0, g1, flush);
     at -= Gm::GS;
   }
   sum.g0 = g0;
