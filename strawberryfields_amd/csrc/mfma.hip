@@ -58,6 +58,10 @@ __device__ __forceinline__ C acc_amp(const f4 (&acc)[Plan<D>::Mb], int q) {
 // fiber f of an axis with stride R (R = 1: innermost) -> offset of amplitude 0
 __device__ __forceinline__ int64_t fiber_base(int64_t f, int64_t R, int D) {
   if (R == 1) return f * D;
+  if (((uint64_t)(f | R) >> 32) == 0) {  // a 32-bit division is a quarter of the instructions
+    const unsigned o = (unsigned)f / (unsigned)R;
+    return (int64_t)o * D * R + ((unsigned)f - o * (unsigned)R);
+  }
   const int64_t o = f / R;
   return o * D * R + (f - o * R);
 }
@@ -230,6 +234,12 @@ k_axis_mfma_adj(const C* __restrict__ psi, const C* __restrict__ lo, C* __restri
 // block's real operator once per task (Mb = ceil(2c / 16) in 1..3) and applies
 // it to 16 fibers per MFMA chain.  Fibers of a chunk are consecutive inner
 // positions of the non-gate axes (coalesced when that run is >= 16).
+// Memory bounds it (adjoint: three states), with about half as much matrix-core
+// time to hide: a wave issues the loads of its next 16 fibers before the
+// products of these, and fiber bases take 32-bit divisions.  One beamsplitter
+// with these, before -> after, against the time of its bytes at a copy's rate:
+// 6 modes, cutoff 16 (134 MB) adjoint 131 -> 106 us (83), forward 67 -> 62 (56);
+// 3-mode density matrix, cutoff 20 (512 MB) 460 -> 406 (318), 279 -> 260 (212).
 constexpr int kBsChunk = 1024;  // 512 or 2048: c5 5.59 -> 5.52 grad-evals/s
 
 struct PairGeo {
@@ -238,6 +248,12 @@ struct PairGeo {
 };
 
 __device__ __forceinline__ int64_t pair_base(int64_t f, const PairGeo& g, int D) {
+  if (((uint64_t)(f | g.B | g.C) >> 32) == 0) {  // a 32-bit division is a quarter of the instructions
+    const unsigned B = (unsigned)g.B, Cn = (unsigned)g.C;
+    const unsigned t = (unsigned)f / B, b = (unsigned)f - t * B;
+    const unsigned a = t / Cn, c = t - a * Cn;
+    return a * (D * g.s_lo) + c * (D * g.s_hi) + b;
+  }
   const int64_t b = f % g.B;
   const int64_t t = f / g.B;
   const int64_t c = t % g.C;
@@ -292,17 +308,26 @@ __device__ __forceinline__ void bs_task(const C* __restrict__ in, C* __restrict_
   const int64_t first = block_first(sp, sq, lo, s, D, diff);
   const int64_t left = NF - f0;
   const int nf = left < kBsChunk ? (int)left : kBsChunk;
-  for (int b16 = threadIdx.x >> 6; b16 * 16 < nf; b16 += blockDim.x >> 6) {
+  // the next 16 fibers' loads are in flight over the product of these
+  const int nw = blockDim.x >> 6;
+  C xn[P];
+  int64_t fbn = 0;
+  auto fetch = [&](int b16) {
+    const int64_t f = f0 + (b16 * 16 + cl < nf ? b16 * 16 + cl : 0);
+    fbn = pair_base(f, geo, D) + first;
+#pragma unroll
+    for (int q = 0; q < P; ++q) xn[q] = in[fbn + (int64_t)clamp_amp(g * P + q, c) * step];
+  };
+  int b16 = threadIdx.x >> 6;
+  if (b16 * 16 < nf) fetch(b16);
+  for (; b16 * 16 < nf; b16 += nw) {
     const bool valid = b16 * 16 + cl < nf;
-    const int64_t f = f0 + (valid ? b16 * 16 + cl : 0);
-    const int64_t fb = pair_base(f, geo, D) + first;
+    const int64_t fb = fbn;
     C x[Q];
 #pragma unroll
-    for (int q = 0; q < Q; ++q) {
-      const int a = g * P + q;
-      const C v = in[fb + (int64_t)clamp_amp(a, c) * step];
-      x[q] = (valid && q < P && a < c) ? v : mk<float>(0.f, 0.f);
-    }
+    for (int q = 0; q < Q; ++q)
+      x[q] = (valid && q < P && g * P + q < c) ? xn[q < P ? q : 0] : mk<float>(0.f, 0.f);
+    if ((b16 + nw) * 16 < nf) fetch(b16 + nw);
     f4 acc[MB];
     apply_op<MB>(A, x, acc, P);
     if (valid) {
@@ -372,21 +397,34 @@ __device__ __forceinline__ void bs_adj_task(const C* __restrict__ psi, const C* 
   const int64_t first = block_first(sp, sq, lo, s, D, diff);
   const int64_t left = NF - f0;
   const int nf = left < kBsChunk ? (int)left : kBsChunk;
-  for (int b16 = threadIdx.x >> 6; b16 * 16 < nf; b16 += blockDim.x >> 6) {
-    __asm__ volatile("" ::: "memory");  // operators stay in LDS (see k_axis_mfma_adj)
+  // the next 16 fibers' loads are in flight over the products of these
+  const int nw = blockDim.x >> 6;
+  C xn[P], ln[P];
+  int64_t fbn = 0;
+  auto fetch = [&](int b16) {
+    const int64_t f = f0 + (b16 * 16 + cl < nf ? b16 * 16 + cl : 0);
+    fbn = pair_base(f, geo, D) + first;
+#pragma unroll
+    for (int q = 0; q < P; ++q) {
+      const int64_t o = fbn + (int64_t)clamp_amp(g * P + q, c) * step;
+      xn[q] = psi[o];
+      ln[q] = lo_[o];
+    }
+  };
+  int b16 = threadIdx.x >> 6;
+  if (b16 * 16 < nf) fetch(b16);
+  for (; b16 * 16 < nf; b16 += nw) {
     const bool valid = b16 * 16 + cl < nf;
-    const int64_t f = f0 + (valid ? b16 * 16 + cl : 0);
-    const int64_t fb = pair_base(f, geo, D) + first;
+    const int64_t fb = fbn;
     C x[Q], l[Q];
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
-      const int a = g * P + q;
-      const bool in_range = valid && q < P && a < c;
-      const int64_t o = fb + (int64_t)clamp_amp(a, c) * step;
-      const C xv = psi[o], lv = lo_[o];
-      x[q] = in_range ? xv : mk<float>(0.f, 0.f);
-      l[q] = in_range ? lv : mk<float>(0.f, 0.f);
+      const bool in_range = valid && q < P && g * P + q < c;
+      x[q] = in_range ? xn[q < P ? q : 0] : mk<float>(0.f, 0.f);
+      l[q] = in_range ? ln[q < P ? q : 0] : mk<float>(0.f, 0.f);
     }
+    if ((b16 + nw) * 16 < nf) fetch(b16 + nw);
+    __asm__ volatile("" ::: "memory");  // operators stay in LDS (see k_axis_mfma_adj)
     f4 acc[MB];
     apply_op_lds<MB>(opl, l, acc, P);
     if (valid) {
@@ -407,7 +445,7 @@ __device__ __forceinline__ void bs_adj_task(const C* __restrict__ psi, const C* 
 }
 
 template <int D>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, D <= 16 ? 4 : 3)
 k_bs_mfma_adj(const C* __restrict__ psi, const C* __restrict__ lo_, C* __restrict__ li, int64_t NF, PairGeo geo,
               int64_t sp, int64_t sq, const C* __restrict__ blk, const C* __restrict__ dblk, int conj, int wa,
               int wb, int diff, double* __restrict__ partial, int nwg, int zp1) {
