@@ -75,21 +75,33 @@ __device__ __forceinline__ int64_t fiber_base(int64_t f, int64_t R, int D) {
 // results go back the same way.  LDS accesses of one wave complete in order,
 // so the buffer needs no barrier, only the compiler's ordering.
 template <int D>
-__device__ __forceinline__ void chain_in(const C* __restrict__ src, C* buf) {
-  constexpr int NV = 8 * D, IT = (NV + 63) / 64;  // 16-byte vectors of 16 D amplitudes
-  const int lane = threadIdx.x & 63;
+struct Chain {
+  static constexpr int NV = 8 * D, IT = (NV + 63) / 64;  // 16-byte vectors of 16 D amplitudes
   f4 v[IT];
+  __device__ __forceinline__ void load(const C* __restrict__ src) {
+    const int lane = threadIdx.x & 63;
 #pragma unroll
-  for (int i = 0; i < IT; ++i) {
-    const int j = lane + 64 * i;
-    v[i] = reinterpret_cast<const f4*>(src)[j < NV ? j : NV - 1];
+    for (int i = 0; i < IT; ++i) {
+      const int j = lane + 64 * i;
+      v[i] = reinterpret_cast<const f4*>(src)[j < NV ? j : NV - 1];
+    }
   }
+  __device__ __forceinline__ void put(C* buf) const {
+    const int lane = threadIdx.x & 63;
 #pragma unroll
-  for (int i = 0; i < IT; ++i) {
-    const int j = lane + 64 * i;
-    if (j < NV) reinterpret_cast<f4*>(buf)[j] = v[i];
+    for (int i = 0; i < IT; ++i) {
+      const int j = lane + 64 * i;
+      if (j < NV) reinterpret_cast<f4*>(buf)[j] = v[i];
+    }
+    __asm__ volatile("" ::: "memory");
   }
-  __asm__ volatile("" ::: "memory");
+};
+
+template <int D>
+__device__ __forceinline__ void chain_in(const C* __restrict__ src, C* buf) {
+  Chain<D> ch;
+  ch.load(src);
+  ch.put(buf);
 }
 
 template <int D>
@@ -166,31 +178,54 @@ k_axis_mfma_adj(const C* __restrict__ psi, const C* __restrict__ lo, C* __restri
   const int64_t nblk = (NF + 15) / 16;
   const int64_t nwave = (int64_t)gridDim.x * (blockDim.x >> 6);
   double g0 = 0.0, g1 = 0.0;
-  for (int64_t blk = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); blk < nblk; blk += nwave) {
-    // keep the operators in LDS: without this barrier the compiler hoists
-    // their loop-invariant reads into (three operators' worth of) registers
-    __asm__ volatile("" ::: "memory");
-    const int64_t f = blk * 16 + c;
-    const bool valid = f < NF;
-    const int64_t fb = fiber_base(valid ? f : 0, R, D);
+  // The next 16 fibers' loads are in flight over the products of these: three
+  // products at cutoff 20 take as long as three quarters of the memory time
+  // (512 MB density matrix 423 -> 386 us, innermost axis 495 -> 390; its bytes at a
+  // copy's rate 318).
+  Chain<D> xc, lc;
+  C xn[P], ln[P];
+  int64_t fbn = 0;
+  auto fetch = [&](int64_t blk) {
+    if constexpr (INNER) {
+      xc.load(psi + blk * CH);
+      lc.load(lo + blk * CH);
+    } else {
+      const int64_t f = blk * 16 + c;
+      fbn = fiber_base(f < NF ? f : 0, R, D);
+#pragma unroll
+      for (int q = 0; q < P; ++q) {
+        const int64_t o = fbn + (int64_t)clamp_amp(g * P + q, D) * R;
+        xn[q] = psi[o];
+        ln[q] = lo[o];
+      }
+    }
+  };
+  int64_t blk = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  if (blk < nblk) fetch(blk);
+  for (; blk < nblk; blk += nwave) {
+    const bool valid = blk * 16 + c < NF;
+    const int64_t fb = fbn;
     C x[Q], l[Q];
     if constexpr (INNER) {
-      chain_in<D>(psi + blk * CH, bx);
-      chain_in<D>(lo + blk * CH, bl);
+      xc.put(bx);
+      lc.put(bl);
     }
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
       x[q] = l[q] = mk<float>(0.f, 0.f);
       if (q >= P) continue;
       const int a = g * P + q;
-      const int64_t o = fb + (int64_t)clamp_amp(a, D) * R;
-      const C xv = INNER ? bx[c * D + clamp_amp(a, D)] : psi[o];
-      const C lv = INNER ? bl[c * D + clamp_amp(a, D)] : lo[o];
+      const C xv = INNER ? bx[c * D + clamp_amp(a, D)] : xn[q];
+      const C lv = INNER ? bl[c * D + clamp_amp(a, D)] : ln[q];
       if (valid && a < D) {
         x[q] = xv;
         l[q] = lv;
       }
     }
+    if (blk + nwave < nblk) fetch(blk + nwave);
+    // keep the operators in LDS: without this barrier the compiler hoists
+    // their loop-invariant reads into (three operators' worth of) registers
+    __asm__ volatile("" ::: "memory");
     f4 acc[MB];
     apply_op_lds<MB>(opl, l, acc, P);
     if constexpr (INNER) {
