@@ -8,6 +8,11 @@ namespace sfamd {
 
 constexpr int kStageMaxGates = 40;   // gates per stage (kernel-argument space)
 constexpr int kStageMaxD = 20;       // cutoffs with compiled stage kernels: 2..20
+// Cutoffs with stages of three modes: just past a matrix-core operand of 8, where
+// one is a quarter full (which stages a plan takes: program.hip).
+__host__ __device__ constexpr bool stage_three_modes(int D, int dtype) {
+  return D == 9 || (D == 10 && dtype == SFAMD_C64);
+}
 constexpr int kStageMaxModes = 24;   // modes outside the tile
 // dynamic LDS a stage may use: gfx950 has 160 KB of LDS per compute unit
 constexpr int64_t kStageLdsPerCu = 160 * 1024;
@@ -52,7 +57,7 @@ __host__ __device__ constexpr int stage_threads(int D, int K) {
   return stage_tile(D, K) >= 1024 ? 1024 : (stage_tile(D, K) <= 256 ? 256 : ((stage_tile(D, K) + 63) / 64) * 64);
 }
 
-bool stage_supported(int D, int K);
+bool stage_supported(int D, int K, int dtype);
 // Beamsplitters at cutoffs up to kFullBsMaxD are staged in the zero-padded
 // per-fiber layout (D^3 entries per matrix), larger ones in the compact block
 // layout of the gate table.

@@ -5,8 +5,8 @@
 
 namespace sfamd {
 
-bool stage_supported(int D, int K) {
-  return D >= 2 && D <= kStageMaxD && K == 2;
+bool stage_supported(int D, int K, int dtype) {
+  return D >= 2 && D <= kStageMaxD && (K == 2 || (K == 3 && stage_three_modes(D, dtype)));
 }
 
 int64_t stage_gate_elems(int kind, int D, bool derivs) {

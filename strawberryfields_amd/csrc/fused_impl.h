@@ -1,6 +1,7 @@
-// Fused gate stages on two modes of a pure state (ket): many gates per pass,
-// in LDS.  Tiles of D^2 amplitudes are too small to fill matrix-core columns;
-// stages of three and more modes are in mstage_impl.h.
+// Fused gate stages on two modes of a pure state (ket), at cutoffs 9 and
+// 10 also on three: many gates per pass, in LDS.  Tiles of D^2 amplitudes are too small to
+// fill matrix-core columns; the other stages of three and more modes are in
+// mstage_impl.h.
 //
 // A stage is a set of K "local" modes and an ordered list of gates that act
 // only on those modes (R, K, D, S on one local mode; BS on two).  The ket is
@@ -546,6 +547,8 @@ int launch_adj(const void* psi, const void* lo, void* li, const void* table, con
 template <typename T, int D>
 int fwd_k(int K, const void* in, void* out, const void* table, const sfamd::StageArgs& a, int grid, hipStream_t s) {
   if (K == 2) return launch_fwd<T, D, 2>(in, out, table, a, grid, s);
+  if constexpr (sfamd::stage_three_modes(D, sizeof(T) == 4 ? SFAMD_C64 : SFAMD_C128))
+    if (K == 3) return launch_fwd<T, D, 3>(in, out, table, a, grid, s);
   return SFAMD_E_ARG;
 }
 
@@ -553,13 +556,15 @@ template <typename T, int D>
 int adj_k(int K, const void* psi, const void* lo, void* li, const void* table, const sfamd::StageArgs& a, int grid,
           double* partial, int nwg, hipStream_t s) {
   if (K == 2) return launch_adj<T, D, 2>(psi, lo, li, table, a, grid, partial, nwg, s);
+  if constexpr (sfamd::stage_three_modes(D, sizeof(T) == 4 ? SFAMD_C64 : SFAMD_C128))
+    if (K == 3) return launch_adj<T, D, 3>(psi, lo, li, table, a, grid, partial, nwg, s);
   return SFAMD_E_ARG;
 }
 
 }  // namespace
 
 // Defines sfamd::stage_fwd_d<d> / stage_adj_d<d>, the launchers of cutoff d
-// (both dtypes, two local modes); each fused_dNN_MM.hip
+// (both dtypes); each fused_dNN_MM.hip
 // translation unit instantiates a range of cutoffs so the kernels compile in
 // parallel.
 #define SFAMD_STAGE_DEFINE_D(d)                                                                                   \

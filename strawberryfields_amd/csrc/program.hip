@@ -467,7 +467,7 @@ StageCost stage_cost(const sfamd_prog* p, const Stages& sg, bool forward_only) {
 // Can a stage of this kind hold one gate of any kind?
 bool stage_fits(const sfamd_prog* p, const Stages& sg, bool forward_only) {
   if (sg.Kc < 2 || sg.Kc > sg.axes) return false;
-  if (sg.kind == kStepStage ? (sg.mixed || sg.axes > kStageMaxModes || !stage_supported(p->D, sg.Kc))
+  if (sg.kind == kStepStage ? (sg.mixed || sg.axes > kStageMaxModes || !stage_supported(p->D, sg.Kc, p->dtype))
                             : (sg.axes > kMstMaxModes || !mst_supported(p->D, sg.Kc)))
     return false;
   int64_t tiles = 1;
@@ -647,10 +647,10 @@ void link_matrix_stage(const sfamd_prog* p, MArgs& a, int spare) {
 // fastest ones reads and writes single amplitudes, one cache line each (6
 // modes, cutoff 16, complex64, 134 MB: two beamsplitters on modes 0 to 2 292 us,
 // one on the last modes 58 us, a device copy 38 us).  The states between the
-// stages are the library's own, so each stage writes its output with the next stage's local modes
-// fastest: reads are whole tiles, and writes are runs of the mode that the two
-// stages share, placed fastest of all.  Unused local modes are chosen to share
-// one with the stage before.
+// stages are the library's own, so each stage writes its output with the next
+// stage's local modes fastest: reads are whole tiles, and writes are runs of the
+// mode that the two stages share, placed fastest of all.  Unused local modes are
+// chosen to share one with the stage before.
 void order_stages(const sfamd_prog* p, std::vector<Step>* steps, size_t first, std::vector<unsigned> masks) {
   const int n = p->n, D = p->D;
   const size_t count = masks.size();
@@ -904,11 +904,25 @@ bool dm_stages_pay(const sfamd_prog* p, bool forward_only) {
   return p->D <= 16 && p->n == 2;
 }
 
+constexpr int kFewTilesModes = 4;  // modes up to which there are at most D tiles of three
+
 // The stages of a plan for a requested number of local modes: matrix-core
 // stages for three and more, vector-ALU stages for two (a beamsplitter on two
 // local modes has one column, so a matrix-core operand would be 15/16 empty) and
 // where the matrix-core adjoint's tiles exceed the LDS.  On a density matrix a
 // stage of fewer modes has the other side's axes for columns.
+//
+// Circuits of R, K, D, S and BS also have vector-ALU stages, which the adjoint
+// takes where operands padded to 16 waste the matrix cores: at cutoff 9 (and 10 in
+// complex64 on 5 modes; 6 modes have too many tiles for its LDS, 64 short stages
+// take 4346 us, against 951 for one layer on the matrix cores) with three modes;
+// and with two where there are at most D tiles of three modes, so that most
+// compute units idle and two modes' stages have D times the workgroups.  Three layers, one gradient from a graph,
+// us, matrix-core / vector-ALU stages: complex64, 3 modes 8 165 / 231, 9 299 / 235, 10
+// 308 / 230, 12 363 / 306, 14 527 / 299; 4 modes 8 306 / 453, 9 551 / 388, 12 603 / 591,
+// 14 945 / 686; 5 modes 9 849 / 606, 10 833 / 740, 12 958 / 1259; 6 modes 9 2656 / 2030;
+// complex128, 3 modes 8 197 / 234, 9 357 / 293, 12 498 / 341; 4 modes 9 623 / 497, 12
+// 883 / 756, 14 1827 / 850; 5 modes 9 984 / 870, 10 989 / 1083.
 Stages pick_stages(const sfamd_prog* p, bool forward_only, bool mixed) {
   const int K = p->fuse_K < p->n ? p->fuse_K : p->n;
   Stages sg{mixed, mixed ? 2 * p->n : p->n, kStepMatrixStage, K};
@@ -916,6 +930,15 @@ Stages pick_stages(const sfamd_prog* p, bool forward_only, bool mixed) {
     sg.Kc = p->fuse_K < 3 ? 3 : p->fuse_K < sg.axes ? p->fuse_K : sg.axes;
     if (!p->fuse_mixed || p->fuse_K < 2 || p->n < 2 || !stage_fits(p, sg, forward_only) || !dm_stages_pay(p, forward_only)) sg.Kc = 0;
     return sg;
+  }
+  bool layered = K == 3 && !forward_only && p->D > 8 && stages_pay(p, kStepMatrixStage, false);
+  for (const OpPlan& op : p->ops)
+    layered = layered && (op.mixed_in || op.kind == SFAMD_OP_LOSS || op.kind == SFAMD_OP_MIX ||
+                          fusable(op, Stages{false, p->n, kStepStage, 2}));
+  if (layered) {
+    const bool three = stage_three_modes(p->D, p->dtype) && (p->D == 9 || p->n == kFewTilesModes + 1);
+    const Stages valu{false, p->n, kStepStage, three ? 3 : 2};
+    if ((three || p->n <= kFewTilesModes) && stage_fits(p, valu, false)) return valu;
   }
   if (K >= 3 && stage_fits(p, sg, forward_only)) {
     if (!stages_pay(p, kStepMatrixStage, forward_only)) sg.Kc = 0;
