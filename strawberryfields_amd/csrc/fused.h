@@ -9,9 +9,10 @@ namespace sfamd {
 constexpr int kStageMaxGates = 40;   // gates per stage (kernel-argument space)
 constexpr int kStageMaxD = 20;       // cutoffs with compiled stage kernels: 2..20
 // Cutoffs with stages of three modes: just past a matrix-core operand of 8, where
-// one is a quarter full (which stages a plan takes: program.hip).
+// one is a quarter full, and large complex128 states at 5 and 6 (which stages a
+// plan takes: program.hip).
 __host__ __device__ constexpr bool stage_three_modes(int D, int dtype) {
-  return D == 9 || (D == 10 && dtype == SFAMD_C64);
+  return D == 9 || (D == 10 && dtype == SFAMD_C64) || ((D == 5 || D == 6) && dtype == SFAMD_C128);
 }
 constexpr int kStageMaxModes = 24;   // modes outside the tile
 // dynamic LDS a stage may use: gfx950 has 160 KB of LDS per compute unit

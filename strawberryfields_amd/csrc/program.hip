@@ -917,7 +917,10 @@ constexpr int kFewTilesModes = 4;  // modes up to which there are at most D tile
 // complex64 on 5 modes; 6 modes have too many tiles for its LDS, 64 short stages
 // take 4346 us, against 951 for one layer on the matrix cores) with three modes;
 // and with two where there are at most D tiles of three modes, so that most
-// compute units idle and two modes' stages have D times the workgroups.  Three layers, one gradient from a graph,
+// compute units idle and two modes' stages have D times the workgroups.  It also
+// takes them, with three modes, on complex128 states past the caches at cutoffs 5 and 6 (one
+// layer, matrix cores or unfused / vector ALUs: 8 modes 6, 27 MB, 3217 / 2922; 9
+// modes 5, 31 MB, 4453 / 4282; within the caches 8 modes 5, 6 MB, 1100 / 1202).  Three layers, one gradient from a graph,
 // us, matrix-core / vector-ALU stages: complex64, 3 modes 8 165 / 231, 9 299 / 235, 10
 // 308 / 230, 12 363 / 306, 14 527 / 299; 4 modes 8 306 / 453, 9 551 / 388, 12 603 / 591,
 // 14 945 / 686; 5 modes 9 849 / 606, 10 833 / 740, 12 958 / 1259; 6 modes 9 2656 / 2030;
@@ -931,12 +934,13 @@ Stages pick_stages(const sfamd_prog* p, bool forward_only, bool mixed) {
     if (!p->fuse_mixed || p->fuse_K < 2 || p->n < 2 || !stage_fits(p, sg, forward_only) || !dm_stages_pay(p, forward_only)) sg.Kc = 0;
     return sg;
   }
-  bool layered = K == 3 && !forward_only && p->D > 8 && stages_pay(p, kStepMatrixStage, false);
+  const bool large = K >= 3 && p->dtype == SFAMD_C128 && (p->D == 5 || p->D == 6) && ipow(p->D, p->n) >= 1250000;
+  bool layered = !forward_only && (large || (K == 3 && p->D > 8 && stages_pay(p, kStepMatrixStage, false)));
   for (const OpPlan& op : p->ops)
     layered = layered && (op.mixed_in || op.kind == SFAMD_OP_LOSS || op.kind == SFAMD_OP_MIX ||
                           fusable(op, Stages{false, p->n, kStepStage, 2}));
   if (layered) {
-    const bool three = stage_three_modes(p->D, p->dtype) && (p->D == 9 || p->n == kFewTilesModes + 1);
+    const bool three = stage_three_modes(p->D, p->dtype) && (large || p->D == 9 || p->n == kFewTilesModes + 1);
     const Stages valu{false, p->n, kStepStage, three ? 3 : 2};
     if ((three || p->n <= kFewTilesModes) && stage_fits(p, valu, false)) return valu;
   }

@@ -526,7 +526,7 @@ def test_fused_single_gate_adjoint_matches_unfused_at_large_cutoffs(D):
     # one and several tiles; 1, 2 and 3 blocks of 16 rows and a last lane group with 0..3 amplitudes missing;
     # column counts below, at and above 16; tile groups (low cutoffs); threads without elements (D = 10, 11)
     [(3, 2, 3), (7, 3, 6), (6, 4, 4), (5, 5, 4), (7, 5, 3), (5, 8, 3), (4, 9, 3), (4, 10, 3), (3, 11, 3), (4, 13, 3),
-     (4, 16, 3), (3, 17, 3), (3, 20, 3), (5, 9, 3), (5, 10, 3), (5, 13, 3)],
+     (4, 16, 3), (3, 17, 3), (3, 20, 3), (5, 9, 3), (5, 10, 3), (5, 13, 3), (8, 6, 4)],
 )
 def test_matrix_core_stages_match_unfused(dtype, n, D, K):
     """Stages of K >= 3 local modes on random states: the forward sweep with
