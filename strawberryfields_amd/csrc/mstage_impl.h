@@ -37,9 +37,11 @@
 // the gate (D: -1, 1; S: -1/2, 1/2; BS: 1, -1; MZ: 1, 0; S2: -1, 1):
 //   g1 = -sum_k k [wa Im conj(lam_in[k]) psi_in[k] + wb Im conj(lam_out[k]) psi_out[k]].
 // Rotation and Kerr gates multiply in place and take no tile: the backward
-// sweep multiplies the state by the conjugate phases again.  Parameter sums are
-// reduced per wave by DPP lane moves and per workgroup in a fixed order
-// (deterministic), one partial per workgroup.
+// sweep multiplies the state by the conjugate phases again.  Products are
+// formed in the state's precision (a rotation's or Kerr gate's in double), the
+// difference in g1 per amplitude, and everything past a lane's few amplitudes
+// of one fiber is summed in double: per lane, per wave by lane moves and per
+// workgroup in a fixed order (deterministic), one partial per workgroup.
 //
 // A density matrix is a ket of 2 n axes: a launch on row axes applies the gates,
 // one on column axes (`side`) their conjugates, as G on the conjugated tile,
@@ -474,7 +476,7 @@ struct AdjOp {
 // while the LDS reads are in flight.
 template <typename T, typename Gm, bool TWO, typename F>
 __device__ __forceinline__ void heavy_adj(const Gate& g, const C<T>* __restrict__ table, const C<T>* xt,
-                                          C<T>* lam, const AdjOp<T, Gm>& op, T& g0, T& g1, F between) {
+                                          C<T>* lam, const AdjOp<T, Gm>& op, double& g0, double& g1, F between) {
   constexpr int N = Gm::items(TWO), J = Gm::per_wave(TWO);
   constexpr bool kReload = TWO && J > 1 && Gm::NW % Gm::D != 0;
   const int wave = wave_index();
@@ -507,19 +509,18 @@ __device__ __forceinline__ void heavy_adj(const Gate& g, const C<T>* __restrict_
         else
           apply_image<T, Gm>(op.d, l, mu);
       }
-      T si = (T)0, so = (T)0, s0 = (T)0;
+      T s0 = (T)0, s1 = (T)0;
 #pragma unroll
       for (int q = 0; q < Gm::P; ++q) {
         // (slots past D - 1: acc and mu are zero, l and po are not)
         const T k = pl.has(q) ? (T)(pl.grp() * Gm::P + q) : (T)0;
-        si += k * im_conj_mul(acc_amp<T>(acc, q), x[q]);
-        so += k * im_conj_mul(l[q], po[q]);
+        s1 += k * (wi * im_conj_mul(acc_amp<T>(acc, q), x[q]) + wo * im_conj_mul(l[q], po[q]));
         s0 += re_conj_mul(acc_amp<T>(mu, q), x[q]);
       }
       write_fiber<T, Gm, TWO>(lam, pl, acc);
       if (pl.valid) {
-        g0 += s0;
-        g1 += wi * si + wo * so;
+        g0 += (double)s0;
+        g1 += (double)s1;
       }
     }
   }
@@ -527,19 +528,17 @@ __device__ __forceinline__ void heavy_adj(const Gate& g, const C<T>* __restrict_
 
 // A gate's per-lane parameter sums, reduced over the wave and added to the
 // wave's slots while the next gate's LDS reads are in flight.
-template <typename T>
 struct Sums {
-  T g0 = (T)0, g1 = (T)0;
+  double g0 = 0.0, g1 = 0.0;
   int gi = -1;
   template <typename Gm>
   __device__ __forceinline__ void flush(double* gsl, bool first) {
     if (gi < 0) return;
-    g0 = wave_sum(g0);
-    g1 = wave_sum(g1);
-    if ((threadIdx.x & 63) == kWaveSumLane) {  // each wave owns its slots: deterministic
-      double* slot = gsl + gi * 2 * Gm::NW + wave_index();
-      slot[0] = first ? (double)g0 : slot[0] + (double)g0;
-      slot[Gm::NW] = first ? (double)g1 : slot[Gm::NW] + (double)g1;
+    const double g = wave_sum_pair(g0, g1);
+    const int lane = threadIdx.x & 63;
+    if ((lane & 31) == 31) {  // each wave owns its slots: deterministic
+      double* slot = gsl + (gi * 2 + (lane >> 5)) * Gm::NW + wave_index();
+      slot[0] = first ? g : slot[0] + g;
     }
   }
 };
@@ -548,24 +547,24 @@ struct Sums {
 template <typename T, typename Gm>
 __device__ __forceinline__ void gate_adj(const Gate& g, int gi, const C<T>* __restrict__ table,
                                          const Walk<T, Gm>& wk, const C<T>* ph, C<T>*& at, C<T>* lam, double* gsl,
-                                         bool first, Sums<T>& sum, const AdjOp<T, Gm>& op, AdjOp<T, Gm>& next) {
+                                         bool first, Sums& sum, const AdjOp<T, Gm>& op, AdjOp<T, Gm>& next) {
   next.load(table, g.padj, g.two & 4);
-  T g0 = (T)0, g1 = (T)0;
+  double g0 = 0.0, g1 = 0.0;
   if (g.kind <= SFAMD_OP_KERR) {
     const C<T>* w0 = ph + g.fwd;
     const int kd = (int)__builtin_amdgcn_ubfe(wk.digits, 5 * g.a0, 5);
     wk.each([&](int d, int o) {
       const int k = g.a0 == 0 ? d : kd;
       const C<T> w = cconj(w0[k]), l = lam[o], x = at[o];
-      g0 -= (T)(g.kind == SFAMD_OP_KERR ? k * k : k) * im_conj_mul(l, x);
+      g0 -= (double)(g.kind == SFAMD_OP_KERR ? k * k : k) * ((double)l.re * x.im - (double)l.im * x.re);
       lam[o] = cmul(w, l);
       at[o] = cmul(w, x);
     });
-    sum.template flush<Gm>(gsl, first);
+    sum.flush<Gm>(gsl, first);
   } else {
     const bool two = g.two & 1;
     const int N = Gm::items(two);
-    auto flush = [&]() { sum.template flush<Gm>(gsl, first); };
+    auto flush = [&]() { sum.flush<Gm>(gsl, first); };
     if (wave_index() >= N) flush();
     if (two)
       heavy_adj<T, Gm, true>(g, table, at - Gm::GS, lam, op, g0, g1, flush);
@@ -634,13 +633,13 @@ k_mst_adj(const C<T>* __restrict__ psi_in, const C<T>* __restrict__ lam_out, C<T
     }
     AdjOp<T, Gm> opA, opB;
     opA.load(table, a.hl_adj, a.hl_two);
-    Sums<T> sum;
+    Sums sum;
     for (int gi = last; gi >= 0; gi -= 2) {
       gate_adj<T, Gm>(a.g[gi], gi, table, wk, ph, at, lam, gsl, grp == tr.first, sum, opA, opB);
       if (gi == 0) break;
       gate_adj<T, Gm>(a.g[gi - 1], gi - 1, table, wk, ph, at, lam, gsl, grp == tr.first, sum, opB, opA);
     }
-    sum.template flush<Gm>(gsl, grp == tr.first);
+    sum.flush<Gm>(gsl, grp == tr.first);
     wk.store(lam, lam_in);
     __syncthreads();  // the tiles are free for the next group's loads
   }

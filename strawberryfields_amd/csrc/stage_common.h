@@ -51,6 +51,25 @@ __device__ __forceinline__ float wave_sum(float v) {
   return v;
 }
 
+// Sums of a and b over the 64 lanes of a wave in one reduction: swapping the
+// upper half of a with the lower half of b leaves a's pair sums in lanes 0 to 31
+// and b's in lanes 32 to 63 after one addition.  a's sum is valid in lane 31, b's
+// in lane 63.
+__device__ __forceinline__ double wave_sum_pair(double a, double b) {
+  const unsigned long long ua = (unsigned long long)__double_as_longlong(a);
+  const unsigned long long ub = (unsigned long long)__double_as_longlong(b);
+  const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)ua, (unsigned)ub, false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(ua >> 32), (unsigned)(ub >> 32), false, false);
+  double v = __longlong_as_double((long long)(((unsigned long long)hi[0] << 32) | lo[0])) +
+             __longlong_as_double((long long)(((unsigned long long)hi[1] << 32) | lo[1]));
+  v += dpp_move<0xB1, 0xF>(v);   // quad_perm [1, 0, 3, 2]
+  v += dpp_move<0x4E, 0xF>(v);   // quad_perm [2, 3, 0, 1]
+  v += dpp_move<0x141, 0xF>(v);  // row_half_mirror
+  v += dpp_move<0x140, 0xF>(v);  // row_mirror
+  v += dpp_move<0x142, 0xA>(v);  // row_bcast:15 into rows 1, 3
+  return v;
+}
+
 // Workgroups are dealt to the 8 XCDs round-robin (block b runs on XCD b % 8),
 // and each XCD has its own L2.  Neighbouring tiles share cache lines whenever
 // the innermost non-local mode has a small stride, so the tiles are cut into 8

@@ -1,0 +1,58 @@
+"""Matrix-core stages, the plans that choose them and what a forward keeps."""
+import numpy as np
+import pytest
+import torch
+
+from strawberryfields_amd import circuits, runtime
+
+pytestmark = pytest.mark.gpu
+
+C64, C128 = torch.complex64, torch.complex128
+DEV = torch.device("cuda:0") if torch.cuda.is_available() else None
+
+
+def _sweep(cc, params, st, lam):
+    """Forward with every step input kept, then the adjoint: out, lam_in, grads [nops, 2]."""
+    cc.build_table(params)
+    saved = [st] + [cc.new_state(i) for i in range(1, cc.nsteps)]
+    out = cc.forward(0, cc.nsteps, st, saved=saved)
+    gin = cc.new_state(0)
+    grads = torch.zeros(2 * cc.nops, dtype=torch.float64, device=DEV)
+    cc.adjoint(0, cc.nsteps, saved, lam, gin, grads)
+    return out, gin, grads.reshape(-1, 2)
+
+
+# ------------------------------------------------------------- gradient sums
+@pytest.mark.parametrize("dtype", [C64, C128])
+def test_stage_gradients_are_summed_in_64_bits(dtype):
+    """All gates at parameter zero are exact identities, and their derivatives
+    exact on the amplitudes used, so every product is a whole number below 2^25
+    and the sums are exact in 64 bits: one addend of 2^24 among ones, which 32
+    bits drop.  (R: -sum k Im conj(l) x; K with k^2; D: Re conj(l_1) x_0.)"""
+    n, D = 4, 8
+    ops = [("R", (0,)), ("D", (1,)), ("K", (2,))]
+    cc = runtime.CompiledCircuit(ops, n, D, False, dtype, DEV, fuse=3)
+    assert cc.nsteps == 1
+    st = torch.zeros([D] * n, dtype=dtype)
+    lam = torch.zeros([D] * n, dtype=dtype)
+    v = torch.ones(D, D, D, dtype=torch.float64)  # digits of modes 0, 2, 3
+    v[1, 1, 5] = v[1, 1, 3] = 2.0**24
+    st[:, 0] = 1.0
+    lam[:, 0] = -1j * v.to(dtype)
+    lam[:, 1] = v.to(dtype)
+    k = torch.arange(D, dtype=torch.float64)
+    want = [-(k[:, None, None] * v).sum(), v.sum(), -(k[None, :, None] ** 2 * v).sum()]
+    _, _, grads = _sweep(cc, torch.zeros(3, 2, dtype=torch.float64, device=DEV), st.to(DEV), lam.to(DEV))
+    assert grads[:, 0].cpu().tolist() == [float(w) for w in want]
+
+
+def test_stage_phase_gradient_subtracts_per_amplitude():
+    """The second-parameter sum of an identity gate is zero amplitude by
+    amplitude, also where the two halves' own sums leave the range of 32 bits."""
+    n, D = 3, 8
+    cc = runtime.CompiledCircuit([("D", (1,))], n, D, False, C64, DEV, fuse=3)
+    st = torch.zeros([D] * n, dtype=C64)
+    st[0, 2:4, 0] = 1e19
+    lam = -1j * st
+    _, _, grads = _sweep(cc, torch.zeros(1, 2, dtype=torch.float64, device=DEV), st.to(DEV), lam.to(DEV))
+    assert float(grads[0, 1]) == 0.0
