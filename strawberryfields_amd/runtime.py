@@ -294,8 +294,9 @@ class CircuitFunction(torch.autograd.Function):
         cc = ctx.cc
         if not ctx.segs:
             return None, g_out, None, None
-        ckpts = ctx.saved_tensors[: len(ctx.segs)]
-        inner = list(ctx.saved_tensors[len(ctx.segs) :])  # the last segment's inputs, if the forward kept them
+        saved = ctx.saved_tensors  # read once: every read unpacks them again under saved-tensor hooks
+        ckpts = saved[: len(ctx.segs)]
+        inner = list(saved[len(ctx.segs) :])  # the last segment's inputs, if the forward kept them
         # the gate table may have been rebuilt by another run of the same plan
         cc.build_table(ctx.params, force=False)
         grads = torch.zeros(cc.nops * 2, dtype=torch.float64, device=cc.device)

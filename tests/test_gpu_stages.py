@@ -56,3 +56,29 @@ def test_stage_phase_gradient_subtracts_per_amplitude():
     lam = -1j * st
     _, _, grads = _sweep(cc, torch.zeros(1, 2, dtype=torch.float64, device=DEV), st.to(DEV), lam.to(DEV))
     assert float(grads[0, 1]) == 0.0
+
+
+# ------------------------------------------------------------- what a forward keeps
+def _kept_case(n=4, D=8, layers=2, fuse=0):
+    ops = [o[:2] for o in circuits.layered(n, layers, np.random.default_rng(0))]
+    cc = runtime.CompiledCircuit(ops, n, D, False, C64, DEV, fuse=fuse)
+    vac = torch.zeros([D] * n, dtype=C64, device=DEV)
+    vac.view(-1)[0] = 1.0
+    rng = np.random.default_rng(3)
+    params = torch.tensor(rng.uniform(0, 0.4, (len(ops), 2)), dtype=torch.float64, device=DEV, requires_grad=True)
+    return cc, vac, params
+
+
+@pytest.mark.parametrize("segment", [None, 5])
+def test_checkpointed_circuits(segment):
+    """Under torch's checkpoint the backward may read its saved tensors once."""
+    from torch.utils.checkpoint import checkpoint
+
+    cc, vac, params = _kept_case()
+    grads = []
+    for wrap in (False, True):
+        params.grad = None
+        run = lambda p: runtime.run_circuit(cc, p, vac, segment)[..., 1].abs().square().sum()  # noqa: E731
+        (checkpoint(run, params, use_reentrant=False) if wrap else run(params)).backward()
+        grads.append(params.grad)
+    assert torch.equal(*grads)
