@@ -18,8 +18,10 @@ needs the forward states; it cannot un-compute them).
 This replaces the TF backend's tape (``tfbackend/circuit.py:72-76`` keeps every
 state; ``tfbackend/ops.py:190-204,318-366`` give the per-gate VJPs).
 """
+import collections
 import ctypes
 import math
+import threading
 
 import numpy as np
 import torch
@@ -28,7 +30,8 @@ from . import _lib
 
 # default memory budget for keeping every operation input alive in backward
 DEFAULT_SAVE_BUDGET = 16 * 2**30
-# step inputs a differentiable forward keeps without a look at the free memory (a 4500th of the card)
+# step inputs that the differentiable forwards on a device keep, all together,
+# without a look at its free memory (a 4500th of the card)
 KEEP_ALWAYS = 64 * 2**20
 
 
@@ -50,6 +53,39 @@ def default_fuse(n, D):
         return 0
     want = 5 if D <= 3 else 4 if D <= 5 or (D == 6 and n >= 7) else 3 if D <= 16 else 2
     return min(want, n)
+
+
+class _KeptInputs:
+    """A share of the bytes that differentiable forwards may keep on a device,
+    held by the autograd node that keeps them and given back when it is freed."""
+
+    _lock = threading.Lock()
+    _held = {}  # by device, what was given back not yet subtracted
+    _back = collections.deque()  # appended to by __del__, which may run anywhere and takes no lock
+
+    def __init__(self, device, nbytes):
+        self.share = (device, nbytes)
+
+    def __del__(self):
+        self._back.append(self.share)
+
+    @classmethod
+    def reserve(cls, device, nbytes):
+        """The share, or None: beyond KEEP_ALWAYS bytes in all, at most a quarter of
+        the free memory goes to one forward and DEFAULT_SAVE_BUDGET to all."""
+        with cls._lock:
+            while cls._back:
+                dev, n = cls._back.popleft()
+                cls._held[dev] -= n
+            held = cls._held.get(device, 0) + nbytes
+            if held > KEEP_ALWAYS and (
+                held > DEFAULT_SAVE_BUDGET
+                or torch.cuda.is_current_stream_capturing()
+                or nbytes > torch.cuda.mem_get_info(device)[0] // 4
+            ):
+                return None
+            cls._held[device] = held
+            return cls(device, nbytes)
 
 
 class CompiledCircuit:
@@ -93,6 +129,7 @@ class CompiledCircuit:
         if self.D == 1:  # sizes cannot tell kets from DMs
             self.mixed_at = [self.mixed_in] * (self.nsteps + 1)
             self.mixed_at[-1] = self.final_mixed
+        self.inner_bytes = sum(self.state_bytes(i) for i in range(1, self.nsteps))  # all step inputs past the first
         buf = (ctypes.c_int32 * max(1, self.nops))()
         self.step_ops = []
         for i in range(self.nsteps):
@@ -209,8 +246,8 @@ class CompiledCircuit:
         segment=None keeps every step input when they fit in `budget` bytes,
         else uses segments of ~sqrt(nsteps) steps; an int gives the segment
         length in steps.  Within a segment the backward recomputes the
-        forward from the segment's checkpoint (the last segment's inputs may
-        be kept, see keeps_inputs).
+        forward from the segment's checkpoint (the inputs of a single segment
+        may be kept, see keeps_inputs).
         """
         ns = self.nsteps
         if ns == 0:
@@ -225,21 +262,22 @@ class CompiledCircuit:
         return [(b, min(b + segment, ns)) for b in range(0, ns, segment)]
 
     def keeps_inputs(self, b, e):
-        """Does a differentiable forward keep the inputs of the last segment's steps b..e?
+        """May a differentiable forward keep the inputs of the last segment's steps b..e?
 
         The backward begins with that segment, so keeping them saves one
         recomputation (3 modes, cutoff 11, 3 layers, complex128: 478 -> 388 us
         a gradient; 6 modes, cutoff 16, 1 layer, complex64, 45 states of 134 MB:
-        11.2 -> 8.7 ms).  They live until the backward is done, next to one
-        further segment's and to those of other forwards: beyond KEEP_ALWAYS
-        bytes only a quarter of the free memory is taken.
+        11.2 -> 8.7 ms).  They live until the backward is done.  Of several
+        segments none is kept: their lengths are chosen so that one of them fits
+        in memory, and this one would stay next to the others.  Under
+        saved-tensor hooks (checkpointing, offloading) none is kept either: what
+        they save has to be the same in every forward, and as small as it can be.
+        Returns the share of the memory that the forward holds on to (see
+        _KeptInputs), or None.
         """
-        need = sum(self.state_bytes(i) for i in range(b + 1, e))
-        if need <= KEEP_ALWAYS:
-            return e - b > 1
-        if torch.cuda.is_current_stream_capturing():
-            return False
-        return need <= torch.cuda.mem_get_info(self.device)[0] // 4
+        if b > 0 or e - b < 2 or torch._C._autograd._top_saved_tensors_default_hooks(True) is not None:
+            return None
+        return _KeptInputs.reserve(self.table.device, self.inner_bytes)
 
 
 def _params_row(p):
@@ -280,8 +318,10 @@ class CircuitFunction(torch.autograd.Function):
         cur = state_in
         for (b, e) in segs:
             ckpts.append(cur)
-            if e == cc.nsteps and cc.keeps_inputs(b, e):
-                inner = [cc.new_state(i) for i in range(b + 1, e)]
+            if e == cc.nsteps:
+                ctx.kept = cc.keeps_inputs(b, e)
+                if ctx.kept:
+                    inner = [cc.new_state(i) for i in range(b + 1, e)]
             cur = cc.forward(b, e, cur, saved=[cur] + inner if inner else None)
         ctx.cc = cc
         ctx.segs = segs

@@ -69,6 +69,44 @@ def _kept_case(n=4, D=8, layers=2, fuse=0):
     return cc, vac, params
 
 
+def test_pending_forwards_keep_no_more_than_the_budget(monkeypatch):
+    """Losses of many circuits summed before one backward: all their forwards
+    together hold at most the budget, and give it back with their graphs."""
+    cc, vac, params = _kept_case()
+    need = sum(cc.state_bytes(i) for i in range(1, cc.nsteps))
+    monkeypatch.setattr(runtime, "KEEP_ALWAYS", int(1.5 * need))
+    monkeypatch.setattr(runtime, "DEFAULT_SAVE_BUDGET", int(3.5 * need))
+    for _ in range(2):
+        start = torch.cuda.memory_allocated(DEV)
+        outs = [runtime.run_circuit(cc, params, vac) for _ in range(8)]
+        others = 8 * cc.state_bytes(0)  # the states returned
+        assert torch.cuda.memory_allocated(DEV) - start <= 3.5 * need + others + 8 * 2**10
+        loss = sum(o[..., 1].abs().square().sum() for o in outs)
+        params.grad = None
+        loss.backward()
+        grad = params.grad
+        outs = loss = None
+        assert torch.cuda.memory_allocated(DEV) - start < need
+    one = runtime.run_circuit(cc, params, vac)[..., 1].abs().square().sum()
+    params.grad = None
+    one.backward()
+    assert float((grad - 8 * params.grad).abs().max()) <= 1e-12 * float(grad.abs().max())
+
+
+@pytest.mark.parametrize("segment", [3, 10])
+def test_segments_hold_their_checkpoints_only(segment):
+    """A segment length is given to save memory: between forward and backward
+    one state per segment is held, besides the one returned."""
+    cc, vac, params = _kept_case()
+    assert cc.nsteps > 2 * segment
+    start = torch.cuda.memory_allocated(DEV)
+    out = runtime.run_circuit(cc, params, vac, segment)
+    held = torch.cuda.memory_allocated(DEV) - start
+    nseg = (cc.nsteps + segment - 1) // segment
+    assert held <= nseg * cc.state_bytes(0) + 2**10
+    out[..., 1].abs().square().sum().backward()
+
+
 @pytest.mark.parametrize("segment", [None, 5])
 def test_checkpointed_circuits(segment):
     """Under torch's checkpoint the backward may read its saved tensors once."""
@@ -79,6 +117,29 @@ def test_checkpointed_circuits(segment):
     for wrap in (False, True):
         params.grad = None
         run = lambda p: runtime.run_circuit(cc, p, vac, segment)[..., 1].abs().square().sum()  # noqa: E731
+        (checkpoint(run, params, use_reentrant=False) if wrap else run(params)).backward()
+        grads.append(params.grad)
+    assert torch.equal(*grads)
+
+
+def test_checkpointed_forwards_save_the_same_tensors_every_time(monkeypatch):
+    """torch's checkpoint compares what the recomputation saves with what the
+    first run saved; the free memory differs between the two."""
+    from torch.utils.checkpoint import checkpoint
+
+    cc, vac, params = _kept_case()
+    monkeypatch.setattr(runtime, "KEEP_ALWAYS", 0)
+    free = [0]
+
+    def mem_get_info(device=None):
+        free[0] = 2**40 - free[0]
+        return free[0], 2**40
+
+    monkeypatch.setattr(torch.cuda, "mem_get_info", mem_get_info)
+    grads = []
+    for wrap in (False, True):
+        params.grad = None
+        run = lambda p: runtime.run_circuit(cc, p, vac)[..., 1].abs().square().sum()  # noqa: E731
         (checkpoint(run, params, use_reentrant=False) if wrap else run(params)).backward()
         grads.append(params.grad)
     assert torch.equal(*grads)
