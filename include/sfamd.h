@@ -287,6 +287,9 @@ typedef struct {
  * step per operation.  With fuse_K | SFAMD_FUSE_MIXED the unitary gates on a
  * density matrix are grouped the same way.  Host memory only. */
 #define SFAMD_FUSE_MIXED 0x100
+/* With fuse_K | SFAMD_FUSE_PAYING matrix-core stages of too few gates to pay run
+ * gate by gate. */
+#define SFAMD_FUSE_PAYING 0x200
 int sfamd_prog_create(const sfamd_op_t* ops, int nops, int n, int D,
                       int mixed_in, int dtype, int fuse_K, sfamd_prog_t** out);
 int sfamd_prog_info(const sfamd_prog_t* prog, sfamd_prog_info_t* info);
@@ -295,6 +298,10 @@ int64_t sfamd_prog_state_elems(const sfamd_prog_t* prog, int i);
 /* operation indices of step `step` in execution order; returns their count */
 int sfamd_prog_step_ops(const sfamd_prog_t* prog, int step, int32_t* ops_out,
                         int cap);
+/* how step `step` runs: 0 one operation, 1 a run of rotation / Kerr gates, 2 a
+ * vector-ALU stage, 3 a matrix-core stage; with forward_only a step of
+ * sfamd_prog_run.  SFAMD_E_ARG past the last step. */
+int sfamd_prog_step_kind(const sfamd_prog_t* prog, int forward_only, int step);
 int sfamd_prog_destroy(sfamd_prog_t* prog);
 
 /* Gate table of all operations from the device parameter vector

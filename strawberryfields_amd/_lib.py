@@ -25,7 +25,8 @@ C64, C128 = 0, 1
     OP_CROSS_KERR,
     OP_CUBIC_PHASE,
 ) = range(11)
-FUSE_MIXED = 0x100  # fuse_K flag of sfamd_prog_create: stages on density matrices too
+# fuse_K flags of sfamd_prog_create: stages on density matrices too; only matrix-core stages that pay
+FUSE_MIXED, FUSE_PAYING = 0x100, 0x200
 
 OP_KINDS = {
     "R": OP_ROTATION,
@@ -117,6 +118,7 @@ SIGNATURES = {
     "sfamd_prog_info": (_I, [_P, ctypes.POINTER(ProgInfo)]),
     "sfamd_prog_state_elems": (_I64, [_P, _I]),
     "sfamd_prog_step_ops": (_I, [_P, _I, ctypes.POINTER(ctypes.c_int32), _I]),
+    "sfamd_prog_step_kind": (_I, [_P, _I, _I]),
     "sfamd_prog_destroy": (_I, [_P]),
     "sfamd_prog_build_table": (_I, [_P, _P, _P, _P]),
     "sfamd_prog_forward": (_I, [_P, _I, _I, _P, _P, _P, ctypes.POINTER(_P), _P, _P]),

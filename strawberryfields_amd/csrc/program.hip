@@ -315,7 +315,7 @@ struct Step {
 };
 
 struct sfamd_prog {
-  int n, D, dtype, mixed_in, nops, nwg, fuse_K, fuse_mixed;
+  int n, D, dtype, mixed_in, nops, nwg, fuse_K, fuse_mixed, fuse_paying;
   std::vector<OpPlan> ops;
   std::vector<int32_t> img0, img1;          // per op: its vector-ALU stage images, or copies of its phases; -1: none
   std::vector<int32_t> mimg_fwd, mimg_adj;  // per op: its matrix-core images, or -1
@@ -406,6 +406,23 @@ Step new_step(int kind, int op) {
   memset(&st.margs, 0, sizeof(st.margs));
   memset(&st.run, 0, sizeof(st.run));
   return st;
+}
+
+// An operation on its own: consecutive rotation / Kerr gates on the same
+// representation share one pass
+void add_single(const sfamd_prog* p, int i, std::vector<Step>* steps) {
+  if (is_diag_kind(p->ops[i].kind) && !steps->empty()) {
+    Step& last = steps->back();
+    if (last.kind <= kStepDiagRun && is_diag_kind(p->ops[last.ops.back()].kind) &&
+        p->ops[last.ops.back()].mixed_in == p->ops[i].mixed_in && (int)last.ops.size() < kDiagRunMax) {
+      last.ops.push_back(i);
+      last.kind = kStepDiagRun;
+      return;
+    }
+  }
+  Step st = new_step(kStepSingle, i);
+  st.ops.push_back(i);
+  steps->push_back(st);
 }
 
 constexpr int kMstGatesForTwo = 4;            // gates each of two workgroups per CU must still hold
@@ -697,13 +714,99 @@ void order_stages(const sfamd_prog* p, std::vector<Step>* steps, size_t first, s
   }
 }
 
+int64_t state_mb(const sfamd_prog* p, bool mixed) {
+  return ipow(p->D, mixed ? 2 * p->n : p->n) * elem_size(p->dtype) / 1000000;
+}
+
+// How many gates make a matrix-core stage pay?  A stage costs its launches (on a
+// density matrix two, its adjoint five), tiles that stride over the state and
+// the gates' operator images in the table build; a gate alone is one coalesced
+// pass, or two on a density matrix.  gate_weight: what a gate alone costs, in
+// halves of a single-mode gate's pass.  stage_need: what the gates of one stage
+// have to weigh together.  Measured with 1 to 9 single-mode gates (d) and 1 to 4
+// beamsplitters (b) in one stage, gates alone / stage, us:
+//   density matrices, forward, complex64: 4 modes 8 (134 MB) 1d 42 / 129, 2d 97 /
+//   145, 3d 165 / 163, 1b 202 / 132; 3 modes 9 3d 23 / 31, 6d 48 / 43, 1b 28 / 25; 12
+//   3d 48 / 66, 6d 94 / 92, 1b 55 / 52; 16 6d 409 / 464, 9d 608 / 564, 2b 282 / 370, 4b
+//   570 / 409; 7 modes 3 3d 104 / 142, 6d 208 / 206; 2 modes 8 1d 7 / 10, 2d 10 / 12,
+//   3d 13 / 11; complex128: 3 modes 9 1d 20 / 35, 2d 43 / 50, 3d 67 / 50, 1b 26 / 38, 2b 62 /
+//   48; 16 1d 320 / 390, 2d 628 / 467; 20 2d 3103 / 3172, 3d 5659 / 3627; 7 modes 3 3d
+//   158 / 168, 6d 310 / 255;
+//   their adjoints: complex64 4 modes 8 2d 531 / 594, 3d 802 / 704, 1b 479 / 519; 3 modes
+//   12 2d 172 / 208, 3d 258 / 250, 1b 147 / 186, 2b 302 / 243; complex128 3 modes 9 1d 86 /
+//   124, 2d 168 / 158; 6 modes 3 3d 109 / 135, 6d 210 / 204;
+//   kets, forward: complex64 9 modes 5 1d 9 / 18, 2d 19 / 21, 3d 28 / 28; 13 modes 3 3d
+//   28 / 38, 6d 56 / 48; 20 modes 2 9d 68 / 68; 8 modes 8 1d 42 / 57, 2d 86 / 69; complex128
+//   13 modes 3 6d 55 / 57; adjoints: complex64 8 modes 8 1d 146 / 192, 2d 294 / 276;
+//   complex128 12 modes 3 6d 82 / 90.
+// Where the gate alone has no kernel that reads whole fibers with coalesced runs (a
+// pair with the last mode, a complex128 gate on it), or one thread per fiber leaves
+// the device idle (complex128 on few fibers), it costs a multiple: CK on 6 modes 16
+// complex64 98 / 63, BS on the last modes of 6 modes 8 complex128 19 / 7, D on 4 modes
+// 15 complex128 18 / 7.
+int gate_weight(const sfamd_prog* p, const Stages& sg, const OpPlan& op) {
+  const int n = p->n, D = p->D;
+  const bool two = two_mode_kind(op.kind);
+  const int64_t N = ipow(D, sg.axes);
+  int64_t inner = ket_stride(n, D, op.m0);  // the innermost run of the gate's passes
+  if (two) inner = std::min(inner, ket_stride(n, D, op.m1));
+  if (sg.mixed) inner *= inner;
+  const bool fib = use_fib(D, inner), tiny = N < kSlabMinState;
+  if (p->dtype == SFAMD_C64) {
+    if (!two) return 2;
+    if (!sg.mixed) return tiny ? 3 : !fib ? (D <= 5 ? 6 : 5) : N <= (1 << 21) ? 4 : 3;
+    if (n == 2) return D <= 12 ? 2 : 4;
+    if (tiny) return 4;
+    return D > 10 || (D > 8 && dm_pair_mfma_supported(n, D, op.m0, op.m1, p->dtype)) ? 6 : 8;
+  }
+  const bool few = D >= 8 && N / D < (sg.mixed ? 16384 : 65536);
+  if (sg.mixed) {
+    if (two && (D <= 3 || n == 2)) return D <= 12 && n == 2 ? 2 : 4;
+    if (fib || N < 1500000) return few ? 4 : 2;
+    return op.kind == SFAMD_OP_TWO_MODE_SQUEEZE || (!two && D > 12) ? 6 : 4;
+  }
+  if (!fib) return tiny ? 2 : two && D < 6 ? 4 : 6;
+  return few || (!two && D >= 8) ? 4 : two ? 3 : 2;
+}
+
+int stage_need(const sfamd_prog* p, const Stages& sg, bool forward_only) {
+  const int n = p->n, D = p->D;
+  const bool c64 = p->dtype == SFAMD_C64, large = state_mb(p, sg.mixed) >= 16;
+  if (sg.mixed && c64) {
+    if (n == 2) return D <= 12 ? 4 : 6;
+    if ((D <= 3 || D == 5) && large) return 12;  // tiles of few amplitudes, operands mostly padding
+    if (forward_only) return D <= 12 ? 8 : 16;
+    return D <= 3 || D == 11 || D == 12 ? 8 : 6;
+  }
+  if (sg.mixed) return D <= 3 ? 8 : D <= 12 || n == 2 ? 4 : 6;
+  if (D <= 3 && ipow(D, n) >= kSlabMinState) return large ? 10 : c64 || forward_only ? 6 : 8;
+  return D == 5 && forward_only ? 6 : 4;
+}
+
+// what the operations `ops` of a stage weigh; rotation and Kerr gates share one pass
+int stage_weight(const sfamd_prog* p, const Stages& sg, const std::vector<int>& ops) {
+  int w = 0, diag = 0;
+  for (int i : ops) {
+    if (is_diag_kind(p->ops[i].kind))
+      diag = 2;
+    else
+      w += gate_weight(p, sg, p->ops[i]);
+  }
+  return w + diag;
+}
+
 // greedy partition of a run of fusable ops into stages of Kc local modes
 void plan_run(const sfamd_prog* p, const std::vector<int>& run, const Stages& sg, bool forward_only,
               std::vector<Step>* steps) {
   const int n = p->n, kind = sg.kind, Kc = sg.modes(n);
   const StageCost sc = stage_cost(p, sg, forward_only);
-  std::vector<unsigned> masks;  // of this run's steps
-  size_t nstages = 0;           // its matrix-core stages
+  // stages that do not pay run gate by gate, if the caller asks for that: each by
+  // itself, but kets forward only all or none (their stages share a mode order)
+  const bool paying = p->fuse_paying && kind == kStepMatrixStage, ordered = forward_only && !sg.mixed;
+  const int need = paying ? stage_need(p, sg, forward_only) : 0;
+  std::vector<unsigned> masks;     // of this run's stages
+  bool all_stages = true;
+  const size_t first = steps->size();
   std::vector<int> rem = run;
   std::vector<unsigned> cands;
   // all Kc-subsets when few, else subsets grown from the next ops
@@ -771,24 +874,26 @@ void plan_run(const sfamd_prog* p, const std::vector<int>& run, const Stages& sg
     }
     if (best.empty()) {
       // no stage holds the next operation: it runs on its own, unfused
-      Step one = new_step(kStepSingle, rem.front());
-      one.ops.push_back(rem.front());
-      steps->push_back(one);
-      masks.push_back(0);
+      add_single(p, rem.front(), steps);
+      all_stages = false;
       rem.erase(rem.begin());
       continue;
     }
-    Step st = new_step(kind, best.front());
-    st.K = sg.Kc;
-    st.mixed = sg.mixed;
-    st.ops = best;
-    if (kind == kStepStage)
-      fill_stage(p, st, bm);
-    else
-      fill_matrix_step(p, st, bm);
-    steps->push_back(st);
-    masks.push_back(bm);
-    nstages += kind == kStepMatrixStage;
+    if (paying && !ordered && stage_weight(p, sg, best) < need) {
+      for (int i : best) add_single(p, i, steps);
+      all_stages = false;
+    } else {
+      Step st = new_step(kind, best.front());
+      st.K = sg.Kc;
+      st.mixed = sg.mixed;
+      st.ops = best;
+      if (kind == kStepStage)
+        fill_stage(p, st, bm);
+      else
+        fill_matrix_step(p, st, bm);
+      steps->push_back(st);
+      masks.push_back(bm);
+    }
     std::vector<int> nrem;
     size_t bi = 0;
     for (int i : rem) {
@@ -799,40 +904,31 @@ void plan_run(const sfamd_prog* p, const std::vector<int>& run, const Stages& sg
     }
     rem.swap(nrem);
   }
-  if (forward_only && !sg.mixed && nstages == masks.size())
-    order_stages(p, steps, steps->size() - masks.size(), masks);
+  if (!ordered || kind != kStepMatrixStage) return;
+  int w = 0;
+  for (size_t i = first; i < steps->size(); ++i) w += stage_weight(p, sg, (*steps)[i].ops);
+  if (paying && w < need * (int)(steps->size() - first)) {
+    steps->resize(first, new_step(kStepSingle, 0));
+    for (int i : run) add_single(p, i, steps);
+  } else if (all_stages) {
+    order_stages(p, steps, first, masks);
+  }
 }
 
 // sg: the stages on kets and on density matrices
 void plan_steps(const sfamd_prog* p, const Stages (&sg)[2], bool forward_only, std::vector<Step>* steps) {
   const int n = p->n, D = p->D;
-  auto is_diag = [&](int i) { return is_diag_kind(p->ops[i].kind); };
   std::vector<int> run;
-  auto single = [&](int i) {
-    // consecutive rotation / Kerr gates on the same representation share one pass
-    if (is_diag(i) && !steps->empty()) {
-      Step& last = steps->back();
-      if (last.kind <= kStepDiagRun && is_diag(last.ops.back()) &&
-          p->ops[last.ops.back()].mixed_in == p->ops[i].mixed_in && (int)last.ops.size() < kDiagRunMax) {
-        last.ops.push_back(i);
-        last.kind = kStepDiagRun;
-        return;
-      }
-    }
-    Step st = new_step(kStepSingle, i);
-    st.ops.push_back(i);
-    steps->push_back(st);
-  };
   auto flush = [&]() {
     if (run.empty()) return;
     const Stages& g = sg[p->ops[run.front()].mixed_in];
     // on a density matrix rotation and Kerr gates alone take one pass, a stage two
     bool heavy = !g.mixed;
-    for (int i : run) heavy = heavy || !is_diag(i);
+    for (int i : run) heavy = heavy || !is_diag_kind(p->ops[i].kind);
     if (heavy)
       plan_run(p, run, g, forward_only, steps);
     else
-      for (int i : run) single(i);
+      for (int i : run) add_single(p, i, steps);
     run.clear();
   };
   for (int i = 0; i < p->nops; ++i) {
@@ -843,7 +939,7 @@ void plan_steps(const sfamd_prog* p, const Stages (&sg)[2], bool forward_only, s
       continue;
     }
     flush();
-    single(i);
+    add_single(p, i, steps);
   }
   flush();
   for (Step& st : *steps) {
@@ -1213,8 +1309,10 @@ extern "C" int sfamd_prog_create(const sfamd_op_t* ops, int nops, int n, int D, 
   p->dtype = dtype;
   p->mixed_in = mixed_in ? 1 : 0;
   p->nops = nops;
-  p->fuse_K = fuse_K & ~SFAMD_FUSE_MIXED;
-  p->fuse_mixed = (fuse_K & SFAMD_FUSE_MIXED) != 0;
+  // negative: none, as zero
+  p->fuse_K = fuse_K < 0 ? 0 : fuse_K & ~(SFAMD_FUSE_MIXED | SFAMD_FUSE_PAYING);
+  p->fuse_mixed = fuse_K >= 0 && (fuse_K & SFAMD_FUSE_MIXED) != 0;
+  p->fuse_paying = fuse_K >= 0 && (fuse_K & SFAMD_FUSE_PAYING) != 0;
   int mixed = p->mixed_in;
   int64_t max_state = ipow(D, mixed ? 2 * n : n);
   for (int i = 0; i < nops; ++i) {
@@ -1279,6 +1377,12 @@ extern "C" int sfamd_prog_step_ops(const sfamd_prog_t* p, int step, int32_t* ops
   const Step& st = p->steps[step];
   for (int i = 0; i < (int)st.ops.size() && i < cap; ++i) ops_out[i] = st.ops[i];
   return (int)st.ops.size();
+}
+
+extern "C" int sfamd_prog_step_kind(const sfamd_prog_t* p, int forward_only, int step) {
+  if (!p) return SFAMD_E_ARG;
+  const std::vector<Step>& steps = forward_only && !p->fsteps.empty() ? p->fsteps : p->steps;
+  return step < 0 || step >= (int)steps.size() ? SFAMD_E_ARG : steps[step].kind;
 }
 
 extern "C" int sfamd_prog_destroy(sfamd_prog_t* p) {

@@ -92,8 +92,11 @@ class CompiledCircuit:
     """A planned circuit (structure only) bound to one device and dtype.
 
     The plan is a list of steps: fused stages (many gates on LDS tiles of
-    ``fuse`` local modes) or single operations.  Checkpoints and
-    segments are expressed in steps; gradients are indexed by operation.
+    ``fuse`` local modes) or single operations.  The default (``fuse=None``)
+    stages gates where enough of them share a tile to pay; a number asks for
+    stages of that many local modes however few gates they hold, and 0 for
+    none.  Checkpoints and segments are expressed in steps; gradients are
+    indexed by operation.
     """
 
     def __init__(self, ops, n, D, mixed_in, dtype, device, fuse=None):
@@ -112,6 +115,8 @@ class CompiledCircuit:
         handle = ctypes.c_void_p()
         self.fuse = default_fuse(self.n, self.D) if fuse is None else int(fuse)
         fuse_K = self.fuse | _lib.FUSE_MIXED if self.fuse >= 2 else self.fuse
+        if fuse is None and self.fuse >= 2:
+            fuse_K |= _lib.FUSE_PAYING
         st = self.lib.sfamd_prog_create(
             arr, len(self.ops), self.n, self.D, int(self.mixed_in), self.code, fuse_K, ctypes.byref(handle)
         )
@@ -149,6 +154,15 @@ class CompiledCircuit:
             except Exception:  # interpreter shutdown
                 pass
             self.handle = None
+
+    def step_kinds(self, forward_only=False):
+        """How each step runs: "op", "diag" (a run of R / K gates), "vector" or
+        "matrix" (stages); forward_only: the steps of a run without gradients."""
+        kinds, i = [], 0
+        while (k := self.lib.sfamd_prog_step_kind(self.handle, int(forward_only), i)) >= 0:
+            kinds.append(("op", "diag", "vector", "matrix")[k])
+            i += 1
+        return kinds
 
     # ---- shapes
     def state_shape(self, i):

@@ -143,3 +143,33 @@ def test_checkpointed_forwards_save_the_same_tensors_every_time(monkeypatch):
         (checkpoint(run, params, use_reentrant=False) if wrap else run(params)).backward()
         grads.append(params.grad)
     assert torch.equal(*grads)
+
+
+# ------------------------------------------------------------- default plans
+@pytest.mark.parametrize("dtype", [C128, C64])
+@pytest.mark.parametrize("n,D,mixed,count", [(3, 9, True, 4), (4, 4, True, 24), (3, 6, True, 60), (2, 16, True, 12),
+                                             (3, 16, False, 20), (5, 6, False, 5), (8, 2, False, 30)])
+def test_default_plans_match_unfused(dtype, n, D, mixed, count):
+    """Random programs whose runs partly leave their stages: forward with step
+    inputs, forward only, lam_in and gradients against one kernel per gate.
+    Every gate is a contraction of D terms (two on a density matrix) with unit
+    roundoff u in either path: at most about 8 (16) D m u for m operations."""
+    rng = np.random.default_rng(n * 100 + D)
+    ops = []
+    while len(ops) < count:
+        kind = ["D", "S", "R", "K", "BS", "S2", "CK", "MZ", "LOSS" if mixed else "BS"][rng.integers(9)]
+        a, b = (int(v) for v in rng.choice(n, 2, replace=False))
+        ops.append((kind, (a, b) if kind in ("BS", "S2", "CK", "MZ") else (a,)))
+    gen = torch.Generator().manual_seed(count)
+    shape = [D] * (2 * n if mixed else n)
+    st = torch.randn(shape, dtype=dtype, generator=gen).to(DEV)
+    lam = torch.randn(shape, dtype=dtype, generator=gen).to(DEV)
+    params = (torch.rand(count, 2, dtype=torch.float64, generator=gen) * 0.4).to(DEV)
+    res = []
+    for fuse in (0, None):
+        cc = runtime.CompiledCircuit(ops, n, D, mixed, dtype, DEV, fuse=fuse)
+        out, gin, grads = _sweep(cc, params, st, lam)
+        res.append((out, cc.run(st), gin, grads))
+    tol = (16 if mixed else 8) * D * count * (2.0**-24 if dtype == C64 else 2.0**-53)
+    for a, b in zip(*res):
+        assert float((a - b).abs().max()) <= tol * float(a.abs().max())

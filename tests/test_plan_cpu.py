@@ -1,0 +1,88 @@
+"""Which steps a plan takes (host memory only: no device is needed)."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from strawberryfields_amd import _lib, circuits, runtime
+
+OP, DIAG, VECTOR, MATRIX = range(4)
+
+
+class Plan:
+    """A plan's steps (kind, operations) and the kinds of its forward-only steps."""
+
+    def __init__(self, ops, n, D, mixed=False, dtype=_lib.C64, fuse=None):
+        lib = _lib.load()
+        arr = (_lib.OpDesc * len(ops))()
+        for i, (name, modes) in enumerate(ops):
+            arr[i].kind = _lib.OP_KINDS[name]
+            arr[i].mode0 = modes[0]
+            arr[i].mode1 = modes[1] if len(modes) > 1 else -1
+        K = runtime.default_fuse(n, D) | _lib.FUSE_PAYING if fuse is None else fuse
+        h = ctypes.c_void_p()
+        assert lib.sfamd_prog_create(arr, len(ops), n, D, int(mixed), dtype, K | _lib.FUSE_MIXED, ctypes.byref(h)) == 0
+        self.steps, self.run = [], []
+        buf = (ctypes.c_int32 * len(ops))()
+        while (k := lib.sfamd_prog_step_kind(h, 0, len(self.steps))) >= 0:
+            m = lib.sfamd_prog_step_ops(h, len(self.steps), buf, len(ops))
+            self.steps.append((k, buf[:m]))
+        while (k := lib.sfamd_prog_step_kind(h, 1, len(self.run))) >= 0:
+            self.run.append(k)
+        lib.sfamd_prog_destroy(h)
+
+    @property
+    def kinds(self):
+        return [k for k, _ in self.steps]
+
+
+def _layered(n, layers=1, loss=False):
+    return [o[:2] for o in circuits.layered(n, layers, np.random.default_rng(0), loss=loss)]
+
+
+# --------------------------------------------------- stages that hold too few gates
+@pytest.mark.parametrize("dtype", [_lib.C64, _lib.C128])
+@pytest.mark.parametrize(
+    "n,D,mixed,ops",
+    [(6, 16, False, [("BS", (0, 1))]), (8, 8, False, [("S2", (0, 1))]), (4, 15, False, [("CK", (0, 3))]),
+     (20, 2, False, [("MZ", (0, 1))]), (3, 9, True, [("D", (0,))]), (3, 16, True, [("S", (1,))]),
+     (4, 6, True, [("D", (0,)), ("LOSS", (0,)), ("D", (1,)), ("LOSS", (1,))]), (7, 3, True, [("D", (0,)), ("S", (1,))])],
+)
+def test_gates_that_share_no_stage_run_alone(n, D, mixed, ops, dtype):
+    """A stage of one or two gates costs more than the gates' own passes, forward
+    only and with the adjoint; an explicit tile still asks for it."""
+    plan = Plan(ops, n, D, mixed, dtype)
+    if dtype == _lib.C64 or D not in (8, 15):
+        assert set(plan.run) == {OP}
+    if dtype == _lib.C64:
+        assert set(plan.kinds) == {OP}
+    if not mixed or D <= 12:
+        assert MATRIX in Plan(ops, n, D, mixed, dtype, fuse=3).run
+
+
+@pytest.mark.parametrize("dtype", [_lib.C64, _lib.C128])
+@pytest.mark.parametrize("n,D,mixed", [(3, 8, False), (6, 8, False), (8, 5, False), (12, 2, False), (12, 3, False), (7, 16, False),
+                                       (2, 8, True), (3, 9, True), (3, 12, True), (4, 6, True), (6, 3, True), (8, 2, True)])
+def test_layers_still_run_in_stages(n, D, mixed, dtype):
+    plan = Plan(_layered(n, 1, mixed), n, D, mixed, dtype)
+    assert plan.run.count(MATRIX) >= len([k for k in plan.run if k == OP]) - n  # (a layer has n losses)
+    assert MATRIX in plan.run
+
+
+@pytest.mark.parametrize("seed", range(12))
+def test_default_plans_keep_every_gate_and_mode_order(seed):
+    """Also where some gates of a run leave their stage."""
+    rng = np.random.default_rng(seed)
+    n, D = [(2, 8), (3, 9), (4, 4), (3, 16), (6, 3), (8, 2)][seed % 6]
+    mixed = bool(seed // 6)
+    ops = []
+    for _ in range(60):
+        kind = ["D", "S", "R", "K", "BS", "S2", "CK", "MZ", "LOSS" if mixed else "D"][rng.integers(9)]
+        a, b = (int(v) for v in rng.choice(n, 2, replace=False))
+        ops.append((kind, (a, b) if kind in ("BS", "S2", "CK", "MZ") else (a,)))
+    for dtype in (_lib.C64, _lib.C128):
+        flat = [i for _, st in Plan(ops, n, D, mixed, dtype).steps for i in st]
+        assert sorted(flat) == list(range(len(ops)))
+        for m in range(n):
+            order = [i for i in flat if m in ops[i][1]]
+            assert order == sorted(order)
