@@ -993,11 +993,23 @@ bool stages_pay(const sfamd_prog* p, int kind, bool forward_only) {
 // staged, us: complex64, 2 modes cutoff 8 177 / 91, 12 225 / 159, 16 313 / 259, 18
 // 421 / 676; 3 modes 6 475 / 190, 8 679 / 176, 10 1167 / 668, 12 1763 / 1560, 13 2593 /
 // 3319, 16 5886 / 10204; complex128, 2 modes 12 374 / 220; 3 modes 8 849 / 247, 12
-// 4109 / 2633, 13 6514 / 7735.  Forward only they always pay: 3 modes cutoff 16,
-// complex64 1780 / 1356, complex128 5537 / 2387; 2 modes 20 159 / 134 and 442 / 242.
+// 4109 / 2633, 13 6514 / 7735.  Forward only they pay longer: 3 modes cutoff 16,
+// complex64 1780 / 1356, complex128 5537 / 2387; 2 modes 20 159 / 134 and 442 / 242;
+// but 3 modes 18 and 20, complex64 3858 / 4875 and 6362 / 7925.  States past the caches
+// lose in complex128 where a stage's operands are mostly padding, with cutoffs 2, 3 and 5:
+// adjoint, 10 modes 2 (17 MB) 7297 / 11013, 7 modes 3 11555 / 16077, 5 modes 5 14058 / 16726
+// (6 modes 3, 9 MB, 2150 / 1747; 6 modes 4 30208 / 24439); forward only with cutoff 2: 10
+// modes 2141 / 2228, 12 modes 33601 / 51918 (7 modes 3 3655 / 2948, 5 modes 5 4374 / 3821).
+// So do cutoffs 9 and 10 (operands half padding) on 4 modes, in both types: 9, complex64 10507 /
+// 12708 forward, 43263 / 52380 one gradient, complex128 16588 / 25757 forward; 10, complex64
+// 19682 / 23069 (3 modes 10, 16 MB, complex128 491 / 275; 4 modes 8, 268 MB, 5991 / 3002).
 bool dm_stages_pay(const sfamd_prog* p, bool forward_only) {
-  if (forward_only || p->D <= 12) return true;
-  return p->D <= 16 && p->n == 2;
+  const int D = p->D;
+  const int64_t mb = state_mb(p, true);
+  if (p->dtype == SFAMD_C128 && mb >= 12 && (D == 2 || (!forward_only && (D == 3 || D == 5)))) return false;
+  if ((D == 9 || D == 10) && mb >= 64) return false;
+  if (forward_only) return p->dtype == SFAMD_C128 || D <= 16 || p->n == 2;
+  return D <= 12 || (D <= 16 && p->n == 2);
 }
 
 constexpr int kFewTilesModes = 4;  // modes up to which there are at most D tiles of three

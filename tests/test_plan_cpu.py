@@ -69,6 +69,20 @@ def test_layers_still_run_in_stages(n, D, mixed, dtype):
     assert MATRIX in plan.run
 
 
+@pytest.mark.parametrize(
+    "n,D,dtype,forward,adjoint",
+    [(3, 18, _lib.C64, False, False), (3, 20, _lib.C64, False, False), (3, 20, _lib.C128, True, False), (2, 20, _lib.C64, True, False),
+     (10, 2, _lib.C128, False, False), (8, 2, _lib.C128, True, True), (10, 2, _lib.C64, True, True), (7, 3, _lib.C128, True, False),
+     (6, 3, _lib.C128, True, True), (5, 5, _lib.C128, True, False), (5, 5, _lib.C64, True, True), (4, 5, _lib.C128, True, True),
+     (4, 9, _lib.C64, False, False), (4, 10, _lib.C128, False, False), (3, 10, _lib.C128, True, True), (4, 8, _lib.C128, True, True)],
+)
+def test_large_density_matrices_leave_stages_where_these_lose(n, D, dtype, forward, adjoint):
+    """States past the caches where a stage's operands are mostly padding, and
+    complex64 forwards above cutoff 16, run gate by gate."""
+    plan = Plan(_layered(n, 1, True), n, D, True, dtype)
+    assert (MATRIX in plan.run, MATRIX in plan.kinds) == (forward, adjoint)
+
+
 @pytest.mark.parametrize("seed", range(12))
 def test_default_plans_keep_every_gate_and_mode_order(seed):
     """Also where some gates of a run leave their stage."""
