@@ -1,5 +1,6 @@
-// Fused pure-state gate stages of two modes: descriptors shared by the planner
-// (program.hip) and the kernels (fused.hip).  Larger stages: mstage.h.
+// Fused pure-state gate stages of two modes, at some cutoffs of three, on the
+// vector ALUs: descriptors shared by the planner (program.hip) and the kernels
+// (fused.hip).  The other stages: mstage.h.
 #pragma once
 
 #include "common.h"
@@ -8,9 +9,9 @@ namespace sfamd {
 
 constexpr int kStageMaxGates = 40;   // gates per stage (kernel-argument space)
 constexpr int kStageMaxD = 20;       // cutoffs with compiled stage kernels: 2..20
-// Cutoffs with stages of three modes: just past a matrix-core operand of 8, where
-// one is a quarter full, and large complex128 states at 5 and 6 (which stages a
-// plan takes: program.hip).
+// Cutoffs with stages of three modes: those that fill about half of a matrix-core
+// operand and less (0.42 at 9, 0.52 at 10, 0.39 at 5, 0.56 at 6; which stages a plan takes:
+// program.hip).
 __host__ __device__ constexpr bool stage_three_modes(int D, int dtype) {
   return D == 9 || (D == 10 && dtype == SFAMD_C64) || ((D == 5 || D == 6) && dtype == SFAMD_C128);
 }

@@ -1,5 +1,6 @@
-// Fused gate stages on two modes of a pure state (ket), at cutoffs 9 and
-// 10 also on three: many gates per pass, in LDS.  Tiles of D^2 amplitudes are too small to
+// Fused gate stages on two modes of a pure state (ket), where a matrix-core
+// operand would be half padding (cutoffs 9 and 10, 5 and 6 in complex128) also on
+// three: many gates per pass, in LDS.  Tiles of D^2 amplitudes are too small to
 // fill matrix-core columns; the other stages of three and more modes are in
 // mstage_impl.h.
 //

@@ -298,8 +298,8 @@ int adjoint_op(const OpPlan& op, int n, int D, const void* table, const void* ps
 }  // namespace
 
 // One step of execution: a single operation (or a run of diagonal gates), or a
-// fused stage of gates on K local modes of a pure state: on the vector ALUs
-// (K = 2, fused.hip) or on the matrix cores (K >= 3, mstage.hip).  On a density
+// fused stage of gates on K local modes: on the vector ALUs (two modes of a ket, at some
+// cutoffs three; fused.hip) or on the matrix cores (K >= 3, mstage.hip).  On a density
 // matrix a matrix-core stage is two launches: the gates on the row axes of its
 // modes, then their conjugates on the column axes.
 enum StepKind { kStepSingle = 0, kStepDiagRun, kStepStage, kStepMatrixStage };
@@ -1021,8 +1021,10 @@ constexpr int kFewTilesModes = 4;  // modes up to which there are at most D tile
 // stage of fewer modes has the other side's axes for columns.
 //
 // Circuits of R, K, D, S and BS also have vector-ALU stages, which the adjoint
-// takes where operands padded to 16 waste the matrix cores: at cutoff 9 (and 10 in
-// complex64 on 5 modes; 6 modes have too many tiles for its LDS, 64 short stages
+// takes where operands padded to 16 rows and 4 columns waste the matrix cores (the
+// share of an operand that an operator of size D fills is 0.39 at 5, 0.56 at 6, 0.42 at
+// 9, 0.52 at 10, 0.63 and more at 11 to 16 and 1 at 8): at cutoff 9 (and 10 in
+// complex64 on 4 and 5 modes; 6 modes have too many tiles for its LDS, 64 short stages
 // take 4346 us, against 951 for one layer on the matrix cores) with three modes;
 // and with two where there are at most D tiles of three modes, so that most
 // compute units idle and two modes' stages have D times the workgroups.  It also
@@ -1033,7 +1035,11 @@ constexpr int kFewTilesModes = 4;  // modes up to which there are at most D tile
 // 308 / 230, 12 363 / 306, 14 527 / 299; 4 modes 8 306 / 453, 9 551 / 388, 12 603 / 591,
 // 14 945 / 686; 5 modes 9 849 / 606, 10 833 / 740, 12 958 / 1259; 6 modes 9 2656 / 2030;
 // complex128, 3 modes 8 197 / 234, 9 357 / 293, 12 498 / 341; 4 modes 9 623 / 497, 12
-// 883 / 756, 14 1827 / 850; 5 modes 9 984 / 870, 10 989 / 1083.
+// 883 / 756, 14 1827 / 850; 5 modes 9 984 / 870, 10 989 / 1083.  4 modes 10 complex64 with
+// stages of two / three modes 497 / 478, six layers 1019 / 891 (3 modes 270 / 286).
+// Forward only they pay at cutoff 9 in complex64, on one tile's worth of workgroups per
+// compute unit and less or on many: 4 modes, 6 layers, from a graph, matrix cores / vector
+// ALUs 338 / 288, 5 modes 499 / 439, 7 modes, one layer 1789 / 1597 (6 modes 246 / 275).
 Stages pick_stages(const sfamd_prog* p, bool forward_only, bool mixed) {
   const int K = p->fuse_K < p->n ? p->fuse_K : p->n;
   Stages sg{mixed, mixed ? 2 * p->n : p->n, kStepMatrixStage, K};
@@ -1042,13 +1048,16 @@ Stages pick_stages(const sfamd_prog* p, bool forward_only, bool mixed) {
     if (!p->fuse_mixed || p->fuse_K < 2 || p->n < 2 || !stage_fits(p, sg, forward_only) || !dm_stages_pay(p, forward_only)) sg.Kc = 0;
     return sg;
   }
-  const bool large = K >= 3 && p->dtype == SFAMD_C128 && (p->D == 5 || p->D == 6) && ipow(p->D, p->n) >= 1250000;
-  bool layered = !forward_only && (large || (K == 3 && p->D > 8 && stages_pay(p, kStepMatrixStage, false)));
+  const bool large =
+      !forward_only && K >= 3 && p->dtype == SFAMD_C128 && (p->D == 5 || p->D == 6) && ipow(p->D, p->n) >= 1250000;
+  bool layered = large || (K == 3 && stages_pay(p, kStepMatrixStage, forward_only) &&
+                           (forward_only ? p->D == 9 && p->dtype == SFAMD_C64 && p->n != 6 : p->D > 8));
   for (const OpPlan& op : p->ops)
     layered = layered && (op.mixed_in || op.kind == SFAMD_OP_LOSS || op.kind == SFAMD_OP_MIX ||
                           fusable(op, Stages{false, p->n, kStepStage, 2}));
   if (layered) {
-    const bool three = stage_three_modes(p->D, p->dtype) && (large || p->D == 9 || p->n == kFewTilesModes + 1);
+    const bool three = stage_three_modes(p->D, p->dtype) &&
+                       (large || p->D == 9 || p->n == kFewTilesModes || p->n == kFewTilesModes + 1);
     const Stages valu{false, p->n, kStepStage, three ? 3 : 2};
     if ((three || p->n <= kFewTilesModes) && stage_fits(p, valu, false)) return valu;
   }
@@ -1066,11 +1075,12 @@ void plan_program(sfamd_prog* p) {
   const Stages both[2] = {pick_stages(p, false, false), pick_stages(p, false, true)};
   plan_steps(p, both, false, &p->steps);
   const Stages fwd[2] = {pick_stages(p, true, false), pick_stages(p, true, true)};
-  bool matrix = false;
-  for (const OpPlan& op : p->ops)
-    matrix = matrix || (fwd[op.mixed_in].Kc >= 3 && fwd[op.mixed_in].kind == kStepMatrixStage &&
-                        fusable(op, fwd[op.mixed_in]));
-  if (matrix) plan_steps(p, fwd, true, &p->fsteps);
+  bool other = false;  // matrix-core stages differ (see stage_cost), vector-ALU stages only where the adjoint has none
+  for (const OpPlan& op : p->ops) {
+    const Stages &f = fwd[op.mixed_in], &b = both[op.mixed_in];
+    other = other || (f.Kc >= 2 && fusable(op, f) && (f.kind == kStepMatrixStage || f.kind != b.kind || f.Kc != b.Kc));
+  }
+  if (other) plan_steps(p, fwd, true, &p->fsteps);
   // state sizes at step inputs
   p->state_elems.clear();
   for (const Step& st : p->steps) {
@@ -1130,17 +1140,19 @@ void place_table(sfamd_prog* p) {
         off += p->D;
       }
   }
+  auto place_images = [&](StageArgs& a, bool adjoint) {
+    a.img_fwd = off;
+    off += a.mat_fwd;
+    a.img_adj = off;
+    if (adjoint) off += a.mat_adj;
+    for (int gi = 0; gi < a.ngates; ++gi) {
+      p->img0[a.g[gi].op] = (int32_t)(a.img_fwd + a.g[gi].moff);
+      if (adjoint) p->img1[a.g[gi].op] = (int32_t)(a.img_adj + a.g[gi].amoff);
+    }
+  };
   for (Step& st : p->steps) {
     if (st.kind == kStepStage) {
-      StageArgs& a = st.args;
-      a.img_fwd = off;
-      off += a.mat_fwd;
-      a.img_adj = off;
-      off += a.mat_adj;
-      for (int gi = 0; gi < a.ngates; ++gi) {
-        p->img0[a.g[gi].op] = (int32_t)(a.img_fwd + a.g[gi].moff);
-        p->img1[a.g[gi].op] = (int32_t)(a.img_adj + a.g[gi].amoff);
-      }
+      place_images(st.args, true);
     } else if (st.kind == kStepMatrixStage) {
       st.margs[0].phases = st.margs[1].phases = (int32_t)off;
       for (int op : st.ops)
@@ -1150,11 +1162,18 @@ void place_table(sfamd_prog* p) {
         }
     }
   }
+  // vector-ALU stages of both plans are the same
+  for (Step& f : p->fsteps) {
+    if (f.kind != kStepStage) continue;
+    const Step* same = nullptr;
+    for (const Step& st : p->steps)
+      if (st.kind == kStepStage && st.op == f.op) same = &st;
+    if (same)
+      f.args = same->args;
+    else
+      place_images(f.args, false);
+  }
   p->table_elems = off;
-  // vector-ALU stages are the same in both plans
-  for (Step& f : p->fsteps)
-    for (size_t i = 0; f.kind == kStepStage && i < p->steps.size(); ++i)
-      if (p->steps[i].kind == kStepStage && p->steps[i].op == f.op) f.args = p->steps[i].args;
   for (std::vector<Step>* steps : {&p->steps, &p->fsteps})
     for (Step& st : *steps) {
       if (st.kind == kStepMatrixStage)

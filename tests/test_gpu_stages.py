@@ -173,3 +173,21 @@ def test_default_plans_match_unfused(dtype, n, D, mixed, count):
     tol = (16 if mixed else 8) * D * count * (2.0**-24 if dtype == C64 else 2.0**-53)
     for a, b in zip(*res):
         assert float((a - b).abs().max()) <= tol * float(a.abs().max())
+
+
+def test_forward_only_vector_stages_next_to_an_unfused_adjoint():
+    """7 modes, cutoff 9, complex64: the forward-only plan has stages of its own,
+    whose matrix images the table holds although the adjoint's plan has none.
+    Bound as above."""
+    n, D = 7, 9
+    ops = [o[:2] for o in circuits.layered(n, 1, np.random.default_rng(0))]
+    gen = torch.Generator(device=DEV).manual_seed(1)
+    st = torch.randn([D] * n, dtype=C64, device=DEV, generator=gen)
+    params = torch.rand(len(ops), 2, dtype=torch.float64, device=DEV, generator=gen) * 0.4
+    out = []
+    for fuse in (0, None):
+        cc = runtime.CompiledCircuit(ops, n, D, False, C64, DEV, fuse=fuse)
+        cc.build_table(params)
+        out.append(cc.run(st))
+    assert "vector" in cc.step_kinds(True) and set(cc.step_kinds()) == {"op", "diag"}
+    assert float((out[0] - out[1]).abs().max()) <= 8 * D * len(ops) * 2.0**-24 * float(out[0].abs().max())

@@ -83,6 +83,19 @@ def test_large_density_matrices_leave_stages_where_these_lose(n, D, dtype, forwa
     assert (MATRIX in plan.run, MATRIX in plan.kinds) == (forward, adjoint)
 
 
+@pytest.mark.parametrize(
+    "n,D,dtype,forward,adjoint,steps",
+    [(3, 9, _lib.C64, VECTOR, VECTOR, 2), (5, 9, _lib.C64, VECTOR, VECTOR, 8), (6, 9, _lib.C64, MATRIX, VECTOR, 15),
+     (7, 9, _lib.C64, VECTOR, OP, 59), (4, 9, _lib.C128, MATRIX, VECTOR, 7), (4, 10, _lib.C64, MATRIX, VECTOR, 5),
+     (5, 10, _lib.C64, MATRIX, VECTOR, 8), (3, 10, _lib.C64, MATRIX, VECTOR, 5), (4, 10, _lib.C128, MATRIX, VECTOR, 12),
+     (9, 5, _lib.C128, MATRIX, VECTOR, 32), (8, 5, _lib.C128, MATRIX, MATRIX, 15), (8, 6, _lib.C128, MATRIX, VECTOR, 25)],
+)
+def test_stages_of_cutoffs_that_half_fill_an_operand(n, D, dtype, forward, adjoint, steps):
+    plan = Plan(_layered(n), n, D, False, dtype)
+    assert max(plan.run) == forward and len(plan.kinds) == steps
+    assert set(plan.kinds) == {adjoint} if adjoint != OP else max(plan.kinds) <= DIAG
+
+
 @pytest.mark.parametrize("seed", range(12))
 def test_default_plans_keep_every_gate_and_mode_order(seed):
     """Also where some gates of a run leave their stage."""
