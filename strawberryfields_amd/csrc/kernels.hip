@@ -683,11 +683,15 @@ k_reduced_dm(const C<T>* __restrict__ st, ModeList ml, int D, int64_t NR, int64_
 // many rows.  Only tiles on and above the diagonal are computed (rho is
 // Hermitian), and the traced range is cut into grid.y chunks so that few tiles
 // still fill the device.  6 modes, cutoff 8, complex128: modes 0 and 1 15 us and
-// one mode 10 us, on average 61 us before.
-template <int MT>
+// one mode 10 us, on average 61 us before.  Up to 4 rows fill a sixteenth of a
+// 16 x 16 tile and less: there the tile is 4 x 4 and its 16 groups of threads share
+// the traced positions (one of 26 modes, cutoff 2, complex128, 1 GB: the last 4511 us,
+// 16050 with the large tile, 13130 one workgroup per output).
+template <int RW, int MT>
 struct RdmTile {
-  static constexpr int TS = 16 * MT;          // rows and columns of a tile
-  static constexpr int RT = MT == 1 ? 64 : 32;  // traced positions staged at once
+  static constexpr int TS = RW * MT;                             // rows and columns of a tile
+  static constexpr int RT = RW == 4 ? 256 : MT == 1 ? 64 : 32;  // traced positions staged at once
+  static constexpr int SL = 256 / (RW * RW);                     // groups of threads over these
 };
 
 __device__ __forceinline__ int64_t mode_offset(int64_t idx, const int32_t* modes, int cnt, int n, int D) {
@@ -708,10 +712,12 @@ __device__ __forceinline__ int64_t mode_offset(int64_t idx, const int32_t* modes
   return off;
 }
 
-template <typename T, int MT>
+template <typename T, int RW, int MT>
 __global__ void __launch_bounds__(256)
 k_rdm_ket(const C<T>* __restrict__ st, ModeList ml, int D, int64_t NA, int64_t NR, int64_t chunk, double* partial) {
-  constexpr int TS = RdmTile<MT>::TS, RT = RdmTile<MT>::RT;
+  using Tile = RdmTile<RW, MT>;
+  constexpr int TS = Tile::TS, RT = Tile::RT, SL = Tile::SL;
+  static_assert(SL == 1 || MT == 1, "groups of threads hold one output per thread");
   __shared__ C<T> sa[2][TS][RT + 1];  // rows of the tile's a and b side
   __shared__ int64_t off[2 * TS], offr[RT];
   const int n = ml.n, k = ml.k, nt = (int)((NA + TS - 1) / TS);
@@ -724,7 +730,7 @@ k_rdm_ket(const C<T>* __restrict__ st, ModeList ml, int D, int64_t NA, int64_t N
     off[threadIdx.x] = x < NA ? mode_offset(x, ml.kept, k, n, D) : -1;
   }
   const bool rows_fast = k > 0 && ml.kept[k - 1] == n - 1;  // neighbouring rows are neighbours in memory
-  const int ta = (int)threadIdx.x >> 4, tb = (int)threadIdx.x & 15;
+  const int ta = (int)threadIdx.x / RW % RW, tb = (int)threadIdx.x % RW, sl = (int)threadIdx.x / (RW * RW);
   double vr[MT][MT], vi[MT][MT];
 #pragma unroll
   for (int i = 0; i < MT; ++i)
@@ -734,7 +740,7 @@ k_rdm_ket(const C<T>* __restrict__ st, ModeList ml, int D, int64_t NA, int64_t N
   const int64_t r1 = (r0 + chunk < NR) ? r0 + chunk : NR;
   for (int64_t r = r0; r < r1; r += RT) {
     __syncthreads();  // the tile is free, off[] is written
-    if (threadIdx.x < RT) offr[threadIdx.x] = r + threadIdx.x < r1 ? mode_offset(r + threadIdx.x, ml.traced, n - k, n, D) : -1;
+    if ((int)threadIdx.x < RT) offr[threadIdx.x] = r + threadIdx.x < r1 ? mode_offset(r + threadIdx.x, ml.traced, n - k, n, D) : -1;
     __syncthreads();
 #pragma unroll
     for (int e = (int)threadIdx.x; e < 2 * TS * RT; e += 256) {
@@ -744,12 +750,12 @@ k_rdm_ket(const C<T>* __restrict__ st, ModeList ml, int D, int64_t NA, int64_t N
     }
     __syncthreads();
 #pragma unroll 8
-    for (int c = 0; c < RT; ++c) {
+    for (int c = sl; c < RT; c += SL) {
       C<T> x[MT], y[MT];
 #pragma unroll
       for (int i = 0; i < MT; ++i) {
-        x[i] = sa[0][ta + 16 * i][c];
-        y[i] = sa[1][tb + 16 * i][c];
+        x[i] = sa[0][ta + RW * i][c];
+        y[i] = sa[1][tb + RW * i][c];
       }
 #pragma unroll
       for (int i = 0; i < MT; ++i)
@@ -760,11 +766,23 @@ k_rdm_ket(const C<T>* __restrict__ st, ModeList ml, int D, int64_t NA, int64_t N
         }
     }
   }
+  if constexpr (SL > 1) {  // the groups' sums, in a fixed order
+    __shared__ double part[SL][RW * RW][2];
+    const int o = (int)threadIdx.x % (RW * RW);
+    part[sl][o][0] = vr[0][0];
+    part[sl][o][1] = vi[0][0];
+    __syncthreads();
+    if (sl) return;
+    for (int u = 1; u < SL; ++u) {
+      vr[0][0] += part[u][o][0];
+      vi[0][0] += part[u][o][1];
+    }
+  }
 #pragma unroll
   for (int i = 0; i < MT; ++i)
 #pragma unroll
     for (int j = 0; j < MT; ++j) {
-      const int64_t a = a0 + ta + 16 * i, b = b0 + tb + 16 * j;
+      const int64_t a = a0 + ta + RW * i, b = b0 + tb + RW * j;
       if (a < NA && b < NA) {
         const int64_t idx = (((int64_t)blockIdx.y * NA + a) * NA + b) * 2;
         partial[idx] = vr[i][j];
@@ -1212,15 +1230,16 @@ extern "C" int sfamd_all_fock_probs_vjp(const void* state, const void* g_probs, 
 // tiles of a ket's reduced DM and chunks of its traced range: about four
 // workgroups per compute unit, of 64 traced positions and more
 struct RdmPlan {
-  int MT, TS;
+  int RW, MT, TS;
   int64_t NA, NR, tiles, chunks, chunk;
 };
 static RdmPlan rdm_plan(int n, int D, int k) {
   RdmPlan p;
   p.NA = ipow(D, k);
   p.NR = ipow(D, n - k);
+  p.RW = p.NA <= 4 ? 4 : 16;
   p.MT = p.NA >= 32 ? 2 : 1;
-  p.TS = 16 * p.MT;
+  p.TS = p.RW * p.MT;
   const int64_t nt = (p.NA + p.TS - 1) / p.TS;
   p.tiles = nt * (nt + 1) / 2;
   int64_t c = (1024 + p.tiles - 1) / p.tiles;
@@ -1246,10 +1265,8 @@ template <typename T>
 int launch_rdm_ket(const void* state, void* out, int D, const ModeList& ml, double* partial, hipStream_t s) {
   const RdmPlan p = rdm_plan(ml.n, D, ml.k);
   const dim3 grid((unsigned)p.tiles, (unsigned)p.chunks);
-  if (p.MT == 1)
-    hipLaunchKernelGGL((k_rdm_ket<T, 1>), grid, dim3(256), 0, s, CP(T, state), ml, D, p.NA, p.NR, p.chunk, partial);
-  else
-    hipLaunchKernelGGL((k_rdm_ket<T, 2>), grid, dim3(256), 0, s, CP(T, state), ml, D, p.NA, p.NR, p.chunk, partial);
+  const auto kernel = p.RW == 4 ? k_rdm_ket<T, 4, 1> : p.MT == 1 ? k_rdm_ket<T, 16, 1> : k_rdm_ket<T, 16, 2>;
+  hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, CP(T, state), ml, D, p.NA, p.NR, p.chunk, partial);
   HIP_RET(hipGetLastError());
   const int lanes = p.chunks >= 8 ? 64 : 1;
   hipLaunchKernelGGL(k_rdm_ket_final<T>, dim3(grid_for(p.NA * p.NA * lanes)), dim3(kBlock), 0, s, partial, MP(T, out), D,

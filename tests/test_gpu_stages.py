@@ -191,3 +191,24 @@ def test_forward_only_vector_stages_next_to_an_unfused_adjoint():
         out.append(cc.run(st))
     assert "vector" in cc.step_kinds(True) and set(cc.step_kinds()) == {"op", "diag"}
     assert float((out[0] - out[1]).abs().max()) <= 8 * D * len(ops) * 2.0**-24 * float(out[0].abs().max())
+
+
+# ------------------------------------------------------------- readout
+@pytest.mark.parametrize("dtype", [C128, C64])
+@pytest.mark.parametrize(
+    "n,D,modes",
+    # 1 to 5 kept rows; traced ranges of one position, and below, at and above the 256 that are staged at once
+    [(1, 2, [0]), (1, 4, [0]), (8, 2, [0]), (9, 2, [8]), (10, 2, [4]), (13, 2, [0]), (13, 2, [12]), (9, 2, [0, 8]), (6, 3, [2]),
+     (7, 3, [6]), (5, 4, [0]), (6, 4, [5]), (5, 5, [4]), (3, 1, [1])],
+)
+def test_reduced_dm_of_few_rows(dtype, n, D, modes):
+    """M M^H with M the kept x traced matrix of a random ket, against complex128 on
+    the CPU: sums of NR products in 64 bits, rounded once to the state's precision."""
+    g = torch.Generator().manual_seed(D * 10 + n)
+    psi = torch.randn([D] * n, dtype=dtype, generator=g)
+    k = len(modes)
+    M = psi.to(C128).permute(modes + [m for m in range(n) if m not in modes]).reshape(D**k, -1)
+    ref = (M @ M.conj().T).reshape([D] * (2 * k)).permute([a for i in range(k) for a in (i, k + i)])
+    got = runtime.reduced_dm(psi.to(DEV), n, D, False, modes).cpu()
+    tol = 2 * M.shape[1] * 2.0**-53 + (2.0**-23 if dtype == C64 else 0.0)
+    assert float((got.to(C128) - ref).abs().max()) <= tol * float(ref.abs().max())
