@@ -8,8 +8,9 @@
 // captured into a HIP graph by the caller (sfamd_graph_*).
 #include <algorithm>
 #include <cstring>
+#include <exception>
 #include <functional>
-#include <new>
+#include <memory>
 #include <vector>
 
 #include "common.h"
@@ -309,7 +310,7 @@ struct Step {
   int K;
   std::vector<int> ops;  // operation indices in execution order
   StageArgs args;
-  MArgs margs[2];  // [1]: the column axes of a density matrix
+  std::vector<MArgs> margs;  // of a matrix-core stage; [1]: the column axes of a density matrix
   bool mixed;      // the stage acts on a density matrix
   DiagRun run;
 };
@@ -372,16 +373,16 @@ struct StageOp {
 // if its modes lie in the mask, no earlier op left outside the stage touches
 // one of them (gates on disjoint modes commute) and the stage's LDS fits.
 // Returns their number; `skip` marks operations that an earlier stage takes,
-// `got` receives the indices.
-int absorb(const std::vector<StageOp>& ops, const std::vector<int>& rem, unsigned mask, const StageCost& sc,
+// `got` receives the indices; `ops` and `skip` begin at operation `base`.
+int absorb(const std::vector<StageOp>& ops, int base, const std::vector<int>& rem, unsigned mask, const StageCost& sc,
            int64_t budget, const char* skip, std::vector<int>* got) {
   if (got) got->clear();
   unsigned blocked = 0;
   int64_t used = sc.base;
   int count = 0;
   for (int i : rem) {
-    const StageOp& op = ops[i];
-    if (!(op.modes & mask) || (skip && skip[i])) continue;
+    const StageOp& op = ops[i - base];
+    if (!(op.modes & mask) || (skip && skip[i - base])) continue;
     if (count < sc.max_gates && !(op.modes & ~mask) && !(op.modes & blocked) && used + op.cost <= budget) {
       if (got) got->push_back(i);
       ++count;
@@ -403,7 +404,6 @@ Step new_step(int kind, int op) {
   st.K = 0;
   st.mixed = false;
   memset(&st.args, 0, sizeof(st.args));
-  memset(&st.margs, 0, sizeof(st.margs));
   memset(&st.run, 0, sizeof(st.run));
   return st;
 }
@@ -559,6 +559,7 @@ ModeOrder canonical_order(int n, int D) {
 void fill_matrix_stage(const sfamd_prog* p, Step& st, unsigned mask, const ModeOrder& in, const ModeOrder& out,
                        int side) {
   const int n = in.n, D = p->D, Kc = st.K;
+  if ((int)st.margs.size() <= side) st.margs.resize(side + 1);
   MArgs& a = st.margs[side];
   memset(&a, 0, sizeof(a));
   a.side = side;
@@ -827,9 +828,10 @@ void plan_run(const sfamd_prog* p, const std::vector<int>& run, const Stages& sg
     }
   }
   std::vector<int> got, best;
-  std::vector<StageOp> sops(p->nops);
-  for (int i : run) sops[i] = StageOp{op_mask(p->ops[i]), sc.gate(p->ops[i])};
-  std::vector<char> taken(p->nops, 0);
+  const int base = run.front();  // (a run's operations follow one another)
+  std::vector<StageOp> sops;
+  for (int i : run) sops.push_back(StageOp{op_mask(p->ops[i]), sc.gate(p->ops[i])});
+  std::vector<char> taken(run.size(), 0);
   while (!rem.empty()) {
     std::vector<unsigned> local = cands;
     if (local.empty()) {
@@ -849,19 +851,19 @@ void plan_run(const sfamd_prog* p, const std::vector<int>& run, const Stages& sg
     for (int64_t bud : {sc.budget, sc.budget_full}) {
       long bkey = -1;
       for (unsigned m : local) {
-        absorb(sops, rem, m, sc, bud, nullptr, &got);
+        absorb(sops, base, rem, m, sc, bud, nullptr, &got);
         // one step of lookahead: the gates this stage takes plus the most the
         // next stage could take after it (on c3: 49 stages instead of 52);
         // ties go to more gates now, then to tiles that include the last
         // modes (contiguous runs)
         long nxt = 0;
         if (!got.empty() && local.size() > 1 && got.size() < rem.size()) {
-          for (int i : got) taken[i] = 1;
+          for (int i : got) taken[i - base] = 1;
           for (unsigned m2 : local) {
-            const long k = absorb(sops, rem, m2, sc, bud, taken.data(), nullptr);
+            const long k = absorb(sops, base, rem, m2, sc, bud, taken.data(), nullptr);
             if (k > nxt) nxt = k;
           }
-          for (int i : got) taken[i] = 0;
+          for (int i : got) taken[i - base] = 0;
         }
         const long key = (((long)got.size() + nxt) << 40) + ((long)got.size() << 26) + (long)m;
         if (key > bkey) {
@@ -1078,7 +1080,8 @@ void plan_program(sfamd_prog* p) {
   bool other = false;  // matrix-core stages differ (see stage_cost), vector-ALU stages only where the adjoint has none
   for (const OpPlan& op : p->ops) {
     const Stages &f = fwd[op.mixed_in], &b = both[op.mixed_in];
-    other = other || (f.Kc >= 2 && fusable(op, f) && (f.kind == kStepMatrixStage || f.kind != b.kind || f.Kc != b.Kc));
+    // (an operation has one slot for the images of vector-ALU stages)
+    other = other || (f.Kc >= 2 && fusable(op, f) && (f.kind == kStepMatrixStage || b.Kc < 2));
   }
   if (other) plan_steps(p, fwd, true, &p->fsteps);
   // state sizes at step inputs
@@ -1133,7 +1136,7 @@ void place_table(sfamd_prog* p) {
   if (matrix) off += 2 * mst_img(p->D);
   for (Step& st : p->fsteps) {
     if (st.kind != kStepMatrixStage) continue;
-    st.margs[0].phases = st.margs[1].phases = (int32_t)off;
+    for (MArgs& a : st.margs) a.phases = (int32_t)off;
     for (int op : st.ops)
       if (in_phases[op]) {
         p->ops[op].off = off;
@@ -1154,7 +1157,7 @@ void place_table(sfamd_prog* p) {
     if (st.kind == kStepStage) {
       place_images(st.args, true);
     } else if (st.kind == kStepMatrixStage) {
-      st.margs[0].phases = st.margs[1].phases = (int32_t)off;
+      for (MArgs& a : st.margs) a.phases = (int32_t)off;
       for (int op : st.ops)
         if (is_diag_kind(p->ops[op].kind)) {
           p->img0[op] = (int32_t)off;
@@ -1176,8 +1179,7 @@ void place_table(sfamd_prog* p) {
   p->table_elems = off;
   for (std::vector<Step>* steps : {&p->steps, &p->fsteps})
     for (Step& st : *steps) {
-      if (st.kind == kStepMatrixStage)
-        for (int side = 0; side <= (st.mixed ? 1 : 0); ++side) link_matrix_stage(p, st.margs[side], spare);
+      for (MArgs& a : st.margs) link_matrix_stage(p, a, spare);
       if (st.kind == kStepDiagRun)
         for (int g = 0; g < st.run.ngates; ++g) st.run.toff[g] = p->ops[st.run.op[g]].off;
     }
@@ -1328,13 +1330,9 @@ extern "C" int sfamd_replace_mode(const void* in, void* out, int n, int D, int m
 }
 
 // ---------------------------------------------------------------- programs
-extern "C" int sfamd_prog_create(const sfamd_op_t* ops, int nops, int n, int D, int mixed_in, int dtype, int fuse_K,
-                                 sfamd_prog_t** out) {
-  CHECK_ARG(out && nops >= 0 && n >= 1 && n <= 32 && (ops || nops == 0));
-  CHECK_ARG(dtype == SFAMD_C64 || dtype == SFAMD_C128);
-  if (D < 1 || D > SFAMD_MAX_CUTOFF) return SFAMD_E_CUTOFF;
-  sfamd_prog* p = new (std::nothrow) sfamd_prog();
-  if (!p) return SFAMD_E_ARG;
+static int create_program(const sfamd_op_t* ops, int nops, int n, int D, int mixed_in, int dtype, int fuse_K,
+                          std::unique_ptr<sfamd_prog>* out) {
+  std::unique_ptr<sfamd_prog> p(new sfamd_prog());
   p->n = n;
   p->D = D;
   p->dtype = dtype;
@@ -1348,15 +1346,9 @@ extern "C" int sfamd_prog_create(const sfamd_op_t* ops, int nops, int n, int D, 
   int64_t max_state = ipow(D, mixed ? 2 * n : n);
   for (int i = 0; i < nops; ++i) {
     const int st = validate_op(ops[i].kind, ops[i].mode0, ops[i].mode1, n, D);
-    if (st != 0) {
-      delete p;
-      return st;
-    }
+    if (st != 0) return st;
     OpPlan op{ops[i].kind, ops[i].mode0, ops[i].mode1, mixed, 0, 0};
-    if (op.kind == SFAMD_OP_MIX && mixed) {
-      delete p;
-      return SFAMD_E_STATE;
-    }
+    if (op.kind == SFAMD_OP_MIX && mixed) return SFAMD_E_STATE;
     if (op.kind == SFAMD_OP_LOSS && !mixed) op.mix_first = 1;
     if (op.kind == SFAMD_OP_LOSS || op.kind == SFAMD_OP_MIX) mixed = 1;
     p->ops.push_back(op);
@@ -1367,8 +1359,8 @@ extern "C" int sfamd_prog_create(const sfamd_op_t* ops, int nops, int n, int D, 
   }
   p->max_state = max_state;
   p->final_mixed = mixed;
-  plan_program(p);
-  place_table(p);
+  plan_program(p.get());
+  place_table(p.get());
   p->state_elems.push_back(ipow(D, mixed ? 2 * n : n));
   int64_t nwg = (max_state + kBlock - 1) / kBlock;
   // and a workgroup for every tile of a stage (6 modes, cutoff 4, one stage of 8 gates: 256 amplitudes
@@ -1376,14 +1368,29 @@ extern "C" int sfamd_prog_create(const sfamd_op_t* ops, int nops, int n, int D, 
   for (const Step& st : p->steps) {
     bool one_pass;
     p->nwg = 4096;
-    const int64_t groups = st.kind == kStepStage || st.kind == kStepMatrixStage ? step_columns(p, st, &one_pass) : 0;
+    const int64_t groups = st.kind == kStepStage || st.kind == kStepMatrixStage ? step_columns(p.get(), st, &one_pass) : 0;
     if (groups > nwg) nwg = groups;
   }
   if (nwg > 4096) nwg = 4096;
   if (nwg < 1) nwg = 1;
   p->nwg = (int)nwg;
-  *out = p;
+  *out = std::move(p);
   return 0;
+}
+
+extern "C" int sfamd_prog_create(const sfamd_op_t* ops, int nops, int n, int D, int mixed_in, int dtype, int fuse_K,
+                                 sfamd_prog_t** out) {
+  CHECK_ARG(out && nops >= 0 && n >= 1 && n <= 32 && (ops || nops == 0));
+  CHECK_ARG(dtype == SFAMD_C64 || dtype == SFAMD_C128);
+  if (D < 1 || D > SFAMD_MAX_CUTOFF) return SFAMD_E_CUTOFF;
+  try {
+    std::unique_ptr<sfamd_prog> p;
+    RET_IF(create_program(ops, nops, n, D, mixed_in, dtype, fuse_K, &p));
+    *out = p.release();
+    return 0;
+  } catch (const std::exception&) {  // out of host memory
+    return SFAMD_E_ARG;
+  }
 }
 
 extern "C" int sfamd_prog_info(const sfamd_prog_t* p, sfamd_prog_info_t* info) {

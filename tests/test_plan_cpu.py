@@ -1,5 +1,8 @@
 """Which steps a plan takes (host memory only: no device is needed)."""
 import ctypes
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -113,3 +116,27 @@ def test_default_plans_keep_every_gate_and_mode_order(seed):
         for m in range(n):
             order = [i for i in flat if m in ops[i][1]]
             assert order == sorted(order)
+
+
+def test_plans_that_do_not_fit_in_host_memory_are_refused():
+    """An error code, not an exception through the C interface."""
+    code = """
+import ctypes, resource, sys
+sys.path.insert(0, %r)
+from strawberryfields_amd import _lib
+lib = _lib.load()
+n = 100000
+arr = (_lib.OpDesc * n)()
+for i in range(n):
+    arr[i].kind, arr[i].mode0, arr[i].mode1 = _lib.OP_KINDS["D"], i %% 3, -1
+h = ctypes.c_void_p()
+assert lib.sfamd_prog_create(arr, n, 3, 24, 0, 0, 0, ctypes.byref(h)) == 0
+lib.sfamd_prog_destroy(h)
+h = ctypes.c_void_p()
+used = int(open("/proc/self/statm").read().split()[0]) * resource.getpagesize()
+resource.setrlimit(resource.RLIMIT_AS, (used + (16 << 20), -1))
+print(lib.sfamd_prog_create(arr, n, 3, 24, 0, 0, 0, ctypes.byref(h)), h.value)
+""" % os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    res = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True)
+    assert res.returncode == 0, res.stderr[-2000:]
+    assert res.stdout.split() == ["-1", "None"]
