@@ -1212,9 +1212,10 @@ int step_forward(const sfamd_prog* p, const Step& st, const void* table, const v
 int step_columns(const sfamd_prog* p, const Step& st, bool* one_pass) {
   const bool stage = st.kind == kStepStage || st.kind == kStepMatrixStage;
   *one_pass = stage && !st.mixed;
+  if (!stage) return p->nwg;
   const int nt = st.kind == kStepStage ? st.args.ntiles
                                        : (st.margs[0].ntiles + (1 << st.margs[0].lgt) - 1) >> st.margs[0].lgt;
-  return stage && nt < p->nwg ? nt : p->nwg;
+  return nt < p->nwg ? nt : p->nwg;
 }
 
 }  // namespace
