@@ -264,7 +264,7 @@ def measure_c2(steps, cpu=False):
     out = {}
     kets = {}
     for name, dtype in (("complex64", torch.complex64), ("complex128", torch.complex128)):
-        K = tuner.best([(o[0], o[1]) for o in ops], n, D, False, dtype, dev)
+        K = tuner.best([(o[0], o[1]) for o in ops], n, D, False, dtype, dev, forward_only=True)
         cc = runtime.CompiledCircuit([(o[0], o[1]) for o in ops], n, D, False, dtype, dev, fuse=K)
         vac = torch.zeros([D] * n, dtype=dtype, device=dev)
         vac.view(-1)[0] = 1.0

@@ -846,22 +846,29 @@ class GradEvaluator:
 
 
 # --------------------------------------------------------------------- autotuning
-def _structure_key(ops, n, D, mixed, dtype):
+# counts the changes of what a number of local modes means to the planner: a
+# choice stored under another number was measured on other kernels
+PLAN_REVISION = 2
+
+
+def _structure_key(ops, n, D, mixed, dtype, forward_only=False):
     import hashlib
 
     h = hashlib.sha1(repr([(name, tuple(m)) for name, m in ops]).encode()).hexdigest()[:16]
-    return "%d:%d:%d:%s:%s" % (n, D, int(mixed), str(dtype).split(".")[-1], h)
+    what = "f" if forward_only else "g"
+    return "v%d%s:%d:%d:%d:%s:%s" % (PLAN_REVISION, what, n, D, int(mixed), str(dtype).split(".")[-1], h)
 
 
 class Autotuner:
     """Measures the stage tile (local modes K per fused stage, 0 = one kernel
     per gate) for a circuit structure and caches the fastest.
 
-    Candidates are the K whose stage kernels exist for the cutoff; each is
-    timed over a forward + adjoint sweep with HIP events on random parameters.
-    The choice is cached in memory and, when `path` is set (default
-    $SFAMD_AUTOTUNE_CACHE), in a JSON file keyed by (modes, cutoff, mixed,
-    dtype, structure hash).
+    Candidates are the K with plans of their own (a K without stage kernels for
+    the cutoff falls back to another plan); each is timed with HIP events on
+    random parameters, over a forward + adjoint sweep or, for circuits that are
+    only run, over the run.  The choice is cached in memory and, when `path` is
+    set (default $SFAMD_AUTOTUNE_CACHE), in a JSON file keyed by the planner's
+    revision, what was timed, (modes, cutoff, mixed, dtype, structure hash).
     """
 
     def __init__(self, path=None, reps=3):
@@ -888,18 +895,28 @@ class Autotuner:
             except OSError:
                 pass
 
+    def _time(self, run, dev):
+        run()
+        torch.cuda.synchronize(dev)
+        e0 = torch.cuda.Event(enable_timing=True)
+        e1 = torch.cuda.Event(enable_timing=True)
+        e0.record()
+        for _ in range(self.reps):
+            run()
+        e1.record()
+        torch.cuda.synchronize(dev)
+        return e0.elapsed_time(e1) * 1e3 / self.reps
+
     @staticmethod
     def candidates(n, D, mixed):
-        if mixed:
+        if n < 2 or not 2 <= D <= 20:
             return [0]
-        out = [0]
-        for K in (2, 3, 4):
-            if K <= n and 2 <= D <= 20 and D**K <= 4096:
-                out.append(K)
-        return out
+        # stages of more than three modes have tiles of at most 4096 amplitudes; on a density matrix
+        # a stage of two modes has the tile of three axes
+        return [0] + [K for K in range(3 if mixed else 2, 7) if (mixed or K <= n) and (K <= 3 or D**K <= 4096)]
 
-    def best(self, ops, n, D, mixed, dtype, device):
-        key = _structure_key(ops, n, D, mixed, dtype)
+    def best(self, ops, n, D, mixed, dtype, device, forward_only=False):
+        key = _structure_key(ops, n, D, mixed, dtype, forward_only)
         if key in self.cache:
             return self.cache[key]["fuse"]
         cands = self.candidates(n, D, mixed)
@@ -912,11 +929,22 @@ class Autotuner:
         st = torch.zeros([D] * (2 * n if mixed else n), dtype=dtype, device=dev)
         st.view(-1)[0] = 1.0
         times = {}
+        plans = []
         for K in cands:
             cc = CompiledCircuit(ops, n, D, mixed, dtype, dev, fuse=K)
-            if K and cc.nsteps == len(ops):
-                continue  # no stage fits this tile
+            kinds = cc.step_kinds(forward_only)
+            if "vector" not in kinds and "matrix" not in kinds:
+                plan = None  # one kernel per gate
+            else:
+                plan = K if forward_only else (kinds, cc.step_ops)
+            if plan in plans:
+                continue  # timed under a smaller K
+            plans.append(plan)
             cc.build_table(params)
+            if forward_only:
+                out = cc.new_state(cc.nsteps)
+                times[K] = self._time(lambda: cc.run(st, out=out), dev)
+                continue
             saved = [st] + [cc.new_state(i) for i in range(1, cc.nsteps)]
             out = cc.new_state(cc.nsteps)
             lam = torch.randn_like(out)
@@ -927,16 +955,7 @@ class Autotuner:
                 cc.forward(0, cc.nsteps, st, out=out, saved=saved)
                 cc.adjoint(0, cc.nsteps, saved, lam, gin, grads)
 
-            run()
-            torch.cuda.synchronize(dev)
-            e0 = torch.cuda.Event(enable_timing=True)
-            e1 = torch.cuda.Event(enable_timing=True)
-            e0.record()
-            for _ in range(self.reps):
-                run()
-            e1.record()
-            torch.cuda.synchronize(dev)
-            times[K] = e0.elapsed_time(e1) * 1e3 / self.reps
+            times[K] = self._time(run, dev)
         best = min(times, key=times.get)
         self.cache[key] = {"fuse": best, "us": {str(k): round(v, 2) for k, v in times.items()}}
         self._save()

@@ -212,3 +212,31 @@ def test_reduced_dm_of_few_rows(dtype, n, D, modes):
     got = runtime.reduced_dm(psi.to(DEV), n, D, False, modes).cpu()
     tol = 2 * M.shape[1] * 2.0**-53 + (2.0**-23 if dtype == C64 else 0.0)
     assert float((got.to(C128) - ref).abs().max()) <= tol * float(ref.abs().max())
+
+
+# ------------------------------------------------------------- autotuner
+def test_autotuner_measures_the_plans_there_are(tmp_path):
+    """A choice stored by an earlier planner is not taken; plans that are the same
+    are timed once; the tile that the default takes is among the candidates; a
+    forward-only choice is measured and stored apart."""
+    import json
+
+    n, D = 6, 3
+    ops = [o[:2] for o in circuits.layered(n, 1, np.random.default_rng(0))]
+    path = tmp_path / "tiles.json"
+    now = runtime._structure_key(ops, n, D, False, C64)
+    path.write_text(json.dumps({now.split(":", 1)[1]: {"fuse": 77, "us": {}}, "v1g:" + now.split(":", 1)[1]: {"fuse": 78, "us": {}}}))
+    tuner = runtime.Autotuner(path=str(path))
+    assert tuner.best(ops, n, D, False, C64, DEV) in (0, 2, 3, 4, 5, 6)
+    assert str(runtime.default_fuse(n, D)) in tuner.cache[now]["us"]
+    tuner.best(ops, n, D, False, C64, DEV, forward_only=True)
+    assert set(json.loads(path.read_text())) > {now, runtime._structure_key(ops, n, D, False, C64, True)}
+    # three modes at cutoff 11: stages of two modes serve the adjoint also where three are asked for
+    ops = [o[:2] for o in circuits.layered(3, 1, np.random.default_rng(0))]
+    tuner.best(ops, 3, 11, False, C64, DEV)
+    assert set(tuner.cache[runtime._structure_key(ops, 3, 11, False, C64)]["us"]) == {"0", "2"}
+    tuner.best(ops, 3, 11, False, C64, DEV, forward_only=True)
+    assert set(tuner.cache[runtime._structure_key(ops, 3, 11, False, C64, True)]["us"]) == {"0", "2", "3"}
+    # density matrices have stages too
+    ops = [o[:2] for o in circuits.layered(2, 1, np.random.default_rng(0), loss=True)]
+    assert tuner.best(ops, 2, 8, True, C64, DEV) > 0

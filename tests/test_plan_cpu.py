@@ -99,6 +99,20 @@ def test_stages_of_cutoffs_that_half_fill_an_operand(n, D, dtype, forward, adjoi
     assert set(plan.kinds) == {adjoint} if adjoint != OP else max(plan.kinds) <= DIAG
 
 
+@pytest.mark.parametrize("n,D", [(2, 8), (3, 4), (5, 3), (6, 5), (8, 8), (4, 13), (3, 17), (4, 20), (3, 24), (1, 8)])
+@pytest.mark.parametrize("mixed", [False, True])
+def test_autotuner_candidates_are_tiles_that_the_planner_has(n, D, mixed):
+    """And the default tile is one of them, or has the plan of one (a density
+    matrix's stage of two modes has the tile of three axes)."""
+    cands = runtime.Autotuner.candidates(n, D, mixed)
+    want = runtime.default_fuse(n, D)
+    assert (max(want, 3) if mixed and want else want) in cands
+    for K in cands[1:]:
+        plan = Plan([("BS", (0, 1))] * 8 + [("S2", (1, 0))], n, D, mixed, _lib.C64, fuse=K)
+        big = D**n * 8 > 20e6 or (mixed and D > 16)
+        assert big or max(plan.run) == (VECTOR if K == 2 else MATRIX)
+
+
 @pytest.mark.parametrize("seed", range(12))
 def test_default_plans_keep_every_gate_and_mode_order(seed):
     """Also where some gates of a run leave their stage."""
