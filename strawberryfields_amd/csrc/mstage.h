@@ -91,6 +91,11 @@ __host__ __device__ constexpr bool mst_two_groups(int D, int dtype) {
 __host__ __device__ constexpr bool mst_group_ok(int D, int K, int lgt) {
   return lgt <= kMstMaxLgt && (mst_tile(D, K) / D << lgt) <= 1024 && (lgt == 0 || mst_tile(D, K) << lgt <= 16384);
 }
+// groups that fill the 16 columns of a two-mode gate's operand; larger ones (for longer
+// runs of the store, program.hip: order_stages) are forward only
+__host__ __device__ constexpr bool mst_group_fills(int D, int K, int lgt) {
+  return mst_group_ok(D, K, lgt) && (lgt == 0 || (mst_tile(D, K) / (D * D) << (lgt - 1)) <= 8);
+}
 
 // One gate, 64 bytes.  Every field is 32 bits wide: with narrower ones the
 // compiler walked the list through a base pointer one byte past a dword, and

@@ -703,35 +703,36 @@ int launch_mst_adj(const void* psi, const void* lo, void* li, const void* table,
   }
 }
 
-// f(integral constants K, LG) for the kernel of (K, lgt), SFAMD_E_ARG if none exists
+// f(integral constants K, LG) for the kernel of (K, lgt), SFAMD_E_ARG if none exists;
+// ADJ: the groups of a plan with an adjoint
 template <int V>
 struct Int {
   static constexpr int v = V;
 };
-template <int D, int K, typename F>
+template <int D, int K, bool ADJ, typename F>
 int mst_with_group(int lgt, F f) {
   if (lgt == 0) return f(Int<K>(), Int<0>());
-  if constexpr (sfamd::mst_group_ok(D, K, 1))
+  if constexpr (ADJ ? sfamd::mst_group_fills(D, K, 1) : sfamd::mst_group_ok(D, K, 1))
     if (lgt == 1) return f(Int<K>(), Int<1>());
-  if constexpr (sfamd::mst_group_ok(D, K, 2))
+  if constexpr (ADJ ? sfamd::mst_group_fills(D, K, 2) : sfamd::mst_group_ok(D, K, 2))
     if (lgt == 2) return f(Int<K>(), Int<2>());
   return SFAMD_E_ARG;
 }
-template <int D, typename F>
+template <int D, bool ADJ, typename F>
 int mst_with(int K, int lgt, F f) {
-  if (K == 3) return mst_with_group<D, 3>(lgt, f);
+  if (K == 3) return mst_with_group<D, 3, ADJ>(lgt, f);
   if constexpr (sfamd::mst_tile(D, 4) <= sfamd::kMstMaxTile)
-    if (K == 4) return mst_with_group<D, 4>(lgt, f);
+    if (K == 4) return mst_with_group<D, 4, ADJ>(lgt, f);
   if constexpr (sfamd::mst_tile(D, 5) <= sfamd::kMstMaxTile)
-    if (K == 5) return mst_with_group<D, 5>(lgt, f);
+    if (K == 5) return mst_with_group<D, 5, ADJ>(lgt, f);
   if constexpr (sfamd::mst_tile(D, 6) <= sfamd::kMstMaxTile)
-    if (K == 6) return mst_with_group<D, 6>(lgt, f);
+    if (K == 6) return mst_with_group<D, 6, ADJ>(lgt, f);
   return SFAMD_E_ARG;
 }
 
 template <typename T, int D>
 int mst_fwd_k(int K, const void* in, void* out, const void* table, const sfamd::MArgs& a, int grid, hipStream_t s) {
-  return mst_with<D>(K, a.lgt, [&](auto k, auto lg) {
+  return mst_with<D, false>(K, a.lgt, [&](auto k, auto lg) {
     return launch_mst_fwd<T, D, decltype(k)::v, decltype(lg)::v>(in, out, table, a, grid, s);
   });
 }
@@ -739,7 +740,7 @@ int mst_fwd_k(int K, const void* in, void* out, const void* table, const sfamd::
 template <typename T, int D>
 int mst_adj_k(int K, const void* psi, const void* lo, void* li, const void* table, const sfamd::MArgs& a, int grid,
               double* partial, int nwg, hipStream_t s) {
-  return mst_with<D>(K, a.lgt, [&](auto k, auto lg) {
+  return mst_with<D, true>(K, a.lgt, [&](auto k, auto lg) {
     return launch_mst_adj<T, D, decltype(k)::v, decltype(lg)::v>(psi, lo, li, table, a, grid, partial, nwg, s);
   });
 }

@@ -434,8 +434,7 @@ int group_log2(const sfamd_prog* p, int axes, int Kc) {
   const int D = p->D;
   const int64_t ntiles = ipow(D, axes - Kc);
   int l = 0;
-  while (mst_group_ok(D, Kc, l + 1) && (mst_tile(D, Kc) / (D * D) << l) <= 8 && (ntiles >> (l + 1)) >= kComputeUnits)
-    ++l;
+  while (mst_group_fills(D, Kc, l + 1) && (ntiles >> (l + 1)) >= kComputeUnits) ++l;
   return l;
 }
 
