@@ -1053,6 +1053,30 @@ def test_c5_structure_dm_layers_with_loss_checkpoints(dtype):
     assert rel < (1e-8 if dtype == C128 else 1e-5), rel
 
 
+@pytest.mark.parametrize("dtype", [C128, C64])
+def test_c5_structure_dm_layers_one_kernel_per_gate(dtype):
+    """The circuit above gate by gate, as it runs at cutoffs where no stage fits: the
+    two-sided dense gates, strided and slab beamsplitters and losses and their
+    adjoints (the default plan at cutoff 10 has stages)."""
+    r = _c5_structure_reference()
+    n, D, ops = r["n"], r["D"], r["ops"]
+    cc = runtime.CompiledCircuit([(o[0], o[1]) for o in ops], n, D, True, dtype, DEV, fuse=0)
+    assert set(cc.step_kinds()) <= {"op", "diag"}
+    rows = np.zeros((len(ops), 2))
+    for i, (_, _, p) in enumerate(ops):
+        rows[i, : len(p)] = p
+    params = torch.tensor(rows, dtype=torch.float64, device=DEV, requires_grad=True)
+    rho0 = torch.as_tensor(r["vac"], dtype=dtype, device=DEV)
+    rho = runtime.CircuitFunction.apply(params, rho0, cc, len(ops) // r["L"])
+    assert np.abs(to_np(rho) - r["ref"]).max() < TOL[dtype]
+    probs = runtime.all_fock_probs(rho, n, D, True).to(torch.float64)
+    (probs * torch.as_tensor(r["w"], device=DEV)).sum().backward()
+    g = params.grad.cpu().numpy()
+    gflat = np.array([g[i, j] for i, (_, _, p) in enumerate(ops) for j in range(len(p))])
+    rel = np.linalg.norm(gflat[r["sel"]] - r["g_fd"]) / np.linalg.norm(r["g_fd"])
+    assert rel < (1e-8 if dtype == C128 else 1e-5), rel
+
+
 # ------------------------------------------------------------------ S2, MZ, CK, V
 def _s2_dense_from_blocks(blk, D):
     """S2 table: block s = D - 1 + d holds G[N][n] for out1 - out2 = in1 - in2 = d."""

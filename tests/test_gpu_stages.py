@@ -193,6 +193,90 @@ def test_forward_only_vector_stages_next_to_an_unfused_adjoint():
     assert float((out[0] - out[1]).abs().max()) <= 8 * D * len(ops) * 2.0**-24 * float(out[0].abs().max())
 
 
+# ------------------------------------------------------------- stages that are what they claim
+def _against_unfused(ops, n, D, mixed, dtype, fuse, seed, adjoint=True):
+    """The plan of `fuse` against one kernel per gate on a random state and cotangent:
+    the plan, and whether out, run, lam_in and gradients differ by at most
+    8 D m u of the largest entry (16 on a density matrix): m contractions of D terms in
+    either path."""
+    gen = torch.Generator(device=DEV).manual_seed(seed)
+    shape = [D] * (2 * n if mixed else n)
+    st = torch.randn(shape, dtype=dtype, device=DEV, generator=gen)
+    lam = torch.randn(shape, dtype=dtype, device=DEV, generator=gen)
+    params = torch.rand(len(ops), 2, dtype=torch.float64, device=DEV, generator=gen) * 0.4
+    for i, op in enumerate(ops):
+        if op[0] == "V":
+            params[i, 0] *= 0.05
+    res = []
+    for f in (0, fuse):
+        cc = runtime.CompiledCircuit(ops, n, D, mixed, dtype, DEV, fuse=f)
+        got = _sweep(cc, params, st, lam) if adjoint else ()
+        cc.build_table(params)
+        res.append((cc.run(st),) + got)
+    tol = (16 if mixed else 8) * D * len(ops) * (2.0**-24 if dtype == C64 else 2.0**-53)
+    return cc, all(float((a - b).abs().max()) <= tol * float(a.abs().max()) for a, b in zip(*res))
+
+
+_GATES = [("S2", (0, 1)), ("R", (0,)), ("MZ", (1, 0)), ("V", (0,)), ("CK", (2, 0)), ("BS", (0, 2)), ("D", (1,)), ("S", (2,)), ("K", (1,)),
+          ("BS", (2, 1)), ("S2", (2, 0)), ("R", (2,))]
+
+
+@pytest.mark.parametrize(
+    "n,D,dtype",
+    # one and two blocks of 16 rows with 0..3 amplitudes missing, and three (complex64 17 and 18,
+    # whose LDS holds one gate with operators); one tile and several
+    [(3, 9, C128), (4, 9, C64), (3, 10, C64), (4, 10, C128), (3, 11, C64), (4, 11, C128), (4, 12, C64), (3, 12, C128), (3, 13, C64),
+     (3, 13, C128), (3, 14, C64), (3, 14, C128), (3, 15, C64), (3, 15, C128), (3, 16, C64), (3, 17, C64), (3, 18, C64)],
+)
+def test_matrix_core_adjoint_of_every_gate(n, D, dtype):
+    """The gates beyond the layered circuit keep these plans off the vector ALUs."""
+    cc, same = _against_unfused(_GATES, n, D, False, dtype, 3, n * 100 + D)
+    assert "matrix" in cc.step_kinds() and "vector" not in cc.step_kinds()
+    assert same
+
+
+@pytest.mark.parametrize(
+    "n,D,dtype,kind",
+    [(5, 11, C64, "matrix"), (5, 12, C64, "matrix"), (5, 11, C128, "matrix"), (6, 9, C64, "vector"), (4, 10, C64, "vector"), (4, 13, C64, "vector"),
+     (9, 5, C128, "vector"), (8, 6, C128, "vector"), (8, 5, C128, "matrix"), (8, 4, C64, "matrix"), (10, 3, C64, "matrix")],
+)
+def test_layered_gradients_by_default_plan(n, D, dtype, kind):
+    ops = [o[:2] for o in circuits.layered(n, 1, np.random.default_rng(0))]
+    cc, same = _against_unfused(ops, n, D, False, dtype, None, n * 100 + D)
+    assert set(cc.step_kinds()) == {kind}
+    assert same
+
+
+@pytest.mark.parametrize("dtype", [C128, C64])
+@pytest.mark.parametrize("n,D,K", [(10, 3, 3), (13, 2, 3), (9, 3, 4), (8, 4, 3)])
+def test_tile_groups(dtype, n, D, K):
+    """Up to four tiles per workgroup, forward and adjoint."""
+    ops = [o[:2] for o in circuits.layered(n, 1, np.random.default_rng(0))]
+    cc, same = _against_unfused(ops, n, D, False, dtype, K, n * 100 + D)
+    assert set(cc.step_kinds()) == set(cc.step_kinds(True)) == {"matrix"}
+    assert same
+
+
+@pytest.mark.parametrize("dtype", [C128, C64])
+@pytest.mark.parametrize("n,D,K", [(3, 8, 3), (3, 7, 3), (5, 3, 3), (4, 4, 4)])
+def test_tile_groups_on_density_matrices(dtype, n, D, K):
+    ops = [o[:2] for o in circuits.layered(n, 1, np.random.default_rng(0), loss=True)]
+    cc, same = _against_unfused(ops, n, D, True, dtype, K, n * 100 + D)
+    assert "matrix" in cc.step_kinds() and set(cc.step_kinds(True)) == {"matrix", "op"}
+    assert same
+
+
+@pytest.mark.parametrize("dtype", [C128, C64])
+@pytest.mark.parametrize("n,D", [(7, 8), (8, 6), (7, 7)])
+def test_forward_groups_of_stages_without_a_shared_mode(dtype, n, D):
+    """At least 2048 tiles: a workgroup takes neighbouring tiles for the runs of its
+    permuted store."""
+    pairs = [(0, 1), (1, 2), (3, 4), (4, 5), (2, 3), (0, 1), (1, 2), (3, 4), (4, 5), (n - 1, 0)]
+    cc, same = _against_unfused([("BS", p) for p in pairs], n, D, False, dtype, 3, n * 100 + D, adjoint=False)
+    assert set(cc.step_kinds(True)) == {"matrix"} and len(cc.step_kinds(True)) > 2
+    assert same
+
+
 # ------------------------------------------------------------- readout
 @pytest.mark.parametrize("dtype", [C128, C64])
 @pytest.mark.parametrize(

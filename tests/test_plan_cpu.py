@@ -63,6 +63,15 @@ def test_gates_that_share_no_stage_run_alone(n, D, mixed, ops, dtype):
         assert MATRIX in Plan(ops, n, D, mixed, dtype, fuse=3).run
 
 
+@pytest.mark.parametrize("D", [4, 9, 12, 17])
+@pytest.mark.parametrize("kind", ["BS", "MZ", "S2", "CK"])
+def test_pairs_followed_by_a_mode_run_in_one_pass(D, kind):
+    """A two-mode gate on the first modes of a complex64 density matrix takes its own
+    one-pass kernel, also by default."""
+    for modes in [(0, 1), (1, 0)]:
+        assert Plan([(kind, modes)], 3, D, True).run == [OP]
+
+
 @pytest.mark.parametrize("dtype", [_lib.C64, _lib.C128])
 @pytest.mark.parametrize("n,D,mixed", [(3, 8, False), (6, 8, False), (8, 5, False), (12, 2, False), (12, 3, False), (7, 16, False),
                                        (2, 8, True), (3, 9, True), (3, 12, True), (4, 6, True), (6, 3, True), (8, 2, True)])
