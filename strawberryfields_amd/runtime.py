@@ -56,8 +56,9 @@ def default_fuse(n, D):
 
 
 class _KeptInputs:
-    """A share of the bytes that differentiable forwards may keep on a device,
-    held by the autograd node that keeps them and given back when it is freed."""
+    """A share of the bytes that differentiable forwards may keep on a device, held
+    with what is kept and given back when the backward is done with it or the
+    graph is freed."""
 
     _lock = threading.Lock()
     _held = {}  # by device, what was given back not yet subtracted
@@ -134,7 +135,6 @@ class CompiledCircuit:
         if self.D == 1:  # sizes cannot tell kets from DMs
             self.mixed_at = [self.mixed_in] * (self.nsteps + 1)
             self.mixed_at[-1] = self.final_mixed
-        self.inner_bytes = sum(self.state_bytes(i) for i in range(1, self.nsteps))  # all step inputs past the first
         buf = (ctypes.c_int32 * max(1, self.nops))()
         self.step_ops = []
         for i in range(self.nsteps):
@@ -260,8 +260,8 @@ class CompiledCircuit:
         segment=None keeps every step input when they fit in `budget` bytes,
         else uses segments of ~sqrt(nsteps) steps; an int gives the segment
         length in steps.  Within a segment the backward recomputes the
-        forward from the segment's checkpoint (the inputs of a single segment
-        may be kept, see keeps_inputs).
+        forward from the segment's checkpoint (the last segment's inputs may be
+        kept, see keeps_inputs).
         """
         ns = self.nsteps
         if ns == 0:
@@ -281,17 +281,16 @@ class CompiledCircuit:
         The backward begins with that segment, so keeping them saves one
         recomputation (3 modes, cutoff 11, 3 layers, complex128: 478 -> 388 us
         a gradient; 6 modes, cutoff 16, 1 layer, complex64, 45 states of 134 MB:
-        11.2 -> 8.7 ms).  They live until the backward is done.  Of several
-        segments none is kept: their lengths are chosen so that one of them fits
-        in memory, and this one would stay next to the others.  Under
-        saved-tensor hooks (checkpointing, offloading) none is kept either: what
-        they save has to be the same in every forward, and as small as it can be.
+        11.2 -> 8.7 ms).  The first backward takes them and frees them with that
+        segment, so that it never holds two segments; a further one over a
+        retained graph recomputes them.  Under saved-tensor hooks (checkpointing,
+        offloading) none are kept: those save as little as they can.
         Returns the share of the memory that the forward holds on to (see
         _KeptInputs), or None.
         """
-        if b > 0 or e - b < 2 or torch._C._autograd._top_saved_tensors_default_hooks(True) is not None:
+        if e - b < 2 or torch._C._autograd._top_saved_tensors_default_hooks(True) is not None:
             return None
-        return _KeptInputs.reserve(self.table.device, self.inner_bytes)
+        return _KeptInputs.reserve(self.table.device, sum(self.state_bytes(i) for i in range(b + 1, e)))
 
 
 def _params_row(p):
@@ -329,6 +328,7 @@ class CircuitFunction(torch.autograd.Function):
         segs = cc.segments(segment)
         ckpts = []
         inner = []
+        ctx.kept = None
         cur = state_in
         for (b, e) in segs:
             ckpts.append(cur)
@@ -340,7 +340,8 @@ class CircuitFunction(torch.autograd.Function):
         ctx.cc = cc
         ctx.segs = segs
         ctx.params = params
-        ctx.save_for_backward(*ckpts, *inner)
+        ctx.inner = inner  # the last segment's step inputs, until the first backward
+        ctx.save_for_backward(*ckpts)
         return cur if segs else state_in.clone()
 
     @staticmethod
@@ -348,24 +349,25 @@ class CircuitFunction(torch.autograd.Function):
         cc = ctx.cc
         if not ctx.segs:
             return None, g_out, None, None
-        saved = ctx.saved_tensors  # read once: every read unpacks them again under saved-tensor hooks
-        ckpts = saved[: len(ctx.segs)]
-        inner = list(saved[len(ctx.segs) :])  # the last segment's inputs, if the forward kept them
+        ckpts = ctx.saved_tensors  # read once: every read unpacks them again under saved-tensor hooks
+        inner, ctx.inner = ctx.inner, []
+        kept, ctx.kept = ctx.kept, None
         # the gate table may have been rebuilt by another run of the same plan
         cc.build_table(ctx.params, force=False)
         grads = torch.zeros(cc.nops * 2, dtype=torch.float64, device=cc.device)
         lam = g_out.to(cc.dtype).contiguous()
         for si in range(len(ctx.segs) - 1, -1, -1):
             b, e = ctx.segs[si]
-            if inner and e == cc.nsteps:
-                saved = [ckpts[si]] + inner
-            else:
-                saved = [ckpts[si]] + [cc.new_state(i) for i in range(b + 1, e)]
+            saved = [ckpts[si]] + inner
+            if not inner:
+                saved += [cc.new_state(i) for i in range(b + 1, e)]
                 if e - b > 1:
                     cc.forward(b, e - 1, ckpts[si], out=saved[-1], saved=saved[:-1])
             g_in = cc.new_state(b)
             cc.adjoint(b, e, saved, lam, g_in, grads)
             lam = g_in
+            # one segment at a time (the device frees in stream order)
+            inner, saved, kept = [], None, None
         return grads.reshape(-1, 2), lam, None, None
 
 

@@ -94,17 +94,20 @@ def test_pending_forwards_keep_no_more_than_the_budget(monkeypatch):
 
 
 @pytest.mark.parametrize("segment", [3, 10])
-def test_segments_hold_their_checkpoints_only(segment):
-    """A segment length is given to save memory: between forward and backward
-    one state per segment is held, besides the one returned."""
+def test_a_gradient_holds_one_segment_at_a_time(segment):
+    """A segment length is given to save memory: forward and backward together hold
+    a checkpoint per segment, the step inputs of one segment, and a few states (the one
+    returned, its cotangents and the temporaries of the loss)."""
     cc, vac, params = _kept_case()
     assert cc.nsteps > 2 * segment
-    start = torch.cuda.memory_allocated(DEV)
-    out = runtime.run_circuit(cc, params, vac, segment)
-    held = torch.cuda.memory_allocated(DEV) - start
-    nseg = (cc.nsteps + segment - 1) // segment
-    assert held <= nseg * cc.state_bytes(0) + 2**10
-    out[..., 1].abs().square().sum().backward()
+    size = cc.state_bytes(0)
+    for _ in range(2):
+        params.grad = None
+        start = torch.cuda.memory_allocated(DEV)
+        torch.cuda.reset_peak_memory_stats(DEV)
+        runtime.run_circuit(cc, params, vac, segment).abs().square().sum().backward()
+        peak = torch.cuda.max_memory_allocated(DEV) - start
+        assert peak <= ((cc.nsteps + segment - 1) // segment + segment - 1 + 6) * size
 
 
 @pytest.mark.parametrize("segment", [None, 5])
