@@ -855,8 +855,13 @@ void plan_run(const sfamd_prog* p, const std::vector<int>& run, const Stages& sg
         // next stage could take after it (on c3: 49 stages instead of 52);
         // ties go to more gates now, then to tiles that include the last
         // modes (contiguous runs)
+        // (the search grows with the square of the mode sets; on a density matrix
+        // of 9 to 11 modes, whose pass is short at that cutoff, it took longer than
+        // tens of runs: 10 modes, cutoff 2, 2 layers 111 ms and 52 stages and losses, without
+        // it 1.7 ms and 55)
         long nxt = 0;
-        if (!got.empty() && local.size() > 1 && got.size() < rem.size()) {
+        const bool look = local.size() > 1 && !(sg.mixed && local.size() > 100);
+        if (look && !got.empty() && got.size() < rem.size()) {
           for (int i : got) taken[i - base] = 1;
           for (unsigned m2 : local) {
             const long k = absorb(sops, base, rem, m2, sc, bud, taken.data(), nullptr);
