@@ -485,14 +485,14 @@ def run_next(args):
 
 
 def stage_adj_traffic():
-    """HBM bytes per k_stage_adj launch measured by the FETCH_SIZE / WRITE_SIZE
+    """HBM bytes per k_mst_adj launch measured by the FETCH_SIZE / WRITE_SIZE
     counter runs recorded in profiles/ (calibrated against a device copy)."""
-    path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "profiles", "c3_stage_adj_hbm_traffic.txt")
+    path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "profiles", "c3_matrix_stage_hbm_traffic.txt")
     try:
         with open(path) as f:
             for line in f:
-                if line.startswith("traffic_bytes_per_launch k_stage_adj:"):
-                    return int(line.split(":")[1]), "profiles/c3_stage_adj_hbm_traffic.txt"
+                if line.startswith("traffic_bytes_per_launch k_mst_adj:"):
+                    return int(line.split(":")[1]), "profiles/c3_matrix_stage_hbm_traffic.txt"
     except OSError:
         pass
     return None, None
@@ -723,14 +723,16 @@ def main():
     t_fsweep = event_time(lambda: cc.forward(0, cc.nsteps, ev.state_in, out=ev.psi, saved=ev.saved), reps)
     t_asweep = event_time(lambda: cc.adjoint(0, cc.nsteps, ev.saved, ev.g_psi, ev.g_in, ev.grads), reps)
     nops = len(ops)
-    traffic, traffic_src = stage_adj_traffic()
+    # the traffic was counted on the default plan's matrix-core stages
+    matrix = args.fuse is None and set(cc.step_kinds()) == {"matrix"}
+    traffic, traffic_src = stage_adj_traffic() if matrix else (None, None)
     adj_bytes = 4 * S * nops
     fwd_bytes = 2 * S * nops
     achieved = adj_bytes / t_asweep / 1e9
     per_launch = t_asweep / cc.nsteps
     roofline = {
         "bound": "hbm",
-        "kernel": "k_stage_adj (fused adjoint gate stages, %d launches per sweep)" % cc.nsteps,
+        "kernel": "k_mst_adj (matrix-core adjoint gate stages, %d launches per sweep)" % cc.nsteps,
         "achieved": round(achieved, 1),
         "peak": HBM_PEAK_GBS,
         "unit": "GB/s",
@@ -744,7 +746,7 @@ def main():
         "measured_traffic_GBs": round(traffic / per_launch / 1e9, 1) if traffic else None,
         "measured_traffic_frac": round(traffic / per_launch / 1e9 / HBM_PEAK_GBS, 4) if traffic else None,
         "limiter": "not HBM: the 2 MiB state stays in cache and a fused stage moves memory once for ~5 gates; "
-        "the stage kernels are bound by LDS / VALU issue and launch latency (frac is algorithmic bytes "
+        "the stage kernels are bound by launch latency and by LDS, barriers and reductions per gate (frac is algorithmic bytes "
         "over time, not HBM utilisation)",
     }
 
