@@ -526,28 +526,44 @@ __device__ __forceinline__ void heavy_adj(const Gate& g, const C<T>* __restrict_
   }
 }
 
-// A gate's per-lane parameter sums, reduced over the wave and added to the
-// wave's slots while the next gate's LDS reads are in flight.
+// The per-lane parameter sums of the last GATES gates, reduced over the wave together
+// and added to the wave's slots while the next gate's LDS reads are in flight.  Two gates
+// at once halve the reductions' latency, which is in every gate's chain (6 modes, cutoff 8, 4
+// layers, complex64, one gradient 1060 -> 1038 us; 10 modes 3, 2 layers, complex128 855 ->
+// 811).  Where registers are short the second pair of sums spills: 5 modes 10, complex64, 40
+// gates 321 -> 331 us, 5 modes 14, complex128, 2 layers 2146 -> 2282 (mst_sums).
+template <int GATES>
 struct Sums {
-  double g0 = 0.0, g1 = 0.0;
-  int gi = -1;
+  double g0[GATES], g1[GATES];
+  int gi = -1;  // the first gate; a second one is gi - 1
   template <typename Gm>
   __device__ __forceinline__ void flush(double* gsl, bool first) {
     if (gi < 0) return;
-    const double g = wave_sum_pair(g0, g1);
     const int lane = threadIdx.x & 63;
-    if ((lane & 31) == 31) {  // each wave owns its slots: deterministic
-      double* slot = gsl + (gi * 2 + (lane >> 5)) * Gm::NW + wave_index();
+    double g;
+    int at = gi;
+    bool owner;
+    if constexpr (GATES == 2) {
+      g = wave_sum_four(g0[0], g0[1], g1[0], g1[1]);
+      at -= (lane >> 4) & 1;
+      owner = (lane & 15) == 15 && at >= 0;
+    } else {
+      g = wave_sum_pair(g0[0], g1[0]);
+      owner = (lane & 31) == 31;
+    }
+    if (owner) {  // each wave owns its slots: deterministic
+      double* slot = gsl + (at * 2 + (lane >> 5)) * Gm::NW + wave_index();
       slot[0] = first ? g : slot[0] + g;
     }
   }
 };
 
-// gate gi backward; `at`: the tile of its output, moved to that of its input; `first`: the workgroup's first group
-template <typename T, typename Gm>
+// gate gi backward; `at`: the tile of its output, moved to that of its input; `first`: the workgroup's first
+// group; SLOT: its place among the gates whose sums are reduced together; the first flushes those before
+template <typename T, typename Gm, int SLOT, int GATES>
 __device__ __forceinline__ void gate_adj(const Gate& g, int gi, const C<T>* __restrict__ table,
                                          const Walk<T, Gm>& wk, const C<T>* ph, C<T>*& at, C<T>* lam, double* gsl,
-                                         bool first, Sums& sum, const AdjOp<T, Gm>& op, AdjOp<T, Gm>& next) {
+                                         bool first, Sums<GATES>& sum, const AdjOp<T, Gm>& op, AdjOp<T, Gm>& next) {
   next.load(table, g.padj, g.two & 4);
   double g0 = 0.0, g1 = 0.0;
   if (g.kind <= SFAMD_OP_KERR) {
@@ -560,11 +576,13 @@ __device__ __forceinline__ void gate_adj(const Gate& g, int gi, const C<T>* __re
       lam[o] = cmul(w, l);
       at[o] = cmul(w, x);
     });
-    sum.flush<Gm>(gsl, first);
+    if (SLOT == 0) sum.template flush<Gm>(gsl, first);
   } else {
     const bool two = g.two & 1;
     const int N = Gm::items(two);
-    auto flush = [&]() { sum.flush<Gm>(gsl, first); };
+    auto flush = [&]() {
+      if (SLOT == 0) sum.template flush<Gm>(gsl, first);
+    };
     if (wave_index() >= N) flush();
     if (two)
       heavy_adj<T, Gm, true>(g, table, at - Gm::GS, lam, op, g0, g1, flush);
@@ -572,9 +590,12 @@ __device__ __forceinline__ void gate_adj(const Gate& g, int gi, const C<T>* __re
       heavy_adj<T, Gm, false>(g, table, at - Gm::GS, lam, op, g0, g1, flush);
     at -= Gm::GS;
   }
-  sum.g0 = g0;
-  sum.g1 = g1;
-  sum.gi = gi;
+  sum.g0[SLOT] = g0;
+  sum.g1[SLOT] = g1;
+  if (SLOT == 0) {
+    if (GATES == 2) sum.g0[GATES - 1] = sum.g1[GATES - 1] = 0.0;
+    sum.gi = gi;
+  }
   __syncthreads();
 }
 
@@ -583,6 +604,12 @@ template <typename T, typename Gm>
 constexpr int adj_waves() {
   return (sfamd::mst_two_groups(Gm::D, sizeof(T) == 4 ? SFAMD_C64 : SFAMD_C128) && Gm::LG == 0 && Gm::NW == 8) ? 4
                                                                                                     : (Gm::NW + 3) / 4;
+}
+
+// gates whose sums are reduced together (see Sums): one where the adjoint kernel has no register left
+template <typename T, typename Gm>
+constexpr int mst_sums() {
+  return Gm::D <= 8 || (Gm::D <= 12 && sizeof(T) == 8) ? 2 : 1;
 }
 
 template <typename T, typename Gm>
@@ -633,13 +660,14 @@ k_mst_adj(const C<T>* __restrict__ psi_in, const C<T>* __restrict__ lam_out, C<T
     }
     AdjOp<T, Gm> opA, opB;
     opA.load(table, a.hl_adj, a.hl_two);
-    Sums sum;
+    constexpr int kGates = mst_sums<T, Gm>();
+    Sums<kGates> sum;
     for (int gi = last; gi >= 0; gi -= 2) {
-      gate_adj<T, Gm>(a.g[gi], gi, table, wk, ph, at, lam, gsl, grp == tr.first, sum, opA, opB);
+      gate_adj<T, Gm, 0>(a.g[gi], gi, table, wk, ph, at, lam, gsl, grp == tr.first, sum, opA, opB);
       if (gi == 0) break;
-      gate_adj<T, Gm>(a.g[gi - 1], gi - 1, table, wk, ph, at, lam, gsl, grp == tr.first, sum, opB, opA);
+      gate_adj<T, Gm, kGates - 1>(a.g[gi - 1], gi - 1, table, wk, ph, at, lam, gsl, grp == tr.first, sum, opB, opA);
     }
-    sum.flush<Gm>(gsl, grp == tr.first);
+    sum.template flush<Gm>(gsl, grp == tr.first);
     wk.store(lam, lam_in);
     __syncthreads();  // the tiles are free for the next group's loads
   }

@@ -51,22 +51,41 @@ __device__ __forceinline__ float wave_sum(float v) {
   return v;
 }
 
-// Sums of a and b over the 64 lanes of a wave in one reduction: swapping the
-// upper half of a with the lower half of b leaves a's pair sums in lanes 0 to 31
-// and b's in lanes 32 to 63 after one addition.  a's sum is valid in lane 31, b's
-// in lane 63.
+// x + y after their upper and lower halves (or odd and even rows of 16 lanes) were
+// swapped: x's pair sums in the lower half (even rows), y's in the upper (odd rows)
+template <bool ROWS>
+__device__ __forceinline__ double swap_add(double x, double y) {
+  const unsigned long long ux = (unsigned long long)__double_as_longlong(x);
+  const unsigned long long uy = (unsigned long long)__double_as_longlong(y);
+  const auto lo = ROWS ? __builtin_amdgcn_permlane16_swap((unsigned)ux, (unsigned)uy, false, false)
+                       : __builtin_amdgcn_permlane32_swap((unsigned)ux, (unsigned)uy, false, false);
+  const auto hi = ROWS ? __builtin_amdgcn_permlane16_swap((unsigned)(ux >> 32), (unsigned)(uy >> 32), false, false)
+                       : __builtin_amdgcn_permlane32_swap((unsigned)(ux >> 32), (unsigned)(uy >> 32), false, false);
+  return __longlong_as_double((long long)(((unsigned long long)hi[0] << 32) | lo[0])) +
+         __longlong_as_double((long long)(((unsigned long long)hi[1] << 32) | lo[1]));
+}
+
+// Sums of a and b over the 64 lanes of a wave in one reduction: a's in lane 31, b's in
+// lane 63.
 __device__ __forceinline__ double wave_sum_pair(double a, double b) {
-  const unsigned long long ua = (unsigned long long)__double_as_longlong(a);
-  const unsigned long long ub = (unsigned long long)__double_as_longlong(b);
-  const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)ua, (unsigned)ub, false, false);
-  const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(ua >> 32), (unsigned)(ub >> 32), false, false);
-  double v = __longlong_as_double((long long)(((unsigned long long)hi[0] << 32) | lo[0])) +
-             __longlong_as_double((long long)(((unsigned long long)hi[1] << 32) | lo[1]));
+  double v = swap_add<false>(a, b);
   v += dpp_move<0xB1, 0xF>(v);   // quad_perm [1, 0, 3, 2]
   v += dpp_move<0x4E, 0xF>(v);   // quad_perm [2, 3, 0, 1]
   v += dpp_move<0x141, 0xF>(v);  // row_half_mirror
   v += dpp_move<0x140, 0xF>(v);  // row_mirror
   v += dpp_move<0x142, 0xA>(v);  // row_bcast:15 into rows 1, 3
+  return v;
+}
+
+// Sums of a, b, c and d over the 64 lanes of a wave in one reduction of six steps, as
+// many as one sum takes: every lane of row 0 (lanes 0 to 15) receives a's, of row 1 b's, of
+// row 2 c's and of row 3 d's.  The summation order is fixed.
+__device__ __forceinline__ double wave_sum_four(double a, double b, double c, double d) {
+  double v = swap_add<true>(swap_add<false>(a, c), swap_add<false>(b, d));
+  v += dpp_move<0xB1, 0xF>(v);   // quad_perm [1, 0, 3, 2]
+  v += dpp_move<0x4E, 0xF>(v);   // quad_perm [2, 3, 0, 1]
+  v += dpp_move<0x141, 0xF>(v);  // row_half_mirror
+  v += dpp_move<0x140, 0xF>(v);  // row_mirror
   return v;
 }
 
