@@ -990,7 +990,7 @@ class BatchEvaluator:
     ones) and joins them before the graph ends.  Most circuits of a mixed batch
     are small and bound by per-launch latency, so many branches pay: on the
     256-circuit workload 8 streams give 5.3 batches/s, 32 give 9.5 and 64 give
-    9.8.  A call copies the stacked parameters into the static buffers and
+    9.8.  A call copies every circuit's parameters into its static buffer and
     launches the graph once.
     """
 
